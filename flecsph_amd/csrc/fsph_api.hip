@@ -422,7 +422,7 @@ void fsph_destroy(fsph_ctx *ctx) {
                        &c->gccount, &c->gmoff, &c->gmask, &c->h_prop,
                        &c->h_prev, &c->hflag, &c->glist, &c->hgflag,
                        &c->hgscan, &c->hcnt, &c->hflag2, &c->hgflag2,
-                       &c->glist2};
+                       &c->glist2, &c->list_off, &c->list_ids};
   for (auto *b : all)
     if (b->p) hipFree(b->p);
   fsph::free_gravity(c);
@@ -883,58 +883,7 @@ int fsph_neighbor_lists(fsph_ctx *ctx, int64_t *off, int64_t *ids,
   CTX_OR_FAIL;
   FSPH_TRY(fsph::need_tree(c));
   if (!off) return fsph::fail(c, FSPH_E_ARG, "off is required");
-  // read back through the tiles the pair passes walk
-  const int64_t n = c->n, nt = c->nt;
-  std::vector<int32_t> ts(nt), tc(nt), sl(nt), cc(nt);
-  std::vector<int64_t> mo(nt);
-  std::vector<uint32_t> mask((size_t)c->mask_words);
-  std::vector<int32_t> nngb(n);
-  FSPH_HIP(c, hipMemcpyAsync(ts.data(), c->tstart.p, nt * 4,
-                             hipMemcpyDeviceToHost, c->stream));
-  FSPH_HIP(c, hipMemcpyAsync(tc.data(), c->tcount.p, nt * 4,
-                             hipMemcpyDeviceToHost, c->stream));
-  FSPH_HIP(c, hipMemcpyAsync(sl.data(), c->tslot.p, nt * 4,
-                             hipMemcpyDeviceToHost, c->stream));
-  FSPH_HIP(c, hipMemcpyAsync(cc.data(), c->tccount.p, nt * 4,
-                             hipMemcpyDeviceToHost, c->stream));
-  FSPH_HIP(c, hipMemcpyAsync(mo.data(), c->tmoff.p, nt * 8,
-                             hipMemcpyDeviceToHost, c->stream));
-  FSPH_HIP(c, hipMemcpyAsync(nngb.data(), c->f[fsph::PF_NNGB].p, n * 4,
-                             hipMemcpyDeviceToHost, c->stream));
-  if (c->mask_words)
-    FSPH_HIP(c, hipMemcpyAsync(mask.data(), c->mask.p, mask.size() * 4,
-                               hipMemcpyDeviceToHost, c->stream));
-  FSPH_HIP(c, hipStreamSynchronize(c->stream));
-  off[0] = 0;
-  for (int64_t i = 0; i < n; ++i) off[i + 1] = off[i] + nngb[i];
-  if (!ids) return FSPH_OK;
-  if (cap < off[n]) return fsph::fail(c, FSPH_E_CAP, "ids buffer too small");
-  std::vector<int32_t> cand;
-  for (int64_t t = 0; t < nt; ++t) {
-    cand.resize(cc[t]);
-    if (cc[t])
-      FSPH_HIP(c, hipMemcpy(cand.data(),
-                            c->cand.as<int32_t>() + (int64_t)sl[t] * c->ccap,
-                            (size_t)cc[t] * 4, hipMemcpyDeviceToHost));
-    const int nw = (cc[t] + 31) / 32;
-    for (int k = 0; k < tc[t]; ++k) {
-      const int64_t i = ts[t] + k;
-      std::vector<int64_t> lst;
-      for (int w = 0; w < nw; ++w) {
-        uint32_t bits = mask[mo[t] + (int64_t)w * tc[t] + k];
-        while (bits) {
-          const int j = __builtin_ctz(bits);
-          bits &= bits - 1;
-          lst.push_back(cand[w * 32 + j]);
-        }
-      }
-      std::sort(lst.begin(), lst.end());
-      if ((int64_t)lst.size() != off[i + 1] - off[i])
-        return fsph::fail(c, FSPH_E_ARG, "inconsistent neighbour count");
-      std::copy(lst.begin(), lst.end(), ids + off[i]);
-    }
-  }
-  return FSPH_OK;
+  return fsph::stage_lists(c, off, ids, cap);
 }
 
 int fsph_phase_times(fsph_ctx *ctx, float ms[FSPH_NTIMERS]) {

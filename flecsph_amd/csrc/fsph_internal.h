@@ -167,6 +167,7 @@ struct Ctx {
   DBuf mask;                 // uint32 words
   int64_t mask_words = 0;
   bool have_tree = false;
+  DBuf list_off, list_ids;   // neighbour lists: row offsets, a part's ids
   // gather tiles of the smoothing-length solver (radius h_search * h)
   int64_t gccap = 4096;
   DBuf gcand, gccount, gmoff, gmask;
@@ -346,6 +347,8 @@ int stage_neighbors(Ctx *c);           // k_neighbors.hip
 // groups are built, tile slot i belonging to group glist[i].
 int stage_gather_tiles(Ctx *c, double scale, const float *hprop = nullptr,
                        const int32_t *glist = nullptr, int64_t ngl = -1);
+// neighbour lists of the tiles into host arrays (k_lists.hip)
+int stage_lists(Ctx *c, int64_t *off, int64_t *ids, int64_t cap);
 int stage_newton_h(Ctx *c, const float *h0);   // k_hsolve.hip
 int stage_learned_h(Ctx *c);                    // k_hsolve.hip
 // MLP (k_mlp.hip): X is B x 8 floats (6 features, 2 zero pads)

@@ -1,0 +1,36 @@
+"""Neighbour lists expanded on the device against the oracle's: tiles of a
+few candidates, tiles with more candidates than one LDS sort holds (a very
+wide sphere puts every particle into many tiles), and lists longer than one
+part of the device buffer (2^24 entries)."""
+import numpy as np
+import pytest
+
+from flecsph_amd import BodySystem, _abi, generators
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,n_ngb,wide", [
+    (2, 40, 0), (65, 40, 0), (129, 10, 1), (9001, 20, 1), (70001, 260, 0)])
+@pytest.mark.parametrize("tile_rows", [64, 128])
+def test_lists_equal_the_oracles(oracle_mod, n, n_ngb, wide, tile_rows):
+    if n == 70001 and tile_rows == 128:
+        pytest.skip("the part boundaries do not depend on the tile width")
+    parts, prm = generators.random_box(n, seed=n, h_spread=0.3, n_ngb=n_ngb)
+    parts["h"][:wide] = 0.9
+    p = _abi.default_params(**prm)
+    g, o = BodySystem(p), oracle_mod.OracleSystem(p, threads=8)
+    g._call("set_tuning", tile_rows, 128)
+    for s in (g, o):
+        s.upload(parts)
+        s.update_iteration()
+    og, ig = g.neighbor_lists()
+    oo, io = o.neighbor_lists()
+    assert np.array_equal(og, oo)
+    # (the oracle's rows are in the traversal's discovery order)
+    io = np.concatenate([np.sort(io[oo[i]:oo[i + 1]]) for i in range(n)])
+    assert np.array_equal(ig, io)
+    if n == 70001:
+        assert og[n] > 1 << 24
+    o.close()
+    g.close()
