@@ -416,7 +416,7 @@ void fsph_destroy(fsph_ctx *ctx) {
                        &c->nchild, &c->nbox, &c->ncom, &c->nmass, &c->nrad,
                        &c->nlap, &c->nlevel, &c->leaf_parent, &c->gstart,
                        &c->gcount, &c->gnode, &c->gflag, &c->gscan, &c->cand,
-                       &c->gtile, &c->tstart, &c->tcount, &c->tslot,
+                       &c->tgrp, &c->rowrel, &c->tstart, &c->tcount, &c->tslot,
                        &c->tccount, &c->tmoff,
                        &c->ccount, &c->moff, &c->mask, &c->gcand,
                        &c->gccount, &c->gmoff, &c->gmask, &c->h_prop,

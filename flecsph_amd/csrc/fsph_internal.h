@@ -149,7 +149,7 @@ struct Ctx {
   int groups_max = 128;      // group_max the current groups were built with
                              // (sizes the kernels that take a group's rows)
   DBuf gstart, gcount, gnode, gflag, gscan;
-  DBuf gtile;                // first tile of each group (int32)
+  DBuf tgrp;                 // group of each tile (int32)
   int64_t nt = 0, nsplit = 0;  // tiles; groups cut in two
   int tile_rows = 64;        // tuning: tile width asked for (64 or 128)
   int tiles_w = 128;         // tile width the current tiles were built with
@@ -159,11 +159,12 @@ struct Ctx {
   int64_t ccap = 2048;       // candidate capacity per slot
   int stack_tier[2] = {0, 0};  // traversal LDS stack size (SPH, gather)
   int chunk = 128;           // candidates per LDS round of the pair kernels
-  // cand: (ng + nsplit) slots of ccap int32 (the traversal fills slot g of
-  // group g; the masks kernel compacts it in place for the group's first
-  // tile and writes the second tile's into slot ng + ...); ccount int32 per
-  // group; moff int64 per group
+  // cand: (ng + 2 nsplit) slots of ccap int32 (the traversal fills slot g
+  // of group g; the masks kernel compacts it in place for a group of one
+  // tile and writes the two tiles of a split group to slots of their own);
+  // ccount int32 per group; moff int64 per group
   DBuf cand, ccount, moff;
+  DBuf rowrel;               // per particle float4: FP32 row of its unit
   DBuf mask;                 // uint32 words
   int64_t mask_words = 0;
   bool have_tree = false;

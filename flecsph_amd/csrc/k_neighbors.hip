@@ -32,6 +32,7 @@ constexpr int kW = 64;          // one wavefront per group
 // the gather tiles).
 constexpr int kStackSmall = 512, kStackMid = 1024, kStackLarge = 4096;
 constexpr int kMaxGroup = 128;  // tree_topology::sub_entities_
+constexpr int kRowBlock = 8;    // mask rows tested as one unrolled block
 
 __device__ inline bool box_box(const double *a, const double *b) {
   // intersects_box_box(min1,max1,min2,max2), tree_geometry.h:306-314
@@ -93,6 +94,9 @@ struct TravArgs {
   const int32_t *glist;  // tile slot -> group (or null: slot = group)
   // batched mode: the walk starts at the root of the group's instance
   const int32_t *inst, *root;
+  // out, per row: position relative to the unit's first particle and
+  // squared radius in FP32, what the masks screen with
+  float4 *rowrel;
 };
 
 // MAXG: the largest group (64 when group_max <= 64, else kMaxGroup), which
@@ -128,6 +132,9 @@ __global__ __launch_bounds__(kW) void k_traverse(TravArgs a) {
     sz[k] = a.z[gs + k];
     sh[k] = !a.gather ? a.h[gs + k]
             : a.rscale * (a.hprop ? (double)a.hprop[gs + k] : a.h[gs + k]);
+    a.rowrel[gs + k] = make_float4(
+        (float)(sx[k] - a.x[gs]), (float)(sy[k] - a.y[gs]),
+        (float)(sz[k] - a.z[gs]), (float)(sh[k] * sh[k]));
   }
   double gb[6];
   if (gn >= 0) {
@@ -318,12 +325,13 @@ struct MaskArgs {
   int gather;
   const float *hprop;    // gather radius base instead of h (or null)
   const int32_t *glist;  // tile slot -> group (or null)
-  // SPH tiles (null: the slot is its own tile, compacted in place into
-  // ccount/cand/mask at moff): first tile of each group, candidate slot of
-  // each tile, and the outputs per tile
-  const int32_t *gtile, *tslot;
+  // SPH tiles: each tile's group, rows and candidate slot, and the outputs
+  // per tile (gather units are their own tiles, compacted in place into
+  // ccount/cand/mask at moff)
+  const int32_t *tgrp, *tstart, *tcount, *tslot;
   int32_t *tcc;
   int64_t *tmo;
+  const float4 *rowrel;  // written by the traversal
 };
 
 // Bit compress (the "compress" of Hacker's Delight, 2nd ed., section 7-4):
@@ -359,68 +367,105 @@ __device__ inline uint32_t compress(uint32_t x, uint32_t m, const Compress &c) {
   return x;
 }
 
-// GATHER selects the gather-mode predicate at compile time (the SPH form
-// keeps its inner loop free of the other mode's code).  The wavefront
-// stages kR candidates per round and deals the round's (particle, mask
-// word) combinations over its lanes, so groups smaller than the wavefront
-// keep every lane busy.  A candidate that fails the centre-of-mass filter
-// (or lies past the tile's end) is staged with a NaN x, which fails every
-// distance test.  max(h_k, h_b)^2 is taken as max(h_k^2, h_b^2): squaring
-// and rounding are monotone, so the bound is the same number.
+// Row data is read through the scalar cache (the row index is uniform over
+// the wavefront): constant-address-space views.
+typedef const __attribute__((address_space(4))) double *ConstD;
+typedef const __attribute__((address_space(4))) float *ConstF;
+__device__ inline ConstD const_view(const double *p) {
+  return (ConstD)(uintptr_t)p;
+}
+__device__ inline ConstF const_view(const float4 *p) {
+  return (ConstF)(uintptr_t)p;
+}
+
+// v_writelane_b32: `old` with lane `lane` (uniform) replaced by v (uniform);
+// the compiler has no __builtin_ form of it
+__device__ int write_lane(int v, int lane, int old)
+    __asm("llvm.amdgcn.writelane.i32");
+
+// Neighbour bits of one tile.  GATHER selects the gather-mode predicate at
+// compile time.  One wavefront per tile holds 64 candidates per round, one
+// per lane, and takes the rows one after the other: a row's comparison over
+// the wavefront is the row's 64 mask bits in a scalar register pair (no bits
+// are put together lane by lane), which a v_writelane per word hands to the
+// lane that owns the row.
 //
-// Then the candidates that are no neighbour of any particle of a tile are
-// dropped from that tile (about a third on Sedov 64^3): each round's column
-// of words is ORed over the tile's rows, the used candidates are written in
-// order to the tile's candidate slot, and every row's bits are compressed
-// to the same used positions, so the pair passes stage and walk only used
-// candidates in an unchanged order.  NH = 2 cuts a group of more than 64
-// particles into two tiles (rows 0-63 and the rest), each with its own used
-// candidates; the first tile's are compacted in place, ahead of the reads.
-// The neighbour predicate is the group's (its candidates and its
-// centre-of-mass filter) whatever the cut.
-template <bool GATHER, int MAXG, int NH>
+// The rows are tested in FP32 first, on positions relative to the unit's
+// first particle (scalar loads of the traversal's rowrel): an FP32 add,
+// multiply or FMA issues in 2.5 cycles here, an FP64 one in 5.  With
+// u = d^2 - max(h_k^2, h_b^2) in FP32 and R the largest coordinate, row or
+// candidate, the rounding of the coordinates (2^-24 R each), of d^2 and of
+// the bound moves u by less than 84 R^2 2^-24 + max(h^2) 2^-22; outside
+// tau = 2^-17 max(R^2, h^2) the sign of u decides, and a round of rows with
+// a u inside it (or not a number; about one in a hundred rounds) is tested
+// over in FP64 with the reference's operations.  A tau too small to be
+// normal counts as infinite: everything is then tested in FP64.
+// d <= max(h_k, h_b)^2 is tested there as d <= h_k^2 or d <= h_b^2: squaring
+// and rounding are monotone, so the outcome is the same.
+//
+// Rows go in unrolled blocks of kRowBlock, whose lane numbers and loads are
+// then constants: with one scalar unit for four SIMDs, the scalar
+// instructions of a loop over rows (mask bookkeeping, lane number, loop)
+// bounded it.  The last block may run over the tile's end: its extra rows
+// are other tiles' (or the buffer's padding) and their lanes are cleared.
+// Sedov 64^3 (474,552 rows and copies) 418 -> 214 us, 1M star 1,000 -> 512,
+// 1.5M collapse 1,594 -> 987 and 1,036 -> 713 (gather), against lanes that
+// held (row, word) pairs, read the candidates from LDS and put the words
+// together bit by bit in FP64; it issues a VALU instruction per 3.7 cycles
+// and SIMD there, 13 per row and round.  A hull box over every eight rows
+// that skips the rounds which miss it saved nothing: 64 candidates in a row
+// cover about the extent of a tile.
+//
+// The candidates that are no neighbour of any of the tile's rows are
+// dropped (about a third on Sedov 64^3): the round's row masks are ORed
+// over the lanes, the used candidates are written in order to the tile's
+// candidate slot, and every row's bits are compressed to the same used
+// positions, so the pair passes stage and walk only used candidates in an
+// unchanged order.  A group cut into two tiles has a wavefront for each
+// (one for both took as long as the largest group: 1.9 wavefronts per SIMD
+// were resident on average on Sedov 64^3), whose candidates go to slots of
+// their own; otherwise they are compacted in place, ahead of the reads.  The
+// neighbour predicate is the group's (its candidates and its centre-of-mass
+// filter) whatever the cut.
+template <bool GATHER, int NR>
 __global__ __launch_bounds__(kW) void k_masks(MaskArgs a) {
 #pragma clang fp contract(off)
-  constexpr int kR = 64;  // candidates per round (2 mask words)
-  constexpr int kRW = kR / 32;
-  __shared__ double cx[kR], cy[kR], cz[kR], ch2[kR];
-  __shared__ double px[MAXG], py[MAXG], pz[MAXG], ph2[MAXG];
-  __shared__ int cnt[MAXG];
-  __shared__ uint32_t rw[kRW][MAXG];
+  __shared__ double ph2[NR * kW];
   const int lane = threadIdx.x;
-  const int64_t gi = xcd_item(blockIdx.x, gridDim.x);
-  const int64_t g = a.glist ? a.glist[gi] : gi;
-  const int64_t gs = a.gstart[g];
-  const int gc = a.gcount[g];
+  const int64_t t = xcd_item(blockIdx.x, gridDim.x);
+  const int64_t g = GATHER ? (a.glist ? a.glist[t] : t) : a.tgrp[t];
+  const int64_t g0 = a.gstart[g];  // the unit's first particle
+  const int64_t gs = GATHER ? g0 : a.tstart[t];
+  const int gc = GATHER ? a.gcount[g] : a.tcount[t];
   const int gn = GATHER ? -1 : a.gnode[g];
-  const int cc = a.ccount[gi];
-  const int64_t mo = a.moff[gi];
-  const int64_t cbase = gi * a.ccap;
-  // tiles of this group: nh of them, rows [64 h, ...) of tile h
-  const int64_t t0 = a.gtile ? a.gtile[g] : gi;
-  const int nh = (NH == 2 && gc > kW) ? 2 : 1;
-  int64_t cout[NH], mout[NH];
-  int rows[NH];
-  {
-    const int nw0 = (cc + 31) >> 5;
+  const int64_t cslot = GATHER ? t : g;
+  const int cc = a.ccount[cslot];
+  const int64_t cbase = cslot * a.ccap;
+  const int64_t cout = GATHER ? cbase : (int64_t)a.tslot[t] * a.ccap;
+  // the group's mask words hold its tiles one after the other
+  const int64_t mout = a.moff[cslot] + (gs - g0) * ((cc + 31) >> 5);
+  const double ox = a.x[g0], oy = a.y[g0], oz = a.z[g0];
+  const float inf = __builtin_inff();
+  float scale2 = 0.f;  // max of the rows' R^2 and squared radii
 #pragma unroll
-    for (int hh = 0; hh < NH; ++hh) {
-      cout[hh] = (a.gtile ? (int64_t)a.tslot[t0 + (hh < nh ? hh : 0)] : gi) *
-                 a.ccap;
-      rows[hh] = nh == 1 ? gc : (hh == 0 ? kW : gc - kW);
-      mout[hh] = mo + (int64_t)hh * kW * nw0;
+  for (int r = 0; r < NR; ++r) {
+    const int k = lane + r * kW;
+    if (k < gc) {
+      const double h = !GATHER ? a.h[gs + k]
+                               : a.rscale * (a.hprop ? (double)a.hprop[gs + k]
+                                                     : a.h[gs + k]);
+      ph2[k] = h * h;
+      const float4 q = a.rowrel[gs + k];
+      const float m = fmaxf(fmaxf(fabsf(q.x), fabsf(q.y)), fabsf(q.z));
+      scale2 = fmaxf(scale2, fmaxf(m * m, q.w));
     }
   }
-  for (int k = lane; k < gc; k += kW) {
-    px[k] = a.x[gs + k];
-    py[k] = a.y[gs + k];
-    pz[k] = a.z[gs + k];
-    const double r =
-        !GATHER ? a.h[gs + k]
-                : a.rscale * (a.hprop ? (double)a.hprop[gs + k] : a.h[gs + k]);
-    ph2[k] = r * r;
-    cnt[k] = 0;
-  }
+  for (int o = 32; o > 0; o >>= 1)
+    scale2 = fmaxf(scale2, __shfl_xor(scale2, o, 64));
+  __syncthreads();
+  const ConstD X = const_view(a.x + gs), Y = const_view(a.y + gs),
+               Z = const_view(a.z + gs);
+  const ConstF RR = const_view(a.rowrel + gs);
   double gcom[3] = {0, 0, 0}, gext_lap = 0, grad = 0;
   if (gn >= 0) {
     gcom[0] = a.com[3 * (int64_t)gn];
@@ -429,180 +474,167 @@ __global__ __launch_bounds__(kW) void k_masks(MaskArgs a) {
     gext_lap = a.lap[gn];
     grad = a.rad[gn];
   }
-  // compaction state per tile: used candidates so far, words written and
-  // bits pending (per row k = lane + 64 r of the tile's rows)
-  int64_t used_so_far[NH] = {};
-  uint64_t pend[MAXG / kW] = {};
-  int nb[NH] = {}, wi[NH] = {};
-  // The next round's candidates are loaded into registers while the
-  // current round's masks are compacted, and stored to LDS after.
-  int32_t cidx[kR / kW];
-  double rx[kR / kW], ry[kR / kW], rz[kR / kW], rh[kR / kW];
-  auto prefetch = [&](int r0) {
-#pragma unroll
-    for (int q = 0; q < kR / kW; ++q) {
-      const int j = r0 + lane + q * kW;
-      cidx[q] = j < cc ? a.cand[cbase + j] : -1;
-    }
-#pragma unroll
-    for (int q = 0; q < kR / kW; ++q) {
-      const int32_t b = cidx[q];
-      if (b < 0) continue;
-      rx[q] = a.x[b];
-      ry[q] = a.y[b];
-      rz[q] = a.z[b];
-      rh[q] = a.h[b];
-    }
+  // compaction state: used candidates so far, words written and bits
+  // pending (per row k = lane + 64 r)
+  int64_t used_so_far = 0;
+  uint64_t pend[NR] = {};
+  int nb = 0, wi = 0, cnt[NR] = {};
+  // The next round's candidates are loaded while the current round's rows
+  // are tested, their indices one round earlier still.
+  double rx = 0, ry = 0, rz = 0, rh = 0;
+  auto index_of = [&](int r0) {
+    const int j = r0 + lane;
+    return j < cc ? a.cand[cbase + j] : -1;
   };
-  if (cc > 0) prefetch(0);
-  for (int r0 = 0; r0 < cc; r0 += kR) {
-    int32_t ccur[kR / kW];
-#pragma unroll
-    for (int q = 0; q < kR / kW; ++q) {
-      const int i = lane + q * kW;
-      ccur[q] = cidx[q];
-      double bx = __builtin_nan(""), by = 0, bz = 0, bh = 0;
-      if (cidx[q] >= 0) {
-        bx = rx[q];
-        by = ry[q];
-        bz = rz[q];
-        bh = rh[q];
-        if (gn >= 0) {
-          // COM filter, tree_topology.h:365-371
-          const double ext = ((bh < gext_lap) ? gext_lap : bh) + grad;
-          if (!within_distance2(bx, by, bz, gcom[0], gcom[1], gcom[2], ext))
-            bx = __builtin_nan("");
-        }
-      }
-      cx[i] = bx;
-      cy[i] = by;
-      cz[i] = bz;
-      ch2[i] = bh * bh;
+  auto fetch = [&](int32_t b) {
+    if (b < 0) return;
+    rx = a.x[b];
+    ry = a.y[b];
+    rz = a.z[b];
+    rh = a.h[b];
+  };
+  int32_t ccur = index_of(0);
+  fetch(ccur);
+  int32_t cnext = index_of(kW);
+  for (int r0 = 0; r0 < cc; r0 += kW) {
+    // a lane without a candidate, or whose candidate fails the
+    // centre-of-mass filter, is infinitely far away
+    const double cx = rx, cy = ry, cz = rz, ch2 = rh * rh;
+    bool on = ccur >= 0;
+    if (gn >= 0) {
+      // COM filter, tree_topology.h:365-371
+      const double ext = ((rh < gext_lap) ? gext_lap : rh) + grad;
+      on = on && within_distance2(cx, cy, cz, gcom[0], gcom[1], gcom[2], ext);
     }
-    __syncthreads();
-    const int nwr = min(kRW, (cc - r0 + 31) >> 5);
-    for (int q = lane; q < nwr * gc; q += kW) {
-      const int w = q / gc, k = q - w * gc;
-      const double qx = px[k], qy = py[k], qz = pz[k], qh2 = ph2[k];
-      uint32_t word = 0;
-      for (int jj = 0; jj < 32; ++jj) {
-        const int j = w * 32 + jj;
-        const double d0 = qx - cx[j], d1 = qy - cy[j], d2 = qz - cz[j];
-        const double d = d0 * d0 + d1 * d1 + d2 * d2;
-        bool in;
-        if (GATHER) {
-          in = d < qh2;
-        } else {
-          // tree_topology.h:372-379: d^2 <= max(h_k, h_b)^2
-          in = d <= fmax(qh2, ch2[j]);
-        }
-        if (in) word |= 1u << jj;
-      }
-      rw[w][k] = word;
-    }
-    __syncthreads();
-    if (a.nngb)  // each row's count, by the lane that owns the row
-      for (int k = lane; k < gc; k += kW) {
-        int nk = 0;
-        for (int w = 0; w < nwr; ++w) nk += __popc(rw[w][k]);
-        cnt[k] += nk;
-      }
-    if (r0 + kR < cc) prefetch(r0 + kR);
+    const float fx = on ? (float)(cx - ox) : inf, fy = (float)(cy - oy),
+                fz = (float)(cz - oz), fh2 = GATHER ? 0.f : (float)ch2;
+    float tau = inf;
     {
-      // candidates of the round that neighbour some row of each tile
-      uint32_t used[NH][kRW];
-      int before[NH][kRW], total[NH];
-#pragma unroll
-      for (int hh = 0; hh < NH; ++hh) {
-        total[hh] = 0;
-#pragma unroll
-        for (int w = 0; w < kRW; ++w) {
-          uint32_t v = 0;
-          if (w < nwr && hh < nh) {
-            if (nh == 1) {
-              for (int k = lane; k < gc; k += kW) v |= rw[w][k];
-            } else {
-              const int k = lane + hh * kW;
-              if (k < gc) v = rw[w][k];
-            }
-          }
-#pragma unroll
-          for (int o = 32; o > 0; o >>= 1) v |= __shfl_xor(v, o, 64);
-          used[hh][w] = __builtin_amdgcn_readfirstlane(v);
-          before[hh][w] = total[hh];
-          total[hh] += __popc(used[hh][w]);
-        }
-      }
-#pragma unroll
-      for (int hh = 0; hh < NH; ++hh) {
-        if (hh >= nh) break;
-        Compress cm[kRW];
-#pragma unroll
-        for (int w = 0; w < kRW; ++w) cm[w] = compress_masks(used[hh][w]);
-#pragma unroll
-        for (int q = 0; q < kR / kW; ++q) {
-          const int i = lane + q * kW, w = i >> 5, bit = i & 31;
-          if (used[hh][w] >> bit & 1u)
-            a.cand[cout[hh] + used_so_far[hh] + before[hh][w] +
-                   __popc(used[hh][w] & ((1u << bit) - 1u))] = ccur[q];
-        }
-        // each row's bits at the used positions, appended after the bits of
-        // the earlier rounds (the same positions for every row of the tile)
-#pragma unroll
-        for (int r = 0; r < MAXG / kW; ++r) {
-          const int k = lane + r * kW;
-          if (k >= gc || (nh == 2 && r != hh)) continue;
-          const int kk = k - (nh == 2 ? hh * kW : 0);
-          uint64_t acc = pend[r];
-          int nbl = nb[hh], wil = wi[hh];
-#pragma unroll
-          for (int w = 0; w < kRW; ++w) {
-            if (w >= nwr) break;
-            acc |= (uint64_t)compress(rw[w][k], used[hh][w], cm[w]) << nbl;
-            nbl += __popc(used[hh][w]);
-            if (nbl >= 32) {
-              a.mask[mout[hh] + (int64_t)wil * rows[hh] + kk] = (uint32_t)acc;
-              acc >>= 32;
-              nbl -= 32;
-              ++wil;
-            }
-          }
-          pend[r] = acc;
-        }
-        for (int w = 0; w < nwr; ++w) {
-          nb[hh] += __popc(used[hh][w]);
-          if (nb[hh] >= 32) {
-            nb[hh] -= 32;
-            ++wi[hh];
-          }
-        }
-        used_so_far[hh] += total[hh];
-      }
+      const float m = fmaxf(fmaxf(fabsf((float)(cx - ox)), fabsf(fy)),
+                            fabsf(fz));
+      const float t2 = 0x1p-17f * fmaxf(scale2, fmaxf(m * m, fh2));
+      if (t2 > 0x1p-100f) tau = t2;
     }
-    __syncthreads();
-  }
+    const uint64_t far = __ballot(!on);
+    fetch(cnext);
+    const int32_t cafter = index_of(r0 + 2 * kW);
+    // bits of row k over the round's candidates, in lane k % 64
+    uint32_t lo[NR] = {}, hi[NR] = {};
 #pragma unroll
-  for (int hh = 0; hh < NH; ++hh) {
-    if (hh >= nh) break;
-    if (nb[hh] > 0)
+    for (int r = 0; r < NR; ++r) {
+      const int nrow = gc - r * kW;
 #pragma unroll
-      for (int r = 0; r < MAXG / kW; ++r) {
+      for (int k0 = 0; k0 < kW; k0 += kRowBlock) {
+        if (k0 >= nrow) break;
+        float q[4 * kRowBlock];
+#pragma unroll
+        for (int u = 0; u < 4 * kRowBlock; ++u)
+          q[u] = RR[4 * (r * kW + k0) + u];
+        uint64_t amb = 0;
+#pragma unroll
+        for (int v = 0; v < kRowBlock; ++v) {
+          const float d0 = q[4 * v] - fx, d1 = q[4 * v + 1] - fy,
+                      d2 = q[4 * v + 2] - fz;
+          const float d = __builtin_fmaf(
+              d2, d2, __builtin_fmaf(d1, d1, d0 * d0));
+          // (the median with infinity: a maximum without the second
+          // instruction that quiets the loaded operand)
+          const float u =
+              d - (GATHER ? q[4 * v + 3]
+                          : __builtin_amdgcn_fmed3f(q[4 * v + 3], fh2, inf));
+          const uint64_t m = __ballot(u <= -tau);
+          amb |= __ballot(!(fabsf(u) >= tau));
+          lo[r] = (uint32_t)write_lane((int)(uint32_t)m, k0 + v, (int)lo[r]);
+          hi[r] = (uint32_t)write_lane((int)(uint32_t)(m >> 32), k0 + v,
+                                       (int)hi[r]);
+        }
+        if (amb & ~far) {
+          const int k1 = min(k0 + kRowBlock, nrow);
+          for (int k = k0; k < k1; ++k) {
+            const int kr = r * kW + k;
+            const double qh2 = ph2[kr];
+            const double e0 = X[kr] - cx, e1 = Y[kr] - cy, e2 = Z[kr] - cz;
+            const double e = e0 * e0 + e1 * e1 + e2 * e2;
+            // tree_topology.h:372-379: d^2 <= max(h_k, h_b)^2
+            const uint64_t m =
+                (GATHER ? __ballot(e < qh2)
+                        : __ballot(e <= qh2) | __ballot(e <= ch2)) & ~far;
+            lo[r] = (uint32_t)write_lane((int)(uint32_t)m, k, (int)lo[r]);
+            hi[r] = (uint32_t)write_lane((int)(uint32_t)(m >> 32), k,
+                                         (int)hi[r]);
+          }
+        }
+      }
+      if (lane >= nrow) lo[r] = hi[r] = 0;
+      cnt[r] += __popc(lo[r]) + __popc(hi[r]);
+    }
+    uint32_t v0 = lo[0], v1 = hi[0];
+    if (NR == 2) {
+      v0 |= lo[NR - 1];
+      v1 |= hi[NR - 1];
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      v0 |= __shfl_xor(v0, o, 64);
+      v1 |= __shfl_xor(v1, o, 64);
+    }
+    const uint32_t u0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)v0);
+    const uint32_t u1 = (uint32_t)__builtin_amdgcn_readfirstlane((int)v1);
+    const uint64_t used = (uint64_t)u1 << 32 | u0;
+    if (used) {
+      const int n0 = __popc(u0), n1 = __popc(u1);
+      const Compress c0 = compress_masks(u0), c1 = compress_masks(u1);
+      if (used >> lane & 1ull)
+        a.cand[cout + used_so_far +
+               __popcll(used & ((1ull << lane) - 1ull))] = ccur;
+      // each row's bits at the used positions, appended after the bits of
+      // the earlier rounds (the same positions for every row of the tile)
+#pragma unroll
+      for (int r = 0; r < NR; ++r) {
         const int k = lane + r * kW;
-        if (k >= gc || (nh == 2 && r != hh)) continue;
-        const int kk = k - (nh == 2 ? hh * kW : 0);
-        a.mask[mout[hh] + (int64_t)wi[hh] * rows[hh] + kk] = (uint32_t)pend[r];
+        if (k >= gc) continue;
+        uint64_t acc = pend[r];
+        int nbl = nb, wil = wi;
+        auto put = [&](uint32_t bits, int n) {
+          acc |= (uint64_t)bits << nbl;
+          nbl += n;
+          if (nbl >= 32) {
+            a.mask[mout + (int64_t)wil * gc + k] = (uint32_t)acc;
+            acc >>= 32;
+            nbl -= 32;
+            ++wil;
+          }
+        };
+        put(compress(lo[r], u0, c0), n0);
+        put(compress(hi[r], u1, c1), n1);
+        pend[r] = acc;
       }
-    if (lane == 0) {
-      if (a.gtile) {
-        a.tcc[t0 + hh] = (int32_t)used_so_far[hh];
-        a.tmo[t0 + hh] = mout[hh];
-      } else {
-        a.ccount[gi] = (int32_t)used_so_far[hh];
-      }
+      nb += n0 + n1;
+      wi += nb >> 5;
+      nb &= 31;
+      used_so_far += n0 + n1;
+    }
+    ccur = cnext;
+    cnext = cafter;
+  }
+  if (nb > 0)
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      const int k = lane + r * kW;
+      if (k < gc) a.mask[mout + (int64_t)wi * gc + k] = (uint32_t)pend[r];
+    }
+  if (lane == 0) {
+    if (GATHER) {
+      a.ccount[t] = (int32_t)used_so_far;
+    } else {
+      a.tcc[t] = (int32_t)used_so_far;
+      a.tmo[t] = mout;
     }
   }
   if (a.nngb)
-    for (int k = lane; k < gc; k += kW) a.nngb[gs + k] = cnt[k];
+#pragma unroll
+    for (int r = 0; r < NR; ++r)
+      if (lane + r * kW < gc) a.nngb[gs + r * kW + lane] = cnt[r];
 }
 
 struct TileBufs {
@@ -624,12 +656,13 @@ int build_tiles(Ctx *c, TileBufs tb, bool gather, double scale,
                                  : c->gstart.as<int32_t>();
   const int32_t *ucount = gather ? c->tcount.as<int32_t>()
                                  : c->gcount.as<int32_t>();
-  // candidate slots: one per unit, plus the second tiles of split groups
-  const int64_t nslots = nu + (gather ? 0 : c->nsplit);
+  // candidate slots: one per unit, plus two per split group
+  const int64_t nslots = nu + (gather ? 0 : 2 * c->nsplit);
   // rows of the largest unit (sizes the kernels' LDS arrays)
   const bool u64 = (gather ? c->tiles_w : c->groups_max) <= kW;
   FSPH_TRY(ensure(c, tb.ccount, (size_t)nu * 4));
   FSPH_TRY(ensure(c, tb.moff, (size_t)(nu + 1) * 8));
+  FSPH_TRY(ensure(c, c->rowrel, (size_t)(c->pcap + kW) * sizeof(float4)));
   for (int attempt = 0;; ++attempt) {
     FSPH_TRY(ensure(c, tb.cand, (size_t)nslots * tb.ccap * 4));
     FSPH_HIP(c, hipMemsetAsync(c->flags.p, 0, sizeof(int), c->stream));
@@ -644,7 +677,8 @@ int build_tiles(Ctx *c, TileBufs tb, bool gather, double scale,
                gather ? 1 : 0,          hprop,
                glist,
                c->batch.n_inst ? c->f[PF_INST].as<int32_t>() : nullptr,
-               c->batch.n_inst ? c->batch.root.as<int32_t>() : nullptr};
+               c->batch.n_inst ? c->batch.root.as<int32_t>() : nullptr,
+               c->rowrel.as<float4>()};
     {
       PhaseTimer tm(c, gather ? FSPH_T_H : FSPH_T_TRAVERSE);
       const int tier = c->stack_tier[gather ? 1 : 0];
@@ -718,23 +752,24 @@ int build_tiles(Ctx *c, TileBufs tb, bool gather, double scale,
              tb.mask.as<uint32_t>(),  nngb,
              scale,                   gather ? 1 : 0,
              hprop,                   glist,
-             tiled ? c->gtile.as<int32_t>() : nullptr,
+             tiled ? c->tgrp.as<int32_t>() : nullptr,
+             c->tstart.as<int32_t>(), c->tcount.as<int32_t>(),
              tiled ? c->tslot.as<int32_t>() : nullptr,
              tiled ? c->tccount.as<int32_t>() : nullptr,
-             tiled ? c->tmoff.as<int64_t>() : nullptr};
+             tiled ? c->tmoff.as<int64_t>() : nullptr,
+             c->rowrel.as<float4>()};
   {
     PhaseTimer tm(c, gather ? FSPH_T_H : FSPH_T_MASKS);
-    const bool split = tiled && c->nsplit > 0;
+    // rows of the widest tile: one or two per lane
+    const unsigned nw = (unsigned)(gather ? nu : c->nt);
     if (gather && u64)
-      k_masks<true, kW, 1><<<(unsigned)nu, kW, 0, c->stream>>>(m);
+      k_masks<true, 1><<<nw, kW, 0, c->stream>>>(m);
     else if (gather)
-      k_masks<true, kMaxGroup, 1><<<(unsigned)nu, kW, 0, c->stream>>>(m);
-    else if (u64)
-      k_masks<false, kW, 1><<<(unsigned)nu, kW, 0, c->stream>>>(m);
-    else if (split)
-      k_masks<false, kMaxGroup, 2><<<(unsigned)nu, kW, 0, c->stream>>>(m);
+      k_masks<true, 2><<<nw, kW, 0, c->stream>>>(m);
+    else if (c->tiles_w <= kW)
+      k_masks<false, 1><<<nw, kW, 0, c->stream>>>(m);
     else
-      k_masks<false, kMaxGroup, 1><<<(unsigned)nu, kW, 0, c->stream>>>(m);
+      k_masks<false, 2><<<nw, kW, 0, c->stream>>>(m);
   }
   return hip_check(c, hipGetLastError(), "k_masks");
 }

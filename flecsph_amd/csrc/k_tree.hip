@@ -390,15 +390,16 @@ __global__ __launch_bounds__(kT) void k_group_flags(
 }
 
 // Writes group g (its start, count and node) and its tiles: tile t0 =
-// g + (split groups before g) holds the first min(count, tw) rows and
-// reads candidate slot g; a split group's second tile t0 + 1 holds the rest
-// and reads slot ng + (split groups before g).
+// g + (split groups before g) holds the first min(count, tw) rows, and a
+// split group's second tile t0 + 1 the rest.  The candidates of a group's
+// only tile are in the group's slot g; a split group (s-th of them) has two
+// slots of its own, ng + 2 s and ng + 2 s + 1.
 __global__ __launch_bounds__(kT) void k_group_write(
     const int64_t *__restrict__ flag, const int64_t *__restrict__ pos,
     const int32_t *__restrict__ start, const int32_t *__restrict__ count,
     int64_t nn, int64_t n, int64_t ng, int tw, int32_t *__restrict__ gstart,
     int32_t *__restrict__ gcount, int32_t *__restrict__ gnode,
-    int32_t *__restrict__ gtile, int32_t *__restrict__ tstart,
+    int32_t *__restrict__ tgrp, int32_t *__restrict__ tstart,
     int32_t *__restrict__ tcount, int32_t *__restrict__ tslot) {
   const int64_t i = (int64_t)blockIdx.x * kT + threadIdx.x;
   if (i >= nn + n || !flag[i]) return;
@@ -417,14 +418,16 @@ __global__ __launch_bounds__(kT) void k_group_write(
   }
   gstart[g] = st;
   gcount[g] = cnt;
-  gtile[g] = (int32_t)t0;
+  tgrp[t0] = (int32_t)g;
   tstart[t0] = st;
   tslot[t0] = (int32_t)g;
   if (cnt > tw) {
     tcount[t0] = tw;
+    tslot[t0] = (int32_t)(ng + 2 * s);
+    tgrp[t0 + 1] = (int32_t)g;
     tstart[t0 + 1] = st + tw;
     tcount[t0 + 1] = cnt - tw;
-    tslot[t0 + 1] = (int32_t)(ng + s);
+    tslot[t0 + 1] = (int32_t)(ng + 2 * s + 1);
   } else {
     tcount[t0] = cnt;
   }
@@ -566,7 +569,7 @@ int stage_groups(Ctx *c) {
   FSPH_TRY(ensure(c, c->gstart, (size_t)ng * 4));
   FSPH_TRY(ensure(c, c->gcount, (size_t)ng * 4));
   FSPH_TRY(ensure(c, c->gnode, (size_t)ng * 4));
-  FSPH_TRY(ensure(c, c->gtile, (size_t)ng * 4));
+  FSPH_TRY(ensure(c, c->tgrp, (size_t)c->nt * 4));
   FSPH_TRY(ensure(c, c->tstart, (size_t)c->nt * 4));
   FSPH_TRY(ensure(c, c->tcount, (size_t)c->nt * 4));
   FSPH_TRY(ensure(c, c->tslot, (size_t)c->nt * 4));
@@ -574,7 +577,7 @@ int stage_groups(Ctx *c) {
       c->gflag.as<int64_t>(), c->gscan.as<int64_t>(), c->nstart.as<int32_t>(),
       c->ncount.as<int32_t>(), nn, n, ng, c->tiles_w,
       c->gstart.as<int32_t>(), c->gcount.as<int32_t>(),
-      c->gnode.as<int32_t>(), c->gtile.as<int32_t>(),
+      c->gnode.as<int32_t>(), c->tgrp.as<int32_t>(),
       c->tstart.as<int32_t>(), c->tcount.as<int32_t>(),
       c->tslot.as<int32_t>());
   return hip_check(c, hipGetLastError(), "k_group_write");

@@ -34,3 +34,39 @@ def test_lists_equal_the_oracles(oracle_mod, n, n_ngb, wide, tile_rows):
         assert og[n] > 1 << 24
     o.close()
     g.close()
+
+
+@pytest.mark.parametrize("scale,offset,lattice", [
+    (1e-25, 0.0, False), (1e-12, 0.0, False), (1e19, 0.0, False),
+    (1e30, 0.0, False), (1.0, 1e6, False), (1.0, 0.0, True)])
+@pytest.mark.parametrize("tile_rows", [64, 128])
+def test_lists_where_fp32_cannot_decide(oracle_mod, scale, offset, lattice,
+                                        tile_rows):
+    """The masks decide pairs in FP32 and fall back to FP64 near the radius:
+    positions whose squares under- or overflow FP32, a large common offset,
+    and a lattice with h on a lattice distance (every shell is a tie)."""
+    if lattice:
+        g1 = np.arange(14) / 16.0
+        x, y, z = (v.ravel() for v in np.meshgrid(g1, g1, g1, indexing="ij"))
+        parts, prm = generators.random_box(len(x), seed=4, n_ngb=40)
+        parts.update(x=x, y=y, z=z, h=np.full(len(x), 0.125))
+    else:
+        parts, prm = generators.random_box(2500, seed=4, h_spread=0.4,
+                                           n_ngb=40)
+        for k in ("x", "y", "z"):
+            parts[k] = parts[k] * scale + offset
+        parts["h"] = parts["h"] * scale
+    p = _abi.default_params(**prm)
+    g, o = BodySystem(p), oracle_mod.OracleSystem(p, threads=8)
+    g._call("set_tuning", tile_rows, 128)
+    for s in (g, o):
+        s.upload(parts)
+        s.update_iteration()
+    og, ig = g.neighbor_lists()
+    oo, io = o.neighbor_lists()
+    assert np.array_equal(og, oo)
+    io = np.concatenate([np.sort(io[oo[i]:oo[i + 1]])
+                         for i in range(len(oo) - 1)])
+    assert np.array_equal(ig, io)
+    o.close()
+    g.close()
