@@ -4,13 +4,18 @@
 // After the neighbour tiles are built, a step runs, with no host round trip
 // in between: density+EOS, acceleration with the signal speed, kick v,
 // du/dt, kick u, the smoothing-length update and the per-instance minimum
-// time step.  These are captured once into a hipGraph as persistent
-// kernels: grids of the resident size whose workgroups take groups from
-// device-side work counters (pair passes) or stride over the particles
-// (per-particle kernels), so the launch shapes do not depend on the step.  Every step then updates the
-// kernel nodes' arguments (pointers after the buffer rotations, group and
-// particle counts) and replays the same executable graph.  The graph is
+// time step.  These are captured once into a hipGraph: the pair passes with
+// one workgroup per tile, the per-particle kernels as grids of a fixed size
+// that stride over the particles.  Every step then updates the kernel nodes'
+// arguments (pointers after the buffer rotations, particle counts) and the
+// pair passes' grids, and replays the same executable graph.  The graph is
 // captured again when the configuration it was built for changes.
+//
+// (The pair passes are the eager ones.  Persistent forms that took tiles from
+// a counter per launch measured slower on 32 blasts and tubes, 2.3M
+// particles and copies: density 946 us against 480, du/dt 1,280 against
+// 1,093, acceleration 1,480 against 1,474: twice the registers, and two
+// barriers and an atomic per tile.)
 #include <cstring>
 
 #include "fsph_internal.h"
@@ -19,26 +24,18 @@ namespace fsph {
 
 namespace {
 
-__global__ void k_zero_u64(unsigned long long *p, int n) {
-  const int i = threadIdx.x;
-  if (i < n) p[i] = 0ull;
-}
-
 constexpr size_t kSlotsBytes = kNSlots * kGraphSlot;
-constexpr size_t kWorkBytes = 64;  // one work descriptor per pair pass
-constexpr size_t kHostBytes = kSlotsBytes + 4 * kWorkBytes + 64;
+constexpr size_t kHostBytes = kSlotsBytes + 64;
 
 struct NodeSpec {
   const void *func;
-  unsigned block;
+  unsigned grid, block;
   void *args[2];
-  bool pair;  // a pair pass (resident grid), else a per-particle kernel
 };
 
 int graph_setup(Ctx *c) {
   auto &G = c->graph;
-  if (G.counters.p) return 0;
-  FSPH_TRY(ensure(c, G.counters, 4 * sizeof(unsigned long long)));
+  if (G.cus) return 0;
   G.host.assign(kHostBytes, 0);
   int cus = 0;
   FSPH_HIP(c, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount,
@@ -52,20 +49,17 @@ int graph_setup(Ctx *c) {
 int step_specs(Ctx *c, NodeSpec *sp) {
   auto &G = c->graph;
   char *h = G.host.data();
-  char *work = h + kSlotsBytes;
-  int64_t *n = reinterpret_cast<int64_t *>(work + 4 * kWorkBytes);
+  int64_t *n = reinterpret_cast<int64_t *>(h + kSlotsBytes);
   sph_graph_args(c, h);
   step_graph_args(c, h);
   *n = c->n;
-  for (int pass = 0; pass < 4; ++pass)
-    sph_graph_work(c, pass, work + pass * kWorkBytes);
   auto pair = [&](int pass) {
-    return NodeSpec{sph_graph_func(c, pass), sph_graph_block(c),
-                    {h + pass * kGraphSlot, work + pass * kWorkBytes}, true};
+    return NodeSpec{sph_graph_func(c, pass), (unsigned)c->nt,
+                    sph_graph_block(c), {h + pass * kGraphSlot, nullptr}};
   };
   auto step = [&](int what) {
-    return NodeSpec{step_graph_func(c, what), 256,
-                    {h + kSlotStep * kGraphSlot, n}, false};
+    return NodeSpec{step_graph_func(c, what), 16u * (unsigned)G.cus, 256,
+                    {h + kSlotStep * kGraphSlot, n}};
   };
   int k = 0;
   sp[k++] = pair(kSlotDens);
@@ -78,36 +72,18 @@ int step_specs(Ctx *c, NodeSpec *sp) {
   return k;
 }
 
-unsigned grid_of(Ctx *c, const NodeSpec &s) {
-  if (!s.pair) return (unsigned)(16 * c->graph.cus);
-  // pair passes: the resident size (at least 8 workgroups per CU, so that
-  // groups of uneven cost keep every CU busy)
-  int per_cu = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, s.func, s.block,
-                                                   0) != hipSuccess)
-    per_cu = 0;
-  return (unsigned)(std::max(per_cu, 8) * c->graph.cus);
-}
-
 int graph_capture(Ctx *c, const NodeSpec *sp, int ns) {
   auto &G = c->graph;
   free_graph(c);
-  for (int i = 0; i < ns; ++i) {
-    G.func[i] = sp[i].func;
-    G.block[i] = sp[i].block;
-    G.grid[i] = grid_of(c, sp[i]);
-  }
+  for (int i = 0; i < ns; ++i) G.func[i] = sp[i].func;
   FSPH_HIP(c, hipStreamBeginCapture(c->stream,
                                     hipStreamCaptureModeThreadLocal));
-  // recorded, not run: counters cleared by a kernel (no memset nodes)
-  k_zero_u64<<<1, 64, 0, c->stream>>>(
-      G.counters.as<unsigned long long>(), 4);
-  hipError_t e = hipGetLastError();
+  hipError_t e = hipSuccess;  // recorded, not run
   for (int i = 0; i < ns && e == hipSuccess; ++i) {
     if (i == ns - 1 && c->p.adaptive_dt && step_graph_seg_init(c))
       e = hipErrorUnknown;
     if (e == hipSuccess)
-      e = hipLaunchKernel(sp[i].func, dim3(G.grid[i]), dim3(G.block[i]),
+      e = hipLaunchKernel(sp[i].func, dim3(sp[i].grid), dim3(sp[i].block),
                           const_cast<void **>(sp[i].args), 0, c->stream);
   }
   hipGraph_t g = nullptr;
@@ -176,8 +152,8 @@ int graph_step_tail(Ctx *c) {
   for (int i = 0; i < ns; ++i) {
     hipKernelNodeParams kp{};
     kp.func = const_cast<void *>(G.func[i]);
-    kp.gridDim = dim3(G.grid[i]);
-    kp.blockDim = dim3(G.block[i]);
+    kp.gridDim = dim3(sp[i].grid);
+    kp.blockDim = dim3(sp[i].block);
     kp.sharedMemBytes = 0;
     kp.kernelParams = sp[i].args;
     kp.extra = nullptr;

@@ -74,7 +74,7 @@ struct Ctx;
 
 // graph argument slots (bytes each) and their order
 constexpr size_t kGraphSlot = 1024;
-enum : int { kSlotDens = 0, kSlotVsig, kSlotAcc, kSlotDudt, kSlotStep,
+enum : int { kSlotDens = 0, kSlotAcc, kSlotDudt, kSlotStep,
              kNSlots };
 
 // Persistent per-particle fields.  FP64 fields are double; derived fields
@@ -229,13 +229,11 @@ struct Ctx {
     hipGraphExec_t exec = nullptr;
     // chunk and width, rsize, adaptive_dt, n_inst, thermokinetic
     int key[5] = {0, 0, 0, 0, 0};
-    DBuf counters;               // work counters of the pair passes
     std::vector<char> host;      // host staging of the kernel arguments
     int cus = 0;
     static constexpr int kNodes = 8;  // replayed kernels, in launch order
     hipGraphNode_t node[kNodes] = {};
     const void *func[kNodes] = {};
-    unsigned grid[kNodes] = {}, block[kNodes] = {};
     int n_nodes = 0;
   } graph;
 
@@ -417,14 +415,12 @@ int batch_reduce(Ctx *c, int what);
 int batch_segments(Ctx *c);
 int batch_roots(Ctx *c);
 // graph mode: host staging of the kernel arguments of one step (k_sph.hip:
-// the four pair passes, with the eager passes' buffer rotations; k_step.hip:
-// kicks, h, dt), the persistent kernels for the current configuration
-// (pass = slot index; what: 0 kick v, 1 kick u, 2 h, 3 dt minimum) and the
-// per-pass work descriptor
+// the pair passes, with the eager passes' buffer rotations; k_step.hip:
+// kicks, h, dt) and the kernels for the current configuration (pass = slot
+// index; what: 0 kick v, 1 kick u, 2 h, 3 dt minimum)
 void sph_graph_args(Ctx *c, char *slots);
 const void *sph_graph_func(const Ctx *c, int pass);
 unsigned sph_graph_block(const Ctx *c);  // threads of the pair kernels
-void sph_graph_work(Ctx *c, int pass, void *work);
 void step_graph_args(Ctx *c, char *slots);
 const void *step_graph_func(const Ctx *c, int what);
 int step_graph_seg_init(Ctx *c);

@@ -860,51 +860,6 @@ __global__ __launch_bounds__(NT) void k_force(ForceArgs<T, MODE> a) {
   force_group<T, MODE, CH, NT, VS, VISC>(a, xcd_item(blockIdx.x, gridDim.x));
 }
 
-// Persistent form (for graph replay): a grid of resident size whose
-// workgroups take groups from a work counter until all ng are done.  The
-// arguments are kernel arguments (held in scalar registers, as in the
-// one-group-per-workgroup form); a replayed graph gets each step's values
-// through its kernel-node parameters.
-struct Work {
-  unsigned long long *counter;  // zeroed before the launch
-  int64_t ng;
-};
-
-// Next group of a persistent workgroup (uniform over the workgroup).
-__device__ inline int64_t next_group(const Work &w, int64_t *s_g) {
-  if (threadIdx.x == 0) *s_g = (int64_t)atomicAdd(w.counter, 1ull);
-  __syncthreads();
-  const int64_t g = *s_g;
-  __syncthreads();
-  return g;
-}
-
-template <class T, int CH, int NT>
-__global__ __launch_bounds__(NT) void k_density_p(DensArgs<T> a, Work w) {
-  __shared__ int64_t s_g;
-  for (int64_t g; (g = next_group(w, &s_g)) < w.ng;) {
-    density_group<T, CH, NT>(a, g);
-    __syncthreads();
-  }
-}
-template <class T, int CH, int NT>
-__global__ __launch_bounds__(NT) void k_vsig_p(VsigArgs<T> a, Work w) {
-  __shared__ int64_t s_g;
-  for (int64_t g; (g = next_group(w, &s_g)) < w.ng;) {
-    vsig_group<T, false, CH, NT>(a, g);
-    __syncthreads();
-  }
-}
-template <class T, int MODE, int CH, int NT, int VS = 0>
-__global__ __launch_bounds__(NT) void k_force_p(ForceArgs<T, MODE> a,
-                                                Work w) {
-  __shared__ int64_t s_g;
-  for (int64_t g; (g = next_group(w, &s_g)) < w.ng;) {
-    force_group<T, MODE, CH, NT, VS>(a, g);
-    __syncthreads();
-  }
-}
-
 // Calls f(CH, NT) (as std::integral_constant values) for the context's
 // chunk and workgroup width: one wavefront for tiles of at most 64 rows,
 // two otherwise.
@@ -1095,21 +1050,18 @@ template <class T, int MODE, int VS = 0> int force_impl(Ctx *c) {
 }
 
 // ---- graph mode -------------------------------------------------------------
-// Host side of the four pair passes of one step, in the eager order (with
+// Host side of the pair passes of one step, in the eager order (with
 // the same buffer rotations), written into the host staging of the graph's
 // argument slots.
 template <class T> void sph_graph_args_t(Ctx *c, char *slots) {
   static_assert(sizeof(DensArgs<T>) <= kGraphSlot, "slot");
   static_assert(sizeof(ForceArgs<T, kDudt>) <= kGraphSlot, "slot");
-  static_assert(sizeof(DensArgs<T>) <= kGraphSlot, "slot");
   std::swap(c->f[PF_C], c->f[PF_COLD]);
   const DensArgs<T> d = dens_args<T>(c);
-  const VsigArgs<T> v = vsig_args<T>(c);
   const ForceArgs<T, kAccel> fa = force_args<T, kAccel>(c);
   // the energy pass's arguments have the same layout in both formulations
   const ForceArgs<T, kDudt> fd = force_args<T, kDudt>(c);
   std::memcpy(slots + kSlotDens * kGraphSlot, &d, sizeof(d));
-  std::memcpy(slots + kSlotVsig * kGraphSlot, &v, sizeof(v));
   std::memcpy(slots + kSlotAcc * kGraphSlot, &fa, sizeof(fa));
   std::memcpy(slots + kSlotDudt * kGraphSlot, &fd, sizeof(fd));
   std::swap(c->f[PF_P], c->g[PF_P]);
@@ -1120,13 +1072,12 @@ template <class T, int CH, int NT>
 const void *sph_graph_func_t(int pass, bool tk) {
   switch (pass) {
     case kSlotDens:
-      return reinterpret_cast<const void *>(k_density_p<T, CH, NT>);
-    case kSlotVsig: return reinterpret_cast<const void *>(k_vsig_p<T, CH, NT>);
+      return reinterpret_cast<const void *>(k_density<T, CH, NT>);
     case kSlotAcc:
-      return reinterpret_cast<const void *>(k_force_p<T, kAccel, CH, NT, 1>);
+      return reinterpret_cast<const void *>(k_force<T, kAccel, CH, NT, 1>);
     default:
-      return tk ? reinterpret_cast<const void *>(k_force_p<T, kDedt, CH, NT>)
-                : reinterpret_cast<const void *>(k_force_p<T, kDudt, CH, NT>);
+      return tk ? reinterpret_cast<const void *>(k_force<T, kDedt, CH, NT>)
+                : reinterpret_cast<const void *>(k_force<T, kDudt, CH, NT>);
   }
 }
 
@@ -1154,11 +1105,6 @@ const void *sph_graph_func(const Ctx *c, int pass) {
 }
 
 unsigned sph_graph_block(const Ctx *c) { return narrow(c) ? 64u : 128u; }
-
-void sph_graph_work(Ctx *c, int pass, void *work) {
-  const Work w{c->graph.counters.as<unsigned long long>() + pass, c->nt};
-  std::memcpy(work, &w, sizeof(w));
-}
 
 int stage_density(Ctx *c) {
   return c->rsize == 4 ? density_impl<float>(c, true)
