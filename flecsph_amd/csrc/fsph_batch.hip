@@ -22,7 +22,7 @@
 using fsph::Ctx;
 
 namespace fsph {
-int upload_particles(Ctx *c, const fsph_particles *in);
+int upload_sets(Ctx *c, const fsph_particles *sets, int ns);
 }
 
 namespace {
@@ -194,45 +194,19 @@ int fsph_upload_batch(fsph_ctx *ctx, const fsph_particles *parts,
   }
   if (n >= (int64_t)1 << 31)
     return fsph::fail(c, FSPH_E_ARG, "total particles must be below 2^31");
-  // concatenate on the host, then upload as one set
-  std::vector<double> d[12];
-  std::vector<int64_t> id((size_t)n);
-  std::vector<int32_t> inst((size_t)n);
-  for (int f = 0; f < 12; ++f)
-    d[f].resize(f < 9 || opt[f - 9] ? (size_t)n : 0);
-  int64_t o = 0;
+  FSPH_TRY(fsph::upload_sets(c, parts, n_inst));
   std::vector<int64_t> segr(n_inst + 1, 0);
   for (int i = 0; i < n_inst; ++i) {
-    const fsph_particles &q = parts[i];
-    const double *src[12] = {q.x, q.y, q.z, q.vx, q.vy, q.vz, q.u,
-                             q.h, q.m, q.rho, q.P, q.c};
-    for (int f = 0; f < 12; ++f)
-      if (src[f]) std::memcpy(d[f].data() + o, src[f], (size_t)q.n * 8);
-    std::memcpy(id.data() + o, q.id, (size_t)q.n * 8);
-    for (int64_t k = 0; k < q.n; ++k) inst[(size_t)(o + k)] = i;
-    B.n_real[i] = q.n;
-    segr[i] = o;
-    o += q.n;
+    B.n_real[i] = parts[i].n;
+    segr[i + 1] = segr[i] + parts[i].n;
   }
-  segr[n_inst] = n;
-  fsph_particles all{};
-  all.n = n;
-  all.x = d[0].data(); all.y = d[1].data(); all.z = d[2].data();
-  all.vx = d[3].data(); all.vy = d[4].data(); all.vz = d[5].data();
-  all.u = d[6].data(); all.h = d[7].data(); all.m = d[8].data();
-  all.id = id.data();
-  all.rho = opt[0] ? d[9].data() : nullptr;
-  all.P = opt[1] ? d[10].data() : nullptr;
-  all.c = opt[2] ? d[11].data() : nullptr;
-  FSPH_TRY(fsph::upload_particles(c, &all));
-  FSPH_HIP(c, hipMemcpyAsync(c->f[fsph::PF_INST].p, inst.data(),
-                             (size_t)n * 4, hipMemcpyHostToDevice, c->stream));
   FSPH_HIP(c, hipMemcpyAsync(B.nreal.p, B.n_real.data(), (size_t)n_inst * 8,
                              hipMemcpyHostToDevice, c->stream));
   FSPH_HIP(c, hipMemcpyAsync(B.segr.p, segr.data(), (size_t)(n_inst + 1) * 8,
                              hipMemcpyHostToDevice, c->stream));
   FSPH_HIP(c, hipMemcpyAsync(B.seg.p, segr.data(), (size_t)(n_inst + 1) * 8,
                              hipMemcpyHostToDevice, c->stream));
+  FSPH_TRY(fsph::batch_index(c));
   B.seg_h = segr;
   B.dt_h.assign(n_inst, c->p.initial_dt);
   B.t_h.assign(n_inst, 0.0);

@@ -126,6 +126,10 @@ struct Ctx {
   DBuf flags;          // int error flags
   DBuf mail;           // device mailbox: scalars read back in one copy
   int64_t *mail_h = nullptr;  // its pinned host copy (kMail words)
+  // pinned halves that gather the small sets of an upload (on first use)
+  char *stage_h = nullptr;
+  int stage_half = 0;
+  hipEvent_t stage_ev[2] = {nullptr, nullptr};
   DBuf range_d;        // range of the last key computation: lo[3], hi[3]
   bool range_pending = false;  // range_d newer than lo/hi
   double lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};
@@ -403,6 +407,10 @@ int put_time(Ctx *c);      // tstate := host dt, totaltime, totaltime_next
 int sync_time(Ctx *c);     // host copies := tstate (waits) if time_dirty
 int stage_dt_rule(Ctx *c); // dt minimum and set_adaptive_timestep's rule
 int stage_advance(Ctx *c); // totaltime := totaltime_next (or += dt)
+// the derived state of n freshly uploaded particles (k_step.hip); rho, P and
+// c are device arrays or null (zero)
+int stage_upload_init(Ctx *c, int64_t n, const double *rho, const double *P,
+                      const double *cs);
 int convert_from_double(Ctx *c, const double *src, float *dst, int64_t n);
 int convert_to_double(Ctx *c, const void *src, size_t esize, double *dst,
                       int64_t n);              // k_step.hip
@@ -414,6 +422,8 @@ int batch_reduce(Ctx *c, int what);
 // seg[] from the sorted instance indices; root[] from the tree
 int batch_segments(Ctx *c);
 int batch_roots(Ctx *c);
+// PF_INST of freshly uploaded particles from segr
+int batch_index(Ctx *c);
 // graph mode: host staging of the kernel arguments of one step (k_sph.hip:
 // the pair passes, with the eager passes' buffer rotations; k_step.hip:
 // kicks, h, dt) and the kernels for the current configuration (pass = slot

@@ -392,6 +392,23 @@ __global__ __launch_bounds__(kT) void k_seg_bounds(
   if (i == n - 1) seg[ni] = n;
 }
 
+// instance of each particle from the instances' offsets (seg[ni] = n)
+__global__ __launch_bounds__(kT) void k_seg_index(
+    const int64_t *__restrict__ seg, int ni, int64_t n,
+    int32_t *__restrict__ inst) {
+  const int64_t i = (int64_t)blockIdx.x * kT + threadIdx.x;
+  if (i >= n) return;
+  int lo = 0, hi = ni - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (seg[mid] <= i)
+      lo = mid;
+    else
+      hi = mid - 1;
+  }
+  inst[i] = lo;
+}
+
 __global__ __launch_bounds__(kT) void k_seg_roots(
     const int64_t *__restrict__ seg, const int64_t *__restrict__ off,
     int ni, int32_t *__restrict__ root) {
@@ -827,6 +844,13 @@ int batch_segments(Ctx *c) {
   return 0;
 }
 
+int batch_index(Ctx *c) {
+  k_seg_index<<<blocks_for(c->n), kT, 0, c->stream>>>(
+      c->batch.segr.as<int64_t>(), c->batch.n_inst, c->n,
+      c->f[PF_INST].as<int32_t>());
+  return hip_check(c, hipGetLastError(), "k_seg_index");
+}
+
 int batch_roots(Ctx *c) {
   const int ni = c->batch.n_inst;
   k_seg_roots<<<(ni + kT - 1) / kT, kT, 0, c->stream>>>(
@@ -890,6 +914,62 @@ int convert_to_double(Ctx *c, const void *src, size_t esize, double *dst,
     k_to_double<double><<<blocks_for(n), kT, 0, c->stream>>>(
         static_cast<const double *>(src), dst, n);
   return hip_check(c, hipGetLastError(), "k_to_double");
+}
+
+// State that an upload does not carry: half-step velocities equal to the
+// velocities, rho, P and c in the context's precision, zero elsewhere.
+namespace {
+template <class T> struct UploadArgs {
+  const double *vx, *vy, *vz, *rho, *P, *c;
+  double *vhx, *vhy, *vhz, *e;
+  T *rho_o, *P_o, *c_o, *zero[15];
+  int32_t *izero[3];
+};
+
+template <class T>
+__global__ __launch_bounds__(kT) void k_upload_init(UploadArgs<T> a,
+                                                    int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * kT + threadIdx.x;
+  if (i >= n) return;
+  a.vhx[i] = a.vx[i];
+  a.vhy[i] = a.vy[i];
+  a.vhz[i] = a.vz[i];
+  a.e[i] = 0.0;
+  a.rho_o[i] = a.rho ? (T)a.rho[i] : T(0);
+  a.P_o[i] = a.P ? (T)a.P[i] : T(0);
+  a.c_o[i] = a.c ? (T)a.c[i] : T(0);
+#pragma unroll
+  for (int q = 0; q < 15; ++q) a.zero[q][i] = T(0);
+#pragma unroll
+  for (int q = 0; q < 3; ++q) a.izero[q][i] = 0;
+}
+
+template <class T>
+int upload_init(Ctx *c, int64_t n, const double *rho, const double *P,
+                const double *cs) {
+  UploadArgs<T> a{c->f[PF_VX].as<double>(),  c->f[PF_VY].as<double>(),
+                  c->f[PF_VZ].as<double>(),  rho,
+                  P,                         cs,
+                  c->f[PF_VHX].as<double>(), c->f[PF_VHY].as<double>(),
+                  c->f[PF_VHZ].as<double>(), c->f[PF_E].as<double>(),
+                  c->f[PF_RHO].as<T>(),      c->f[PF_P].as<T>(),
+                  c->f[PF_C].as<T>(),        {},
+                  {}};
+  const int z[15] = {PF_VSIG, PF_AX,  PF_AY,   PF_AZ,   PF_DUDT,
+                     PF_GX,   PF_GY,  PF_GZ,   PF_PHI,  PF_COLD,
+                     PF_LDIV, PF_DLH, PF_DEDT, PF_DIVV, PF_DDIVV};
+  for (int q = 0; q < 15; ++q) a.zero[q] = c->f[z[q]].as<T>();
+  const int zi[3] = {PF_NNGB, PF_HNGB, PF_HITER};
+  for (int q = 0; q < 3; ++q) a.izero[q] = c->f[zi[q]].as<int32_t>();
+  k_upload_init<T><<<blocks_for(n), kT, 0, c->stream>>>(a, n);
+  return hip_check(c, hipGetLastError(), "k_upload_init");
+}
+}  // namespace
+
+int stage_upload_init(Ctx *c, int64_t n, const double *rho, const double *P,
+                      const double *cs) {
+  return c->rsize == 4 ? upload_init<float>(c, n, rho, P, cs)
+                       : upload_init<double>(c, n, rho, P, cs);
 }
 
 int convert_from_double(Ctx *c, const double *src, float *dst, int64_t n) {

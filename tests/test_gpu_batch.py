@@ -318,3 +318,28 @@ def test_open_instance_in_a_periodic_batch_equals_its_own_run():
             assert np.array_equal(b.instance_get(i, f)[o], ref[f]), (i, f)
         assert b.instance_time(i) == ref["time"], i
     b.close()
+
+
+@pytest.mark.parametrize("precision", [_abi.PREC_FP32, _abi.PREC_FP64])
+def test_upload_of_small_and_large_sets(precision):
+    """Small sets of a batch go to the device through a pinned buffer (more
+    than its two halves hold here), large ones directly; every field arrives
+    in order, rho, P and c in the context's precision."""
+    rng = np.random.default_rng(3)
+    sizes = [2, 7000, 8191, 8192, 8193] + [7500] * 40 + [30000, 3]
+    sets = []
+    for n in sizes:
+        d = {k: rng.random(n) for k in ("x", "y", "z", "vx", "vy", "vz", "u",
+                                        "h", "m", "rho", "P", "c")}
+        d["id"] = rng.permutation(n)
+        sets.append(d)
+    s = BatchSystem(_abi.default_params(precision=precision), len(sizes))
+    s.upload(sets)
+    for f in ("x", "vz", "vhy", "u", "h", "m", "id", "rho", "P", "c"):
+        want = np.concatenate([d["vy" if f == "vhy" else f] for d in sets])
+        if precision == _abi.PREC_FP32 and f in ("rho", "P", "c"):
+            want = want.astype(np.float32)
+        assert np.array_equal(s.get(f), want), f
+    for f in ("ax", "dudt", "phi", "nngb", "e"):
+        assert not s.get(f).any(), f
+    s.close()
