@@ -180,7 +180,8 @@ __global__ __launch_bounds__(KB) void k_newton(NewtonArgs<T> a) {
         sid[j] = b;
       }
       const uint32_t *src = a.mask + mo + (int64_t)(c0 >> 5) * gc;
-      for (int q = t; q < nw * gc; q += KB) smask[q] = src[q];
+      for (int q = t; q < CHW * gc; q += KB)
+        smask[q] = q < nw * gc ? src[q] : 0u;
       __syncthreads();
       const int np = schedule(S, smask, nw, gc, eval);
       double wx = 0, wy = 0, wz = 0, wh2 = 0, wlo2 = 0, whi2 = 0;
@@ -188,7 +189,7 @@ __global__ __launch_bounds__(KB) void k_newton(NewtonArgs<T> a) {
       int wk = 0, rc = 0;
       int32_t wia = 0;
       KSum<T> r0, r1;
-      walk_run(
+      walk_run<CH>(
           S, smask, gc, np,
           [&](int k) {
             wx = qx[k]; wy = qy[k]; wz = qz[k];
@@ -199,7 +200,8 @@ __global__ __launch_bounds__(KB) void k_newton(NewtonArgs<T> a) {
             wk = k;
             wia = (int32_t)(gs + k);
           },
-          [&](int j) {
+          [&](int j, bool valid) {
+            if (!valid) return;
             const double d0 = wx - sx[j], d1 = wy - sy[j], d2 = wz - sz[j];
             const double rr2 = d0 * d0 + d1 * d1 + d2 * d2;
             if (!final_pass && rr2 >= wlo2 && rr2 <= whi2) {
@@ -223,9 +225,9 @@ __global__ __launch_bounds__(KB) void k_newton(NewtonArgs<T> a) {
             r0.add(sm[j] * W);
             r1.add(sm[j] * (-(T(3) * W + rdW) * wih));
           },
-          [&](int k, int kind) {
-            put(R, 0, k, kind, r0.s - r0.c);
-            put(R, 1, k, kind, r1.s - r1.c);
+          [&](int k) {
+            put(R, 0, k, r0.s - r0.c);
+            put(R, 1, k, r1.s - r1.c);
             r0 = KSum<T>();
             r1 = KSum<T>();
             if (rc) atomicAdd(&rcnt[k], rc);

@@ -154,12 +154,14 @@ __device__ inline Grp grp_of(const Tiles &t, int64_t g) {
   return c;
 }
 
-// Stages the chunk's mask words ([word][particle] layout, contiguous) in LDS.
-template <int NT>
+// Stages the chunk's mask words ([word][particle] layout, contiguous) in
+// LDS; words past the tile's end are zero.
+template <int NT, int CH>
 __device__ inline void stage_masks(const Tiles &t, const Grp &c, int c0,
                                    int nw, uint32_t *smask) {
   const uint32_t *src = t.mask + c.mo + (int64_t)(c0 >> 5) * c.gc;
-  for (int q = threadIdx.x; q < nw * c.gc; q += NT) smask[q] = src[q];
+  for (int q = threadIdx.x; q < CH / 32 * c.gc; q += NT)
+    smask[q] = q < nw * c.gc ? src[q] : 0u;
 }
 
 // ---------------------------------------------------------------------------
@@ -215,36 +217,37 @@ __device__ inline void density_group(const DensArgs<T> &a, int64_t g) {
       sz[j] = (P)(a.z[b] - oz);
       sh[j] = (T)a.h[b]; sm[j] = (T)a.m[b];
     }
-    stage_masks<NT>(a.t, c, c0, nw, smask);
+    stage_masks<NT, CH>(a.t, c, c0, nw, smask);
     __syncthreads();
     const int np = schedule(S, smask, nw, c.gc);
     P px = 0, py = 0, pz = 0;
     T ph = 1;
     KSum<T> acc, ag[3];
-    walk_run(
+    walk_run<CH>(
         S, smask, c.gc, np,
         [&](int k) { px = qx[k]; py = qy[k]; pz = qz[k]; ph = qh[k]; },
-        [&](int j) {
+        [&](int j, bool valid) {
           const T dx = (T)(px - sx[j]), dy = (T)(py - sy[j]),
                   dz = (T)(pz - sz[j]);
           const T r2 = dx * dx + dy * dy + dz * dz;
           const T ir = r2 > T(0) ? rsq(r2) : T(0);
           const T r = r2 * ir;
           const T ih = rcp(T(0.5) * (ph + sh[j]));
-          acc.add(sm[j] * kernel_W<T>(a.ph.kernel, r, ih));
+          const T mb = valid ? sm[j] : T(0);
+          acc.add(mb * kernel_W<T>(a.ph.kernel, r, ih));
           if (CULL) {
-            const T mf = sm[j] * kernel_F<T>(a.ph.kernel, r, ir, ih);
+            const T mf = mb * kernel_F<T>(a.ph.kernel, r, ir, ih);
             ag[0].add(mf * dx);
             ag[1].add(mf * dy);
             ag[2].add(mf * dz);
           }
         },
-        [&](int k, int kind) {
-          put(R, 0, k, kind, acc.s - acc.c);
+        [&](int k) {
+          put(R, 0, k, acc.s - acc.c);
           acc = KSum<T>();
           if (CULL)
             for (int d = 0; d < 3; ++d) {
-              put(R, 1 + d, k, kind, ag[d].s - ag[d].c);
+              put(R, 1 + d, k, ag[d].s - ag[d].c);
               ag[d] = KSum<T>();
             }
         });
@@ -335,13 +338,13 @@ __device__ inline void vsig_group(const VsigArgs<T> &a, int64_t g) {
         sm[j] = (T)a.m[b];
       }
     }
-    stage_masks<NT>(a.t, c, c0, nw, smask);
+    stage_masks<NT, CH>(a.t, c, c0, nw, smask);
     __syncthreads();
     const int np = schedule(S, smask, nw, c.gc);
     P px = 0, py = 0, pz = 0;
     T pvx = 0, pvy = 0, pvz = 0, pc = 0, ph = 1, rvs = 0, rdv = 0;
     int32_t ia = 0;
-    walk_run(
+    walk_run<CH>(
         S, smask, c.gc, np,
         [&](int k) {
           px = qx[k]; py = qy[k]; pz = qz[k];
@@ -350,10 +353,11 @@ __device__ inline void vsig_group(const VsigArgs<T> &a, int64_t g) {
           if (DIV) ph = qh[k];
           ia = (int32_t)(c.gs + k);
         },
-        [&](int j) {
+        [&](int j, bool valid) {
           // coincident pairs (m_b := 0, default_physics.h:378) add 0
           const P ddx = px - sx[j], ddy = py - sy[j], ddz = pz - sz[j];
-          const bool same = ddx == P(0) && ddy == P(0) && ddz == P(0);
+          const bool same =
+              !valid || (ddx == P(0) && ddy == P(0) && ddz == P(0));
           const T dx = (T)ddx, dy = (T)ddy, dz = (T)ddz;
           const T r2 = dx * dx + dy * dy + dz * dz;
           const T ir = same ? T(0) : rsq(r2);
@@ -369,9 +373,9 @@ __device__ inline void vsig_group(const VsigArgs<T> &a, int64_t g) {
             rdv += sm[j] * vdr * kernel_F<T>(a.kernel, r2 * ir, ir, ih);
           }
         },
-        [&](int k, int kind) {
-          put(R, 0, k, kind, rvs);
-          if (DIV) put(R, NV - 1, k, kind, rdv);
+        [&](int k) {
+          put(R, 0, k, rvs);
+          if (DIV) put(R, NV - 1, k, rdv);
           rvs = 0;
           rdv = 0;
         });
@@ -452,7 +456,7 @@ __device__ inline void alpha_group(const AlphaArgs<T> &a, int64_t g) {
       const T dv = a.divv[b];  // signnum_c (viscosity.h:63-67)
       ssg[j] = dv > T(0) ? T(1) : (dv < T(0) ? T(-1) : dv);
     }
-    stage_masks<NT>(a.t, c, c0, nw, smask);
+    stage_masks<NT, CH>(a.t, c, c0, nw, smask);
     __syncthreads();
     const int np = schedule(S, smask, nw, c.gc);
     P px = 0, py = 0, pz = 0;
@@ -460,16 +464,17 @@ __device__ inline void alpha_group(const AlphaArgs<T> &a, int64_t g) {
     T acc[NV - 1];
 #pragma unroll
     for (int q = 0; q < NV - 1; ++q) acc[q] = 0;
-    walk_run(
+    walk_run<CH>(
         S, smask, c.gc, np,
         [&](int k) {
           px = qx[k]; py = qy[k]; pz = qz[k];
           pvx = qvx[k]; pvy = qvy[k]; pvz = qvz[k];
           pc = qc[k]; ph = qh[k];
         },
-        [&](int j) {
+        [&](int j, bool valid) {
           const P ddx = px - sx[j], ddy = py - sy[j], ddz = pz - sz[j];
-          const bool same = ddx == P(0) && ddy == P(0) && ddz == P(0);
+          const bool same =
+              !valid || (ddx == P(0) && ddy == P(0) && ddz == P(0));
           const T d[3] = {(T)ddx, (T)ddy, (T)ddz};
           const T r2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
           const T ir = same ? T(0) : rsq(r2);
@@ -480,19 +485,20 @@ __device__ inline void alpha_group(const AlphaArgs<T> &a, int64_t g) {
           const T v = same ? T(0) : cab - (vdn < T(0) ? vdn : T(0));
           rvs = rvs < v ? v : rvs;
           const T ih = rcp(T(0.5) * (ph + sh[j]));
-          acc[0] += ssg[j] * sm[j] * kernel_W<T>(a.kernel, r, ih);
-          const T mf = sm[j] * kernel_F<T>(a.kernel, r, ir, ih);
+          const T mb = valid ? sm[j] : T(0);
+          acc[0] += ssg[j] * mb * kernel_W<T>(a.kernel, r, ih);
+          const T mf = mb * kernel_F<T>(a.kernel, r, ir, ih);
 #pragma unroll
           for (int p = 0; p < 3; ++p)
 #pragma unroll
             for (int q = 0; q < 3; ++q) acc[1 + 3 * p + q] -= mf * vab[p] * d[q];
         },
-        [&](int k, int kind) {
-          put(R, 0, k, kind, rvs);
+        [&](int k) {
+          put(R, 0, k, rvs);
           rvs = 0;
 #pragma unroll
           for (int q = 0; q < NV - 1; ++q) {
-            put(R, 1 + q, k, kind, acc[q]);
+            put(R, 1 + q, k, acc[q]);
             acc[q] = 0;
           }
         });
@@ -719,7 +725,7 @@ __device__ inline void force_group(const ForceArgs<T, MODE> &a, int64_t g) {
 #pragma unroll
     for (int q = 0; q < MPER; ++q) {
       const int w = t + q * NT;
-      if (w < nw * c.gc) smask[w] = pm[q];
+      if (w < CH / 32 * c.gc) smask[w] = pm[q];
     }
     __syncthreads();
     if (c0 + CH < c.cc) {
@@ -732,7 +738,7 @@ __device__ inline void force_group(const ForceArgs<T, MODE> &a, int64_t g) {
     T ph = 1, prho = 1, pprho2 = 0, pc = 0, rvs = 0, rdv = 0, pal = 0;
     int32_t ia = 0;
     KSum<T> s[NS];
-    walk_run(
+    walk_run<CH>(
         S, smask, c.gc, np,
         [&](int k) {
           px = qx[k]; py = qy[k]; pz = qz[k];
@@ -744,11 +750,13 @@ __device__ inline void force_group(const ForceArgs<T, MODE> &a, int64_t g) {
           if (VISC) pal = qal[k];
           ia = (int32_t)(c.gs + k);
         },
-        [&](int j) {
-          // coincident pairs (m_b := 0, default_physics.h:378) add 0: with
-          // ir = 0, F = 0 and every term below is 0
+        [&](int j, bool valid) {
+          // coincident pairs (m_b := 0, default_physics.h:378) and pairs
+          // that are not valid add 0: with ir = 0, F = 0 and every term
+          // below is 0
           const P ddx = px - sx[j], ddy = py - sy[j], ddz = pz - sz[j];
-          const bool same = ddx == P(0) && ddy == P(0) && ddz == P(0);
+          const bool same =
+              !valid || (ddx == P(0) && ddy == P(0) && ddz == P(0));
           const T dx = (T)ddx, dy = (T)ddy, dz = (T)ddz;
           const T r2 = dx * dx + dy * dy + dz * dz;
           const T ir = same ? T(0) : rsq(r2);
@@ -798,14 +806,14 @@ __device__ inline void force_group(const ForceArgs<T, MODE> &a, int64_t g) {
             s[1].add(mv * Pi);
           }
         },
-        [&](int k, int kind) {
+        [&](int k) {
 #pragma unroll
           for (int n = 0; n < NS; ++n) {
-            put(R, n, k, kind, s[n].s - s[n].c);
+            put(R, n, k, s[n].s - s[n].c);
             s[n] = KSum<T>();
           }
-          if (VS) put(R, NS, k, kind, rvs);
-          if (VS == 2) put(R, NV - 1, k, kind, rdv);
+          if (VS) put(R, NS, k, rvs);
+          if (VS == 2) put(R, NV - 1, k, rdv);
           rvs = 0;
           rdv = 0;
         });

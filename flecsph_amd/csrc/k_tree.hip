@@ -390,8 +390,10 @@ __global__ __launch_bounds__(kT) void k_group_flags(
 }
 
 // Writes group g (its start, count and node) and its tiles: tile t0 =
-// g + (split groups before g) holds the first min(count, tw) rows, and a
-// split group's second tile t0 + 1 the rest.  The candidates of a group's
+// g + (split groups before g) holds its rows, or the first half of a split
+// group's, whose second half makes tile t0 + 1 (halves, not tw rows and the
+// rest: a tile's cost grows with its rows, and the longest of one wavefront
+// each bound the last part of a launch; @SPLIT@).  The candidates of a group's
 // only tile are in the group's slot g; a split group (s-th of them) has two
 // slots of its own, ng + 2 s and ng + 2 s + 1.
 __global__ __launch_bounds__(kT) void k_group_write(
@@ -421,12 +423,13 @@ __global__ __launch_bounds__(kT) void k_group_write(
   tgrp[t0] = (int32_t)g;
   tstart[t0] = st;
   tslot[t0] = (int32_t)g;
-  if (cnt > tw) {
-    tcount[t0] = tw;
+  if (cnt > tw) {  // (cnt <= 2 tw: groups hold at most 128 particles)
+    const int32_t half = (cnt + 1) / 2;
+    tcount[t0] = half;
     tslot[t0] = (int32_t)(ng + 2 * s);
     tgrp[t0 + 1] = (int32_t)g;
-    tstart[t0 + 1] = st + tw;
-    tcount[t0 + 1] = cnt - tw;
+    tstart[t0 + 1] = st + half;
+    tcount[t0 + 1] = cnt - half;
     tslot[t0 + 1] = (int32_t)(ng + 2 * s + 1);
   } else {
     tcount[t0] = cnt;
