@@ -235,8 +235,10 @@ __global__ __launch_bounds__(KB) void k_newton(NewtonArgs<T> a) {
           });
       __syncthreads();
       if (eval && S.off[t + 1] > S.off[t]) {
-        s0.add(row_total<false>(S, R, 0, t, np));
-        s1.add(row_total<false>(S, R, 1, t, np));
+        T v[2];
+        row_results<0u>(S, R, t, np, v);
+        s0.add(v[0]);
+        s1.add(v[1]);
       }
     }
     __syncthreads();  // counts and band entries of the pass are complete

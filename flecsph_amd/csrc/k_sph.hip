@@ -50,12 +50,19 @@ __device__ inline double rsq(double x) { return 1.0 / sqrt(x); }
 // group's first particle (one FP64 subtraction, one rounding: the error of a
 // pair difference is below 2^-24 of the particles' distance from that
 // origin, a few smoothing lengths), FP64 kernels absolute.
-template <class T> using Pos = typename std::conditional<sizeof(T) == 4, float,
-                                                         double>::type;
 template <class T> __device__ inline double pos_origin(const double *x,
                                                        int64_t gs) {
   return sizeof(T) == 4 ? x[gs] : 0.0;
 }
+
+// Four values of a candidate or row in LDS, read at once (ds_read_b128 in
+// FP32): a pair reads its candidate in a few wide loads, and an array of
+// them spreads random candidates over all banks.  With the kernel function a
+// template parameter (below) this took the acceleration pass from 265 to 227
+// us on Sedov 64^3, 586 to 496 on the 1M star and 955 to 795 on the 1.5M
+// collapse against one array per value.
+template <class T> struct alignas(4 * sizeof(T)) V4 { T a, b, c, d; };
+template <class T> struct alignas(2 * sizeof(T)) V2 { T a, b; };
 
 struct Phys {
   int kernel;
@@ -188,15 +195,12 @@ template <class T> struct DensArgs {
 };
 
 // CULL: also sum m_b grad W_ab for compute_divv
-template <class T, int CH, int NT, bool CULL = false>
+template <class T, int CH, int NT, int KERN, bool CULL = false>
 __device__ inline void density_group(const DensArgs<T> &a, int64_t g) {
-  using P = Pos<T>;
   constexpr int NV = CULL ? 4 : 1;
-  __shared__ P sx[CH], sy[CH], sz[CH];
-  __shared__ T sh[CH], sm[CH];
+  __shared__ V4<T> s0[CH], q0[NT];  // x y z h
+  __shared__ T sm[CH];
   __shared__ uint32_t smask[(CH / 32) * NT];
-  __shared__ P qx[NT], qy[NT], qz[NT];
-  __shared__ T qh[NT];
   __shared__ Sched<NT> S;
   __shared__ Parts<T, NV, NT> R;
   const Grp c = grp_of(a.t, g);
@@ -205,38 +209,36 @@ __device__ inline void density_group(const DensArgs<T> &a, int64_t g) {
                oz = pos_origin<T>(a.z, c.gs);
   if (t < c.gc) {
     const int64_t i = c.gs + t;
-    qx[t] = (P)(a.x[i] - ox); qy[t] = (P)(a.y[i] - oy);
-    qz[t] = (P)(a.z[i] - oz); qh[t] = (T)a.h[i];
+    q0[t] = V4<T>{(T)(a.x[i] - ox), (T)(a.y[i] - oy), (T)(a.z[i] - oz),
+                  (T)a.h[i]};
   }
   KSum<T> rho, gw[3];
   for (int c0 = 0; c0 < c.cc; c0 += CH) {
     const int nch = min(CH, c.cc - c0), nw = (nch + 31) >> 5;
     for (int j = t; j < nch; j += NT) {
       const int64_t b = a.t.cand[c.cb + c0 + j];
-      sx[j] = (P)(a.x[b] - ox); sy[j] = (P)(a.y[b] - oy);
-      sz[j] = (P)(a.z[b] - oz);
-      sh[j] = (T)a.h[b]; sm[j] = (T)a.m[b];
+      s0[j] = V4<T>{(T)(a.x[b] - ox), (T)(a.y[b] - oy), (T)(a.z[b] - oz),
+                    (T)a.h[b]};
+      sm[j] = (T)a.m[b];
     }
     stage_masks<NT, CH>(a.t, c, c0, nw, smask);
     __syncthreads();
     const int np = schedule(S, smask, nw, c.gc);
-    P px = 0, py = 0, pz = 0;
-    T ph = 1;
+    V4<T> p{0, 0, 0, 1};
     KSum<T> acc, ag[3];
     walk_run<CH>(
-        S, smask, c.gc, np,
-        [&](int k) { px = qx[k]; py = qy[k]; pz = qz[k]; ph = qh[k]; },
+        S, smask, c.gc, np, [&](int k) { p = q0[k]; },
         [&](int j, bool valid) {
-          const T dx = (T)(px - sx[j]), dy = (T)(py - sy[j]),
-                  dz = (T)(pz - sz[j]);
+          const V4<T> s = s0[j];
+          const T dx = p.a - s.a, dy = p.b - s.b, dz = p.c - s.c;
           const T r2 = dx * dx + dy * dy + dz * dz;
           const T ir = r2 > T(0) ? rsq(r2) : T(0);
           const T r = r2 * ir;
-          const T ih = rcp(T(0.5) * (ph + sh[j]));
+          const T ih = rcp(T(0.5) * (p.d + s.d));
           const T mb = valid ? sm[j] : T(0);
-          acc.add(mb * kernel_W<T>(a.ph.kernel, r, ih));
+          acc.add(mb * kernel_W<T>(KERN, r, ih));
           if (CULL) {
-            const T mf = mb * kernel_F<T>(a.ph.kernel, r, ir, ih);
+            const T mf = mb * kernel_F<T>(KERN, r, ir, ih);
             ag[0].add(mf * dx);
             ag[1].add(mf * dy);
             ag[2].add(mf * dz);
@@ -253,10 +255,11 @@ __device__ inline void density_group(const DensArgs<T> &a, int64_t g) {
         });
     __syncthreads();
     if (t < c.gc && S.off[t + 1] > S.off[t]) {
-      rho.add(row_total<false>(S, R, 0, t, np));
+      T v[NV];
+      row_results<0u>(S, R, t, np, v);
+      rho.add(v[0]);
       if (CULL)
-        for (int d = 0; d < 3; ++d)
-          gw[d].add(row_total<false>(S, R, 1 + d, t, np));
+        for (int d = 0; d < 3; ++d) gw[d].add(v[(1 + d) % NV]);
     }
   }
   if (t < c.gc) {
@@ -297,18 +300,22 @@ template <class T> struct VsigArgs {
   int kernel;
 };
 
-template <class T, bool DIV, int CH, int NT>
+// Candidate index relative to the tile's first particle, as a T: it is only
+// compared with rows of the tile, so it is clamped to just outside them.
+template <class T, int NT>
+__device__ inline T rel_index(int64_t b, int64_t gs) {
+  const int64_t r = b - gs;
+  return (T)(int)(r < -1 ? -1 : (r > NT ? NT : r));
+}
+
+template <class T, bool DIV, int CH, int NT, int KERN>
 __device__ inline void vsig_group(const VsigArgs<T> &a, int64_t g) {
-  using P = Pos<T>;
   constexpr int NV = DIV ? 2 : 1;
-  __shared__ P sx[CH], sy[CH], sz[CH];
-  __shared__ T svx[CH], svy[CH], svz[CH], scn[CH], sco[CH];
-  __shared__ T sh[DIV ? CH : 1], sm[DIV ? CH : 1];
-  __shared__ int32_t sid[CH];
+  // x y z, index relative to the tile; velocity, c; c_old, h, m
+  __shared__ V4<T> s0[CH], s1[CH], q0[NT], q1[NT];
+  __shared__ T sco[CH];
+  __shared__ V2<T> s2[DIV ? CH : 1];
   __shared__ uint32_t smask[(CH / 32) * NT];
-  __shared__ P qx[NT], qy[NT], qz[NT];
-  __shared__ T qvx[NT], qvy[NT], qvz[NT], qc[NT];
-  __shared__ T qh[DIV ? NT : 1];
   __shared__ Sched<NT> S;
   __shared__ Parts<T, NV, NT> R;
   const Grp c = grp_of(a.t, g);
@@ -317,60 +324,53 @@ __device__ inline void vsig_group(const VsigArgs<T> &a, int64_t g) {
                oz = pos_origin<T>(a.z, c.gs);
   if (t < c.gc) {
     const int64_t i = c.gs + t;
-    qx[t] = (P)(a.x[i] - ox); qy[t] = (P)(a.y[i] - oy);
-    qz[t] = (P)(a.z[i] - oz);
-    qvx[t] = (T)a.vx[i]; qvy[t] = (T)a.vy[i]; qvz[t] = (T)a.vz[i];
-    qc[t] = a.c[i];
-    if (DIV) qh[t] = (T)a.h[i];
+    q0[t] = V4<T>{(T)(a.x[i] - ox), (T)(a.y[i] - oy), (T)(a.z[i] - oz),
+                  DIV ? (T)a.h[i] : T(0)};
+    q1[t] = V4<T>{(T)a.vx[i], (T)a.vy[i], (T)a.vz[i], a.c[i]};
   }
   T vs = 0, dv = 0;  // thread t: particle t's totals
   for (int c0 = 0; c0 < c.cc; c0 += CH) {
     const int nch = min(CH, c.cc - c0), nw = (nch + 31) >> 5;
     for (int j = t; j < nch; j += NT) {
       const int32_t b = a.t.cand[c.cb + c0 + j];
-      sx[j] = (P)(a.x[b] - ox); sy[j] = (P)(a.y[b] - oy);
-      sz[j] = (P)(a.z[b] - oz);
-      svx[j] = (T)a.vx[b]; svy[j] = (T)a.vy[b]; svz[j] = (T)a.vz[b];
-      scn[j] = a.c[b]; sco[j] = a.c_old[b];
-      sid[j] = b;
-      if (DIV) {
-        sh[j] = (T)a.h[b];
-        sm[j] = (T)a.m[b];
-      }
+      s0[j] = V4<T>{(T)(a.x[b] - ox), (T)(a.y[b] - oy), (T)(a.z[b] - oz),
+                    rel_index<T, NT>(b, c.gs)};
+      s1[j] = V4<T>{(T)a.vx[b], (T)a.vy[b], (T)a.vz[b], a.c[b]};
+      sco[j] = a.c_old[b];
+      if (DIV) s2[j] = V2<T>{(T)a.h[b], (T)a.m[b]};
     }
     stage_masks<NT, CH>(a.t, c, c0, nw, smask);
     __syncthreads();
     const int np = schedule(S, smask, nw, c.gc);
-    P px = 0, py = 0, pz = 0;
-    T pvx = 0, pvy = 0, pvz = 0, pc = 0, ph = 1, rvs = 0, rdv = 0;
-    int32_t ia = 0;
+    V4<T> p{0, 0, 0, 1}, pv{0, 0, 0, 0};
+    T rvs = 0, rdv = 0, ia = 0;
     walk_run<CH>(
         S, smask, c.gc, np,
         [&](int k) {
-          px = qx[k]; py = qy[k]; pz = qz[k];
-          pvx = qvx[k]; pvy = qvy[k]; pvz = qvz[k];
-          pc = qc[k];
-          if (DIV) ph = qh[k];
-          ia = (int32_t)(c.gs + k);
+          p = q0[k];
+          pv = q1[k];
+          ia = (T)k;
         },
         [&](int j, bool valid) {
-          // coincident pairs (m_b := 0, default_physics.h:378) add 0
-          const P ddx = px - sx[j], ddy = py - sy[j], ddz = pz - sz[j];
-          const bool same =
-              !valid || (ddx == P(0) && ddy == P(0) && ddz == P(0));
-          const T dx = (T)ddx, dy = (T)ddy, dz = (T)ddz;
+          // coincident pairs (m_b := 0, default_physics.h:378) and pairs
+          // that are not valid add 0
+          const V4<T> s = s0[j], sv = s1[j];
+          const T co = sco[j];
+          const T dx = p.a - s.a, dy = p.b - s.b, dz = p.c - s.c;
+          const bool same = !valid || (dx == T(0) && dy == T(0) && dz == T(0));
           const T r2 = dx * dx + dy * dy + dz * dz;
           const T ir = same ? T(0) : rsq(r2);
           const T vdr =
-              (pvx - svx[j]) * dx + (pvy - svy[j]) * dy + (pvz - svz[j]) * dz;
+              (pv.a - sv.a) * dx + (pv.b - sv.b) * dy + (pv.c - sv.c) * dz;
           const T vdn = vdr * ir;
-          const T cb = sid[j] >= ia ? scn[j] : sco[j];
-          const T cab = pc < cb ? cb : pc;
+          const T cb = s.d >= ia ? sv.d : co;
+          const T cab = pv.d < cb ? cb : pv.d;
           const T v = same ? T(0) : cab - (vdn < T(0) ? vdn : T(0));
           rvs = rvs < v ? v : rvs;
           if (DIV) {
-            const T ih = rcp(T(0.5) * (ph + sh[j]));
-            rdv += sm[j] * vdr * kernel_F<T>(a.kernel, r2 * ir, ir, ih);
+            const V2<T> hm = s2[j];
+            const T ih = rcp(T(0.5) * (p.d + hm.a));
+            rdv += hm.b * vdr * kernel_F<T>(KERN, r2 * ir, ir, ih);
           }
         },
         [&](int k) {
@@ -381,9 +381,10 @@ __device__ inline void vsig_group(const VsigArgs<T> &a, int64_t g) {
         });
     __syncthreads();
     if (t < c.gc && S.off[t + 1] > S.off[t]) {
-      const T u = row_total<true>(S, R, 0, t, np);
-      vs = vs < u ? u : vs;
-      if (DIV) dv += row_total<false>(S, R, NV - 1, t, np);
+      T v[NV];
+      row_results<1u>(S, R, t, np, v);
+      vs = vs < v[0] ? v[0] : vs;
+      if (DIV) dv += v[NV - 1];
     }
   }
   if (t < c.gc) {
@@ -417,15 +418,13 @@ template <class T> struct AlphaArgs {
   double alpha_max, delta, l;
 };
 
-template <class T, int CH, int NT>
+template <class T, int CH, int NT, int KERN>
 __device__ inline void alpha_group(const AlphaArgs<T> &a, int64_t g) {
-  using P = Pos<T>;
   constexpr int NV = 11;  // vsig, R, G (9)
-  __shared__ P sx[CH], sy[CH], sz[CH];
-  __shared__ T svx[CH], svy[CH], svz[CH], sc[CH], sh[CH], sm[CH], ssg[CH];
+  // x y z h; velocity, c; m, sign(div v)
+  __shared__ V4<T> s0[CH], s1[CH], q0[NT], q1[NT];
+  __shared__ V2<T> s2[CH];
   __shared__ uint32_t smask[(CH / 32) * NT];
-  __shared__ P qx[NT], qy[NT], qz[NT];
-  __shared__ T qvx[NT], qvy[NT], qvz[NT], qc[NT], qh[NT];
   __shared__ Sched<NT> S;
   __shared__ Parts<T, NV, NT> R;
   const Grp c = grp_of(a.t, g);
@@ -434,11 +433,9 @@ __device__ inline void alpha_group(const AlphaArgs<T> &a, int64_t g) {
                oz = pos_origin<T>(a.z, c.gs);
   if (t < c.gc) {
     const int64_t i = c.gs + t;
-    qx[t] = (P)(a.x[i] - ox); qy[t] = (P)(a.y[i] - oy);
-    qz[t] = (P)(a.z[i] - oz);
-    qvx[t] = (T)a.vx[i]; qvy[t] = (T)a.vy[i]; qvz[t] = (T)a.vz[i];
-    qc[t] = a.c[i];
-    qh[t] = (T)a.h[i];
+    q0[t] = V4<T>{(T)(a.x[i] - ox), (T)(a.y[i] - oy), (T)(a.z[i] - oz),
+                  (T)a.h[i]};
+    q1[t] = V4<T>{(T)a.vx[i], (T)a.vy[i], (T)a.vz[i], a.c[i]};
   }
   T vs = 0, tot[NV - 1];  // thread t: particle t's totals
 #pragma unroll
@@ -447,47 +444,45 @@ __device__ inline void alpha_group(const AlphaArgs<T> &a, int64_t g) {
     const int nch = min(CH, c.cc - c0), nw = (nch + 31) >> 5;
     for (int j = t; j < nch; j += NT) {
       const int32_t b = a.t.cand[c.cb + c0 + j];
-      sx[j] = (P)(a.x[b] - ox); sy[j] = (P)(a.y[b] - oy);
-      sz[j] = (P)(a.z[b] - oz);
-      svx[j] = (T)a.vx[b]; svy[j] = (T)a.vy[b]; svz[j] = (T)a.vz[b];
-      sc[j] = a.c[b];
-      sh[j] = (T)a.h[b];
-      sm[j] = (T)a.m[b];
+      s0[j] = V4<T>{(T)(a.x[b] - ox), (T)(a.y[b] - oy), (T)(a.z[b] - oz),
+                    (T)a.h[b]};
+      s1[j] = V4<T>{(T)a.vx[b], (T)a.vy[b], (T)a.vz[b], a.c[b]};
       const T dv = a.divv[b];  // signnum_c (viscosity.h:63-67)
-      ssg[j] = dv > T(0) ? T(1) : (dv < T(0) ? T(-1) : dv);
+      s2[j] = V2<T>{(T)a.m[b],
+                    dv > T(0) ? T(1) : (dv < T(0) ? T(-1) : dv)};
     }
     stage_masks<NT, CH>(a.t, c, c0, nw, smask);
     __syncthreads();
     const int np = schedule(S, smask, nw, c.gc);
-    P px = 0, py = 0, pz = 0;
-    T pvx = 0, pvy = 0, pvz = 0, pc = 0, ph = 1, rvs = 0;
+    V4<T> p{0, 0, 0, 1}, pv{0, 0, 0, 0};
+    T rvs = 0;
     T acc[NV - 1];
 #pragma unroll
     for (int q = 0; q < NV - 1; ++q) acc[q] = 0;
     walk_run<CH>(
         S, smask, c.gc, np,
         [&](int k) {
-          px = qx[k]; py = qy[k]; pz = qz[k];
-          pvx = qvx[k]; pvy = qvy[k]; pvz = qvz[k];
-          pc = qc[k]; ph = qh[k];
+          p = q0[k];
+          pv = q1[k];
         },
         [&](int j, bool valid) {
-          const P ddx = px - sx[j], ddy = py - sy[j], ddz = pz - sz[j];
+          const V4<T> s = s0[j], sv = s1[j];
+          const V2<T> ms = s2[j];
+          const T d[3] = {p.a - s.a, p.b - s.b, p.c - s.c};
           const bool same =
-              !valid || (ddx == P(0) && ddy == P(0) && ddz == P(0));
-          const T d[3] = {(T)ddx, (T)ddy, (T)ddz};
+              !valid || (d[0] == T(0) && d[1] == T(0) && d[2] == T(0));
           const T r2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
           const T ir = same ? T(0) : rsq(r2);
           const T r = r2 * ir;
-          const T vab[3] = {pvx - svx[j], pvy - svy[j], pvz - svz[j]};
+          const T vab[3] = {pv.a - sv.a, pv.b - sv.b, pv.c - sv.c};
           const T vdn = (vab[0] * d[0] + vab[1] * d[1] + vab[2] * d[2]) * ir;
-          const T cab = pc < sc[j] ? sc[j] : pc;
+          const T cab = pv.d < sv.d ? sv.d : pv.d;
           const T v = same ? T(0) : cab - (vdn < T(0) ? vdn : T(0));
           rvs = rvs < v ? v : rvs;
-          const T ih = rcp(T(0.5) * (ph + sh[j]));
-          const T mb = valid ? sm[j] : T(0);
-          acc[0] += ssg[j] * mb * kernel_W<T>(a.kernel, r, ih);
-          const T mf = mb * kernel_F<T>(a.kernel, r, ir, ih);
+          const T ih = rcp(T(0.5) * (p.d + s.d));
+          const T mb = valid ? ms.a : T(0);
+          acc[0] += ms.b * mb * kernel_W<T>(KERN, r, ih);
+          const T mf = mb * kernel_F<T>(KERN, r, ir, ih);
 #pragma unroll
           for (int p = 0; p < 3; ++p)
 #pragma unroll
@@ -504,11 +499,11 @@ __device__ inline void alpha_group(const AlphaArgs<T> &a, int64_t g) {
         });
     __syncthreads();
     if (t < c.gc && S.off[t + 1] > S.off[t]) {
-      const T u = row_total<true>(S, R, 0, t, np);
-      vs = vs < u ? u : vs;
+      T v[NV];
+      row_results<1u>(S, R, t, np, v);
+      vs = vs < v[0] ? v[0] : vs;
 #pragma unroll
-      for (int q = 0; q < NV - 1; ++q)
-        tot[q] += row_total<false>(S, R, 1 + q, t, np);
+      for (int q = 0; q < NV - 1; ++q) tot[q] += v[1 + q];
     }
   }
   if (t >= c.gc) return;
@@ -543,9 +538,9 @@ __device__ inline void alpha_group(const AlphaArgs<T> &a, int64_t g) {
   }
 }
 
-template <class T, int CH, int NT>
+template <class T, int CH, int NT, int KERN>
 __global__ __launch_bounds__(NT) void k_alpha(AlphaArgs<T> a) {
-  alpha_group<T, CH, NT>(a, xcd_item(blockIdx.x, gridDim.x));
+  alpha_group<T, CH, NT, KERN>(a, xcd_item(blockIdx.x, gridDim.x));
 }
 
 // ---------------------------------------------------------------------------
@@ -612,26 +607,22 @@ __device__ inline void energy_tail(const ForceArgs<T, MODE> &a, int64_t i,
 // VISC: 0 the constant viscosity (viscosity.h:128-137), 1 the Cullen-Dehnen
 // form -alpha_ab (c_ab - 2 mu_ab) mu_ab / rho_ab with alpha_ab the mean of
 // the particles' alphas (viscosity.h:151-155, default_physics.h:375-379)
-template <class T, int MODE, int CH, int NT, int VS = 0, int VISC = 0>
+template <class T, int MODE, int CH, int NT, int KERN, int VS = 0,
+          int VISC = 0>
 __device__ inline void force_group(const ForceArgs<T, MODE> &a, int64_t g) {
-  using P = Pos<T>;
   constexpr bool DUDT = MODE != kAccel;  // an energy pass
   constexpr bool DEDT = MODE == kDedt;
   constexpr bool V = DUDT || VS > 0;  // velocities staged
   constexpr int NS = DEDT ? 1 : (DUDT ? 2 : 3);  // compensated sums
   constexpr int NV = NS + (VS > 0) + (VS == 2);
-  __shared__ P sx[CH], sy[CH], sz[CH];
-  __shared__ T svhx[CH], svhy[CH], svhz[CH];
-  __shared__ T svx[V ? CH : 1], svy[V ? CH : 1], svz[V ? CH : 1];
-  __shared__ T sh[CH], sm[CH], srho[CH], sprho2[CH], sc[CH];
-  __shared__ T sco[VS ? CH : 1];
-  __shared__ int32_t sid[VS ? CH : 1];
-  __shared__ T sal[VISC ? CH : 1], qal[VISC ? NT : 1];
+  // candidates: x y z h; half-step velocity, m; velocity, c_old; rho,
+  // P / rho^2, c, index relative to the tile; alpha
+  __shared__ V4<T> s0[CH], s1[CH], s2[V ? CH : 1], s3[CH];
+  __shared__ T sal[VISC ? CH : 1];
+  // rows: x y z h; half-step velocity, c; velocity, alpha; rho, P / rho^2
+  __shared__ V4<T> q0[NT], q1[NT], q2[V || VISC ? NT : 1];
+  __shared__ V2<T> q3[NT];
   __shared__ uint32_t smask[(CH / 32) * NT];
-  __shared__ P qx[NT], qy[NT], qz[NT];
-  __shared__ T qvhx[NT], qvhy[NT], qvhz[NT];
-  __shared__ T qvx[V ? NT : 1], qvy[V ? NT : 1], qvz[V ? NT : 1];
-  __shared__ T qh[NT], qrho[NT], qprho2[NT], qc[NT];
   __shared__ Sched<NT> S;
   __shared__ Parts<T, NV, NT> R;
   const Grp c = grp_of(a.t, g);
@@ -641,18 +632,14 @@ __device__ inline void force_group(const ForceArgs<T, MODE> &a, int64_t g) {
   const T alpha = (T)a.ph.alpha, beta = (T)a.ph.beta, eps = (T)a.ph.eps;
   if (t < c.gc) {
     const int64_t i = c.gs + t;
-    qx[t] = (P)(a.x[i] - ox); qy[t] = (P)(a.y[i] - oy);
-    qz[t] = (P)(a.z[i] - oz);
-    qvhx[t] = (T)a.vhx[i]; qvhy[t] = (T)a.vhy[i]; qvhz[t] = (T)a.vhz[i];
-    if (V) {
-      qvx[t] = (T)a.vx[i]; qvy[t] = (T)a.vy[i]; qvz[t] = (T)a.vz[i];
-    }
-    qh[t] = (T)a.h[i];
+    q0[t] = V4<T>{(T)(a.x[i] - ox), (T)(a.y[i] - oy), (T)(a.z[i] - oz),
+                  (T)a.h[i]};
+    q1[t] = V4<T>{(T)a.vhx[i], (T)a.vhy[i], (T)a.vhz[i], a.c[i]};
+    if (V || VISC)
+      q2[t] = V4<T>{V ? (T)a.vx[i] : T(0), V ? (T)a.vy[i] : T(0),
+                    V ? (T)a.vz[i] : T(0), VISC ? a.alpha[i] : T(0)};
     const T rho = a.rho[i];
-    qrho[t] = rho;
-    qprho2[t] = a.P[i] / (rho * rho);
-    qc[t] = a.c[i];
-    if (VISC) qal[t] = a.alpha[i];
+    q3[t] = V2<T>{rho, a.P[i] / (rho * rho)};
   }
   KSum<T> tot[NS];  // thread t: particle t's totals
   T vs = 0, dv = 0;
@@ -704,22 +691,14 @@ __device__ inline void force_group(const ForceArgs<T, MODE> &a, int64_t g) {
     for (int q = 0; q < PER; ++q) {
       const int j = t + q * NT;
       if (j >= nch) continue;
-      sx[j] = (P)(rx[q] - ox); sy[j] = (P)(ry[q] - oy);
-      sz[j] = (P)(rz[q] - oz);
-      svhx[j] = (T)rvhx[q]; svhy[j] = (T)rvhy[q]; svhz[j] = (T)rvhz[q];
-      if (V) {
-        svx[j] = (T)rvx[q]; svy[j] = (T)rvy[q]; svz[j] = (T)rvz[q];
-      }
-      if (VS) {
-        sco[j] = rco[q];
-        sid[j] = rid[q];
-      }
-      sh[j] = (T)rh[q];
-      sm[j] = (T)rm[q];
+      s0[j] = V4<T>{(T)(rx[q] - ox), (T)(ry[q] - oy), (T)(rz[q] - oz),
+                    (T)rh[q]};
+      s1[j] = V4<T>{(T)rvhx[q], (T)rvhy[q], (T)rvhz[q], (T)rm[q]};
+      if (V)
+        s2[j] = V4<T>{(T)rvx[q], (T)rvy[q], (T)rvz[q], VS ? rco[q] : T(0)};
       const T rb = rrho[q];
-      srho[j] = rb;
-      sprho2[j] = rP[q] / (rb * rb);
-      sc[j] = rc[q];
+      s3[j] = V4<T>{rb, rP[q] / (rb * rb), rc[q],
+                    VS ? rel_index<T, NT>(rid[q], c.gs) : T(0)};
       if (VISC) sal[j] = ral[q];
     }
 #pragma unroll
@@ -733,60 +712,63 @@ __device__ inline void force_group(const ForceArgs<T, MODE> &a, int64_t g) {
       if (c0 + 2 * CH < c.cc) load_idx(c0 + 2 * CH);
     }
     const int np = schedule(S, smask, nw, c.gc);
-    P px = 0, py = 0, pz = 0;
-    T pvhx = 0, pvhy = 0, pvhz = 0, pvx = 0, pvy = 0, pvz = 0;
-    T ph = 1, prho = 1, pprho2 = 0, pc = 0, rvs = 0, rdv = 0, pal = 0;
-    int32_t ia = 0;
+    V4<T> p{0, 0, 0, 1}, pvh{0, 0, 0, 0}, pv{0, 0, 0, 0};
+    V2<T> pr{1, 0};
+    T rvs = 0, rdv = 0, ia = 0;
     KSum<T> s[NS];
     walk_run<CH>(
         S, smask, c.gc, np,
         [&](int k) {
-          px = qx[k]; py = qy[k]; pz = qz[k];
-          pvhx = qvhx[k]; pvhy = qvhy[k]; pvhz = qvhz[k];
-          if (V) {
-            pvx = qvx[k]; pvy = qvy[k]; pvz = qvz[k];
-          }
-          ph = qh[k]; prho = qrho[k]; pprho2 = qprho2[k]; pc = qc[k];
-          if (VISC) pal = qal[k];
-          ia = (int32_t)(c.gs + k);
+          p = q0[k];
+          pvh = q1[k];
+          if (V || VISC) pv = q2[k];
+          pr = q3[k];
+          ia = (T)k;
         },
         [&](int j, bool valid) {
           // coincident pairs (m_b := 0, default_physics.h:378) and pairs
           // that are not valid add 0: with ir = 0, F = 0 and every term
           // below is 0
-          const P ddx = px - sx[j], ddy = py - sy[j], ddz = pz - sz[j];
-          const bool same =
-              !valid || (ddx == P(0) && ddy == P(0) && ddz == P(0));
-          const T dx = (T)ddx, dy = (T)ddy, dz = (T)ddz;
+          const V4<T> b0 = s0[j], b1 = s1[j], b3 = s3[j];
+          V4<T> b2{0, 0, 0, 0};
+          if (V) b2 = s2[j];
+          const T m = b1.d, cb = b3.c;
+          const T dx = p.a - b0.a, dy = p.b - b0.b, dz = p.c - b0.c;
+          const bool same = !valid || (dx == T(0) && dy == T(0) && dz == T(0));
           const T r2 = dx * dx + dy * dy + dz * dz;
           const T ir = same ? T(0) : rsq(r2);
           const T r = r2 * ir;
-          const T hab = T(0.5) * (ph + sh[j]);
+          const T hab = T(0.5) * (p.d + b0.d);
           const T ih = rcp(hab);
-          const T F = kernel_F<T>(a.ph.kernel, r, ir, ih);
+          const T F = kernel_F<T>(KERN, r, ir, ih);
           if (VS) {
             // default_physics.h:237-265 (see vsig_group)
-            const T vdr = (pvx - svx[j]) * dx + (pvy - svy[j]) * dy +
-                          (pvz - svz[j]) * dz;
+            const T vdr = (pv.a - b2.a) * dx + (pv.b - b2.b) * dy +
+                          (pv.c - b2.c) * dz;
             const T vdn = vdr * ir;
-            const T cb = sid[j] >= ia ? sc[j] : sco[j];
-            const T cmax = pc < cb ? cb : pc;
+            const T cn = b3.d >= ia ? cb : b2.d;
+            const T cmax = pvh.d < cn ? cn : pvh.d;
             const T v = same ? T(0) : cmax - (vdn < T(0) ? vdn : T(0));
             rvs = rvs < v ? v : rvs;
-            if (VS == 2) rdv += sm[j] * vdr * F;
+            if (VS == 2) rdv += m * vdr * F;
           }
-          const T vhdr = (pvhx - svhx[j]) * dx + (pvhy - svhy[j]) * dy +
-                         (pvhz - svhz[j]) * dz;
+          const T vhdr = (pvh.a - b1.a) * dx + (pvh.b - b1.b) * dy +
+                         (pvh.c - b1.c) * dz;
           T mu = T(0);
-          if (vhdr < T(0)) mu = hab * vhdr * rcp(r2 + eps * hab * hab);
-          const T rhoab = T(0.5) * (prho + srho[j]);
-          const T cab = T(0.5) * (pc + sc[j]);
+          if (sizeof(T) == 4) {
+            const T mn = hab * vhdr * rcp(r2 + eps * hab * hab);
+            mu = vhdr < T(0) ? mn : T(0);
+          } else if (vhdr < T(0)) {
+            mu = hab * vhdr * rcp(r2 + eps * hab * hab);
+          }
+          const T rhoab = T(0.5) * (pr.a + b3.a);
+          const T cab = T(0.5) * (pvh.d + cb);
           const T Pi =
-              VISC ? -(T(0.5) * (pal + sal[j])) * (cab - T(2) * mu) * mu *
+              VISC ? -(T(0.5) * (pv.d + sal[j])) * (cab - T(2) * mu) * mu *
                          rcp(rhoab)
                    : (-alpha * cab + beta * mu) * mu * rcp(rhoab);
           if (!DUDT) {
-            const T f = -sm[j] * (pprho2 + sprho2[j] + Pi) * F;
+            const T f = -m * (pr.b + b3.b + Pi) * F;
             s[0].add(f * dx);
             s[1].add(f * dy);
             s[NS - 1].add(f * dz);
@@ -794,14 +776,13 @@ __device__ inline void force_group(const ForceArgs<T, MODE> &a, int64_t g) {
             // m_b (P_a/rho_a^2 v_b.DW + P_b/rho_b^2 v_a.DW
             //      + Pi/2 (v_a + v_b).DW), summed and negated below
             const T wx = F * dx, wy = F * dy, wz = F * dz;
-            const T va = pvx * wx + pvy * wy + pvz * wz;
-            const T vb = svx[j] * wx + svy[j] * wy + svz[j] * wz;
-            s[0].add(sm[j] *
-                     (pprho2 * vb + va * sprho2[j] + T(0.5) * Pi * (vb + va)));
+            const T va = pv.a * wx + pv.b * wy + pv.c * wz;
+            const T vb = b2.a * wx + b2.b * wy + b2.c * wz;
+            s[0].add(m * (pr.b * vb + va * b3.b + T(0.5) * Pi * (vb + va)));
           } else {
-            const T vdw = ((pvx - svx[j]) * dx + (pvy - svy[j]) * dy +
-                           (pvz - svz[j]) * dz) * F;
-            const T mv = sm[j] * vdw;
+            const T vdw = ((pv.a - b2.a) * dx + (pv.b - b2.b) * dy +
+                           (pv.c - b2.c) * dz) * F;
+            const T mv = m * vdw;
             s[0].add(mv);
             s[1].add(mv * Pi);
           }
@@ -819,18 +800,17 @@ __device__ inline void force_group(const ForceArgs<T, MODE> &a, int64_t g) {
         });
     __syncthreads();
     if (t < c.gc && S.off[t + 1] > S.off[t]) {
+      T v[NV];
+      row_results<VS ? 1u << NS : 0u>(S, R, t, np, v);
 #pragma unroll
-      for (int n = 0; n < NS; ++n) tot[n].add(row_total<false>(S, R, n, t, np));
-      if (VS) {
-        const T u = row_total<true>(S, R, NS, t, np);
-        vs = vs < u ? u : vs;
-      }
-      if (VS == 2) dv += row_total<false>(S, R, NV - 1, t, np);
+      for (int n = 0; n < NS; ++n) tot[n].add(v[n]);
+      if (VS) vs = vs < v[NS % NV] ? v[NS % NV] : vs;
+      if (VS == 2) dv += v[NV - 1];
     }
   }
   if (t >= c.gc) return;
   const int64_t i = c.gs + t;
-  const T prho = qrho[t];
+  const T prho = q3[t].a;
   if (VS) a.vsig[i] = vs;
   if (VS == 2) a.divv[i] = -dv / prho;
   if (!DUDT) {
@@ -839,7 +819,7 @@ __device__ inline void force_group(const ForceArgs<T, MODE> &a, int64_t g) {
     a.az[i] = tot[NS - 1].s - tot[NS - 1].c;
     a.gx[i] = T(0); a.gy[i] = T(0); a.gz[i] = T(0); a.phi[i] = T(0);
   } else if (!DEDT) {
-    const T du = qprho2[t] * (tot[0].s - tot[0].c) +
+    const T du = q3[t].b * (tot[0].s - tot[0].c) +
                  T(0.5) * (tot[1].s - tot[1].c);
     a.dudt[i] = du;
     // recompute_pressure_soundspeed (default_physics.h:154-161)
@@ -855,38 +835,49 @@ __device__ inline void force_group(const ForceArgs<T, MODE> &a, int64_t g) {
 }
 
 // One workgroup per group (grid = number of groups).
-template <class T, int CH, int NT, bool CULL = false>
+template <class T, int CH, int NT, int KERN, bool CULL = false>
 __global__ __launch_bounds__(NT) void k_density(DensArgs<T> a) {
-  density_group<T, CH, NT, CULL>(a, xcd_item(blockIdx.x, gridDim.x));
+  density_group<T, CH, NT, KERN, CULL>(a, xcd_item(blockIdx.x, gridDim.x));
 }
-template <class T, bool DIV, int CH, int NT>
+template <class T, bool DIV, int CH, int NT, int KERN>
 __global__ __launch_bounds__(NT) void k_vsig(VsigArgs<T> a) {
-  vsig_group<T, DIV, CH, NT>(a, xcd_item(blockIdx.x, gridDim.x));
+  vsig_group<T, DIV, CH, NT, KERN>(a, xcd_item(blockIdx.x, gridDim.x));
 }
-template <class T, int MODE, int CH, int NT, int VS = 0, int VISC = 0>
+template <class T, int MODE, int CH, int NT, int KERN, int VS = 0,
+          int VISC = 0>
 __global__ __launch_bounds__(NT) void k_force(ForceArgs<T, MODE> a) {
-  force_group<T, MODE, CH, NT, VS, VISC>(a, xcd_item(blockIdx.x, gridDim.x));
+  force_group<T, MODE, CH, NT, KERN, VS, VISC>(a, xcd_item(blockIdx.x, gridDim.x));
 }
 
-// Calls f(CH, NT) (as std::integral_constant values) for the context's
-// chunk and workgroup width: one wavefront for tiles of at most 64 rows,
-// two otherwise.
+// Calls f(CH, NT, KERN) (as std::integral_constant values) for the
+// context's chunk, workgroup width (one wavefront for tiles of at most 64
+// rows, two otherwise) and kernel function (a branch on it inside the pair
+// loop kept the pairs of an iteration from overlapping).
 template <int V> using IC = std::integral_constant<int, V>;
 // (by the width the tiles were built with: a tile width changed since
 // applies from the next update_iteration)
 inline bool narrow(const Ctx *c) { return c->tiles_w <= 64; }
 template <class F> void dispatch(const Ctx *c, F &&f) {
   const bool nr = narrow(c);
-  switch (c->chunk) {
-    case 64:
-      if (nr) f(IC<64>{}, IC<64>{}); else f(IC<64>{}, IC<128>{});
-      break;
-    case 256:
-      if (nr) f(IC<256>{}, IC<64>{}); else f(IC<256>{}, IC<128>{});
-      break;
-    default:
-      if (nr) f(IC<128>{}, IC<64>{}); else f(IC<128>{}, IC<128>{});
-  }
+  auto go = [&](auto kern) {
+    switch (c->chunk) {
+      case 64:
+        if (nr) f(IC<64>{}, IC<64>{}, kern);
+        else f(IC<64>{}, IC<128>{}, kern);
+        break;
+      case 256:
+        if (nr) f(IC<256>{}, IC<64>{}, kern);
+        else f(IC<256>{}, IC<128>{}, kern);
+        break;
+      default:
+        if (nr) f(IC<128>{}, IC<64>{}, kern);
+        else f(IC<128>{}, IC<128>{}, kern);
+    }
+  };
+  if (c->p.kernel == FSPH_KERNEL_CUBIC_SPLINE)
+    go(IC<FSPH_KERNEL_CUBIC_SPLINE>{});
+  else
+    go(IC<FSPH_KERNEL_WENDLAND_C6>{});
 }
 
 Phys phys_of(const Ctx *c) {
@@ -915,8 +906,9 @@ Tiles tiles_of(const Ctx *c) {
 }
 
 template <class T, bool DIV> void vsig_launch(Ctx *c, const VsigArgs<T> &v) {
-  dispatch(c, [&](auto ch, auto nt) {
-    k_vsig<T, DIV, decltype(ch)::value, decltype(nt)::value>
+  dispatch(c, [&](auto ch, auto nt, auto kern) {
+    k_vsig<T, DIV, decltype(ch)::value, decltype(nt)::value,
+           decltype(kern)::value>
         <<<(unsigned)c->nt, (unsigned)decltype(nt)::value, 0, c->stream>>>(v);
   });
 }
@@ -1012,13 +1004,14 @@ template <class T> int density_impl(Ctx *c, bool with_vsig) {
   const bool cull = c->p.viscosity == FSPH_VISC_CULLEN;
   {
     PhaseTimer tm(c, FSPH_T_DENSITY);
-    dispatch(c, [&](auto ch, auto nt) {
+    dispatch(c, [&](auto ch, auto nt, auto kern) {
       constexpr int CH = decltype(ch)::value, NT = decltype(nt)::value;
+      constexpr int K = decltype(kern)::value;
       if (cull)
-        k_density<T, CH, NT, true>
+        k_density<T, CH, NT, K, true>
             <<<(unsigned)c->nt, (unsigned)NT, 0, c->stream>>>(a);
       else
-        k_density<T, CH, NT>
+        k_density<T, CH, NT, K>
             <<<(unsigned)c->nt, (unsigned)NT, 0, c->stream>>>(a);
     });
   }
@@ -1041,12 +1034,14 @@ template <class T, int MODE, int VS = 0> int force_impl(Ctx *c) {
     PhaseTimer tm(c, MODE != kAccel ? FSPH_T_DUDT : FSPH_T_ACCEL);
     const unsigned ng = (unsigned)c->nt;
     const bool cull = c->p.viscosity == FSPH_VISC_CULLEN;
-    dispatch(c, [&](auto ch, auto nt) {
+    dispatch(c, [&](auto ch, auto nt, auto kern) {
       constexpr int CH = decltype(ch)::value, NT = decltype(nt)::value;
+      constexpr int K = decltype(kern)::value;
       if (cull)
-        k_force<T, MODE, CH, NT, VS, 1><<<ng, (unsigned)NT, 0, c->stream>>>(a);
+        k_force<T, MODE, CH, NT, K, VS, 1>
+            <<<ng, (unsigned)NT, 0, c->stream>>>(a);
       else
-        k_force<T, MODE, CH, NT, VS><<<ng, (unsigned)NT, 0, c->stream>>>(a);
+        k_force<T, MODE, CH, NT, K, VS><<<ng, (unsigned)NT, 0, c->stream>>>(a);
     });
   }
   FSPH_HIP(c, hipGetLastError());
@@ -1076,23 +1071,24 @@ template <class T> void sph_graph_args_t(Ctx *c, char *slots) {
   std::swap(c->f[PF_C], c->g[PF_C]);
 }
 
-template <class T, int CH, int NT>
+template <class T, int CH, int NT, int K>
 const void *sph_graph_func_t(int pass, bool tk) {
   switch (pass) {
     case kSlotDens:
-      return reinterpret_cast<const void *>(k_density<T, CH, NT>);
+      return reinterpret_cast<const void *>(k_density<T, CH, NT, K>);
     case kSlotAcc:
-      return reinterpret_cast<const void *>(k_force<T, kAccel, CH, NT, 1>);
+      return reinterpret_cast<const void *>(k_force<T, kAccel, CH, NT, K, 1>);
     default:
-      return tk ? reinterpret_cast<const void *>(k_force<T, kDedt, CH, NT>)
-                : reinterpret_cast<const void *>(k_force<T, kDudt, CH, NT>);
+      return tk ? reinterpret_cast<const void *>(k_force<T, kDedt, CH, NT, K>)
+                : reinterpret_cast<const void *>(k_force<T, kDudt, CH, NT, K>);
   }
 }
 
 template <class T> const void *sph_graph_func_c(const Ctx *c, int pass) {
   const void *f = nullptr;
-  dispatch(c, [&](auto ch, auto nt) {
-    f = sph_graph_func_t<T, decltype(ch)::value, decltype(nt)::value>(
+  dispatch(c, [&](auto ch, auto nt, auto kern) {
+    f = sph_graph_func_t<T, decltype(ch)::value, decltype(nt)::value,
+                         decltype(kern)::value>(
         pass, c->p.thermokinetic != 0);
   });
   return f;
@@ -1170,8 +1166,9 @@ template <class T> int alpha_impl(Ctx *c) {
   a.alpha_max = c->p.visc_alpha_max;
   a.delta = c->p.visc_delta;
   a.l = c->p.visc_l;
-  dispatch(c, [&](auto ch, auto nt) {
-    k_alpha<T, decltype(ch)::value, decltype(nt)::value>
+  dispatch(c, [&](auto ch, auto nt, auto kern) {
+    k_alpha<T, decltype(ch)::value, decltype(nt)::value,
+            decltype(kern)::value>
         <<<(unsigned)c->nt, (unsigned)decltype(nt)::value, 0, c->stream>>>(a);
   });
   return hip_check(c, hipGetLastError(), "k_alpha");

@@ -393,7 +393,8 @@ __global__ __launch_bounds__(kT) void k_group_flags(
 // g + (split groups before g) holds its rows, or the first half of a split
 // group's, whose second half makes tile t0 + 1 (halves, not tw rows and the
 // rest: a tile's cost grows with its rows, and the longest of one wavefront
-// each bound the last part of a launch; @SPLIT@).  The candidates of a group's
+// each bound the last part of a launch: acceleration on the 1.5M
+// collapse 1,042 -> 955 us, Newton-h phase 5.23 -> 4.85 ms).  The candidates of a group's
 // only tile are in the group's slot g; a split group (s-th of them) has two
 // slots of its own, ng + 2 s and ng + 2 s + 1.
 __global__ __launch_bounds__(kT) void k_group_write(

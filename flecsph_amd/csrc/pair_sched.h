@@ -141,8 +141,10 @@ template <int CH> struct RowBits {
 // them (the ones past the row's or the run's end come with valid false and
 // must add nothing): some thread of the wavefront changes rows in nearly
 // every iteration, so that code is paid once for kPairs pairs, and their
-// LDS reads and chains overlap.  The row's bits stay in registers.
-// @MEAS@
+// LDS reads and chains overlap.  The row's bits stay in registers.  The
+// acceleration pass (FP32, chunk 128) went from 341 to 273 us on Sedov 64^3
+// and 726 to 596 us on the 1M star; three pairs measured 318 and 703 us, four
+// 332 and 737 (more of them past a row's end, more registers).
 constexpr int kPairs = 2;
 template <int CH, int NT, class Load, class Pair, class Flush>
 __device__ inline void walk_run(const Sched<NT> &S, const uint32_t *smask,
@@ -189,20 +191,26 @@ __device__ inline void put(Parts<T, NV, NT> &R, int i, int k, T v) {
   R.v[i][(int)threadIdx.x + k] = v;
 }
 
-// Row k's result of this chunk, component i (after the walk; the row must
-// hold pairs); MAX combines with max instead of +.
-template <bool MAX, class T, int NV, int NT>
-__device__ inline T row_total(const Sched<NT> &S, const Parts<T, NV, NT> &R,
-                              int i, int k, int total) {
-  const int q = (total + NT - 1) / NT;
-  const int a = S.off[k], b = S.off[k + 1];
-  const int la = a / q, lb = (b - 1) / q;
-  T v = R.v[i][k + la];
-  for (int l = la + 1; l <= lb; ++l) {
-    const T u = R.v[i][k + l];
-    v = MAX ? (v < u ? u : v) : v + u;
-  }
-  return v;
+// Row k's results of this chunk into v (after the walk; the row must hold
+// pairs): its pieces in run order, added up or, for the components whose bit
+// is set in MAXED, the largest.  The runs that hold the row's first and last
+// pair are quotients by the run length: exact through FP32, as the numbers
+// stay below 2^15 and (pair + 0.5) / q is at least 0.5 / q from an integer.
+template <unsigned MAXED, class T, int NV, int NT>
+__device__ inline void row_results(const Sched<NT> &S,
+                                   const Parts<T, NV, NT> &R, int k, int total,
+                                   T (&v)[NV]) {
+  const float rq = 1.0f / (float)((total + NT - 1) / NT);
+  const int la = (int)(((float)S.off[k] + 0.5f) * rq);
+  const int lb = (int)(((float)S.off[k + 1] - 0.5f) * rq);
+#pragma unroll
+  for (int i = 0; i < NV; ++i) v[i] = R.v[i][k + la];
+  for (int l = la + 1; l <= lb; ++l)
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const T u = R.v[i][k + l];
+      v[i] = MAXED >> i & 1u ? (v[i] < u ? u : v[i]) : v[i] + u;
+    }
 }
 
 }  // namespace sched
