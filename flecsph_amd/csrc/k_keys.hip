@@ -1,5 +1,7 @@
 // k_keys.hip -- periodic WALL copies, range of x +- h, Morton keys, LSD
 // radix sort of (key, index), and the particle permutation.
+#include <type_traits>
+
 #include "fsph_internal.h"
 
 namespace fsph {
@@ -322,13 +324,22 @@ __global__ __launch_bounds__(kT) void k_keys(
 }
 
 // ---------------------------------------------------------------------------
-// LSD radix sort, 8 bits per pass, 2048 keys per tile (256 threads x 8).
-// Per pass: tile digit counts, a scan of every digit's row of tile counts
-// (one workgroup per digit), and a stable scatter that adds the digits'
-// bases (a scan of the 256 row totals) itself.
+// LSD radix sort, 8 bits per pass, 2048 keys per tile (256 threads x 8), in
+// one of two forms by the number of keys:
+//  * up to kSortOne: all passes in one workgroup, keys in LDS (one launch);
+//  * more: per pass, tile digit counts, a scan of every digit's row of tile
+//    counts (one workgroup per digit), and a stable scatter that adds the
+//    digits' bases (a scan of the 256 row totals) itself.
+// A launch takes 4-5 us here whatever it does: with three per pass 2,000
+// keys took 116 us and 10,007 132, in one workgroup 33 and 91 (its 12 keys
+// per thread are what its LDS holds).  At 38,880 and 91,125 keys the three
+// launches take 141 and 145 us; two per pass, the scatter summing the counts
+// of the tiles before it, took 145 and 195, and one per pass, the scatter
+// counting the next pass's digits with atomics, 136 and 184.
 // ---------------------------------------------------------------------------
 constexpr int kRsItems = 8;
 constexpr int kRsTile = kT * kRsItems;
+constexpr int64_t kSortOne = 12288;
 
 // Digit of a pass: 8 key bits at `shift`, or (inst given) the instance of
 // the particle the entry points to.
@@ -523,6 +534,94 @@ __global__ __launch_bounds__(kT) void k_radix_scatter(
   }
 }
 
+// All passes for up to 1024 ITEMS keys in one workgroup: the ranking of
+// k_radix_scatter over 16 wavefronts, the entries reordered in LDS.
+template <int ITEMS>
+__global__ __launch_bounds__(1024) void k_sort_one(
+    const uint64_t *kin, uint64_t *kout, uint32_t *vout, int n, int passes,
+    const int32_t *__restrict__ inst) {
+  constexpr int kWv = 16;
+  __shared__ uint64_t sk[1024 * ITEMS];
+  __shared__ uint16_t sv[1024 * ITEMS];
+  __shared__ int32_t wcnt[kWv][256];
+  __shared__ int32_t wsum[4];
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
+  const int base = w * 64 * ITEMS + lane;
+  uint64_t k[ITEMS];
+  uint32_t v[ITEMS];
+#pragma unroll
+  for (int r = 0; r < ITEMS; ++r) {
+    const int i = base + r * 64;
+    k[r] = i < n ? kin[i] : 0ull;
+    v[r] = (uint32_t)i;
+  }
+  for (int pass = 0; pass < passes; ++pass) {
+    const int32_t *pi = pass == 8 ? inst : nullptr;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) wcnt[w][lane * 4 + j] = 0;
+    int d[ITEMS], rk[ITEMS];
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+      const bool valid = base + r * 64 < n;
+      const uint32_t dg = valid ? rs_digit(k[r], v[r], pass * 8, pi) : 0u;
+      const uint64_t peers = match_digit(dg, valid);
+      const int rank = __popcll(peers & lt);
+      const int prev = wcnt[w][dg];
+      if (valid && rank == 0) wcnt[w][dg] = prev + __popcll(peers);
+      d[r] = (int)dg;
+      rk[r] = prev + rank;
+    }
+    __syncthreads();
+    // thread t < 256: digit t's total, its start, then the wavefronts' bases
+    int tot = 0, inc = 0;
+    if (t < 256) {
+#pragma unroll
+      for (int q = 0; q < kWv; ++q) tot += wcnt[q][t];
+      inc = tot;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int u = __shfl_up(inc, o, 64);
+        if (lane >= o) inc += u;
+      }
+      if (lane == 63) wsum[w] = inc;
+    }
+    __syncthreads();
+    if (t < 256) {
+      int ex = inc - tot;
+      for (int q = 0; q < w; ++q) ex += wsum[q];
+#pragma unroll
+      for (int q = 0; q < kWv; ++q) {
+        const int c = wcnt[q][t];
+        wcnt[q][t] = ex;
+        ex += c;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r)
+      if (base + r * 64 < n) {
+        const int pos = wcnt[w][d[r]] + rk[r];
+        sk[pos] = k[r];
+        sv[pos] = (uint16_t)v[r];
+      }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r)
+      if (base + r * 64 < n) {
+        k[r] = sk[base + r * 64];
+        v[r] = sv[base + r * 64];
+      }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int r = 0; r < ITEMS; ++r)
+    if (base + r * 64 < n) {
+      kout[base + r * 64] = k[r];
+      vout[base + r * 64] = v[r];
+    }
+}
+
 __global__ __launch_bounds__(kT) void k_check_dup(
     const uint64_t *__restrict__ key, const uint32_t *__restrict__ val,
     const int32_t *__restrict__ inst, int64_t n, int *flags) {
@@ -694,31 +793,49 @@ int stage_sort(Ctx *c) {
   const int64_t nb = (n + kRsTile - 1) / kRsTile;
   FSPH_TRY(ensure(c, c->key2, (size_t)c->pcap * 8));
   FSPH_TRY(ensure(c, c->val2, (size_t)c->pcap * 4));
-  FSPH_TRY(ensure(c, c->hist, (size_t)256 * nb * sizeof(int32_t) +
-                                  (size_t)(256 * nb + 264) * sizeof(int64_t)));
-  int32_t *hist = c->hist.as<int32_t>();
-  int64_t *hoff = reinterpret_cast<int64_t *>(
-      c->hist.as<char>() + (((size_t)256 * nb * sizeof(int32_t) + 7) & ~(size_t)7));
-  int64_t *rowtot = hoff + 256 * nb;
   uint64_t *k0 = c->key.as<uint64_t>(), *k1 = c->key2.as<uint64_t>();
   uint32_t *v0 = c->val.as<uint32_t>(), *v1 = c->val2.as<uint32_t>();
   // 8 passes over the key bytes; in batched mode a ninth, stable pass on
   // the instance gives (instance, key, id) order.
   const int32_t *inst = c->batch.n_inst ? c->f[PF_INST].as<int32_t>() : nullptr;
   const int passes = inst ? 9 : 8;
-  for (int pass = 0; pass < passes; ++pass) {
-    const int shift = pass * 8;
-    const int32_t *pi = pass == 8 ? inst : nullptr;
-    k_radix_hist<<<(unsigned)nb, kT, 0, c->stream>>>(k0, v0, n, shift, pi,
-                                                     hist, nb);
-    k_radix_rowscan<<<256, kT, 0, c->stream>>>(hist, hoff, rowtot, nb);
-    k_radix_scatter<<<(unsigned)nb, kT, 0, c->stream>>>(
-        k0, v0, k1, v1, n, shift, pi, hoff, rowtot, nb);
+  if (n <= kSortOne) {
+    auto go = [&](auto items) {
+      k_sort_one<decltype(items)::value><<<1, 1024, 0, c->stream>>>(
+          k0, k0, v0, (int)n, passes, inst);
+    };
+    if (n <= 2048)
+      go(std::integral_constant<int, 2>{});
+    else if (n <= 4096)
+      go(std::integral_constant<int, 4>{});
+    else if (n <= 8192)
+      go(std::integral_constant<int, 8>{});
+    else
+      go(std::integral_constant<int, 12>{});
     FSPH_HIP(c, hipGetLastError());
-    std::swap(k0, k1);
-    std::swap(v0, v1);
+  } else {
+    FSPH_TRY(ensure(c, c->hist,
+                    (size_t)256 * nb * sizeof(int32_t) +
+                        (size_t)(256 * nb + 264) * sizeof(int64_t)));
+    int32_t *hist = c->hist.as<int32_t>();
+    int64_t *hoff = reinterpret_cast<int64_t *>(
+        c->hist.as<char>() +
+        (((size_t)256 * nb * sizeof(int32_t) + 7) & ~(size_t)7));
+    int64_t *rowtot = hoff + 256 * nb;
+    for (int pass = 0; pass < passes; ++pass) {
+      const int shift = pass * 8;
+      const int32_t *pi = pass == 8 ? inst : nullptr;
+      k_radix_hist<<<(unsigned)nb, kT, 0, c->stream>>>(k0, v0, n, shift, pi,
+                                                       hist, nb);
+      k_radix_rowscan<<<256, kT, 0, c->stream>>>(hist, hoff, rowtot, nb);
+      k_radix_scatter<<<(unsigned)nb, kT, 0, c->stream>>>(
+          k0, v0, k1, v1, n, shift, pi, hoff, rowtot, nb);
+      FSPH_HIP(c, hipGetLastError());
+      std::swap(k0, k1);
+      std::swap(v0, v1);
+    }
   }
-  if (passes & 1) {
+  if (k0 != c->key.as<uint64_t>()) {
     // keep the sorted keys in c->key for the tree
     std::swap(c->key, c->key2);
     std::swap(c->val, c->val2);

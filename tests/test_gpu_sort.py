@@ -1,0 +1,51 @@
+"""The two forms of the radix sort (one workgroup, three launches per pass)
+at the edges of their ranges and of their tiles:
+keys and ids in the oracle's order, and a batch in its instances' own."""
+import numpy as np
+import pytest
+
+from flecsph_amd import BatchSystem, BodySystem, _abi, generators
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n", [2, 3, 63, 65, 1025, 2048, 2049, 4096, 4097,
+                               8192, 8193, 12288, 12289, 63489])
+def test_sorted_keys_equal_the_oracles(oracle_mod, n):
+    parts, prm = generators.random_box(n, seed=n)
+    if 3 < n < 20000:  # half of them in a corner: equal high digits
+        for k in ("x", "y", "z", "h"):
+            parts[k][: n // 2] *= 0.03
+    p = _abi.default_params(**prm)
+    g, o = BodySystem(p), oracle_mod.OracleSystem(p, threads=8)
+    for s in (g, o):
+        s.upload(parts)
+        s.update_iteration()
+    for f in ("key", "id", "x", "h"):
+        assert np.array_equal(g.get(f), o.get(f)), f
+    o.close()
+    g.close()
+
+
+@pytest.mark.parametrize("sizes", [(2, 3, 40), (700, 1349), (3000, 5192),
+                                   (3000, 9286, 2), (3000, 9287, 2),
+                                   (40000, 91072, 2)])
+def test_sorted_keys_of_a_batch(sizes):
+    sets = [generators.random_box(n, seed=n + i) for i, n in enumerate(sizes)]
+    prm = sets[0][1]
+    prm["eta"] = 1.2
+    b = BatchSystem(_abi.default_params(**prm), len(sizes))
+    b.upload([parts for parts, _ in sets])
+    b.update_iteration()
+    key, ids = b.get("key"), b.get("id")
+    o = 0
+    for parts, _ in sets:
+        n = len(parts["x"])
+        s = BodySystem(_abi.default_params(**prm))
+        s.upload(parts)
+        s.update_iteration()
+        assert np.array_equal(key[o:o + n], s.get("key"))
+        assert np.array_equal(ids[o:o + n], s.get("id"))
+        s.close()
+        o += n
+    b.close()
