@@ -89,10 +89,7 @@ int ensure_particles(Ctx *c, int64_t cap, bool keep) {
   return 0;
 }
 
-// Copies the first `words` words of the device mailbox to the host and waits.
-int read_mail(Ctx *c, int words) {
-  FSPH_HIP(c, hipMemcpyAsync(c->mail_h, c->mail.p, (size_t)words * 8,
-                             hipMemcpyDeviceToHost, c->stream));
+int read_mail(Ctx *c) {
   FSPH_HIP(c, hipStreamSynchronize(c->stream));
   return 0;
 }
@@ -102,8 +99,8 @@ __global__ void k_total_mail(const int64_t *__restrict__ total,
                              const int *__restrict__ scan_word,
                              int64_t *__restrict__ mail) {
   if (threadIdx.x == 0) {
-    mail[0] = *total;
-    mail[1] = *scan_word;
+    mail_put(mail + 0, *total);
+    mail_put(mail + 1, *scan_word);
   }
 }
 }  // namespace
@@ -111,9 +108,9 @@ __global__ void k_total_mail(const int64_t *__restrict__ total,
 int read_scan_total(Ctx *c, const int64_t *dev_total, int64_t *out) {
   k_total_mail<<<1, 64, 0, c->stream>>>(dev_total,
                                         c->flags.as<int>() + kScanWord,
-                                        c->mail.as<int64_t>());
+                                        c->mail_d);
   FSPH_HIP(c, hipGetLastError());
-  FSPH_TRY(read_mail(c, 2));
+  FSPH_TRY(read_mail(c));
   if (c->mail_h[1] & kFlagScanStall)
     return fail(c, FSPH_E_HIP, "scan: a tile's look-back did not complete");
   *out = c->mail_h[0];
@@ -131,7 +128,7 @@ namespace {
 
 int do_update_iteration(Ctx *c) {
   c->have_tree = false;
-  FSPH_HIP(c, hipMemsetAsync(c->flags.p, 0, 16 * sizeof(int), c->stream));
+  FSPH_TRY(stage_begin(c));
   {
     PhaseTimer t(c, FSPH_T_BOUNDARY);
     FSPH_TRY(stage_boundary(c));
@@ -225,6 +222,9 @@ int do_update_h(Ctx *c) {
 
 int do_step(Ctx *c) {
   c->ev_used = 0;
+  uint32_t tail_kick = 0;  // energy kick left to the fused end of the step
+  const bool fused = !c->batch.n_inst && c->p.adaptive_dt;
+  const bool closed = c->p.h_mode == FSPH_H_CLOSED;
   if (!c->initial_done) {
     // hydro/main_driver.cc:102-173 (iteration 0: no integration)
     FSPH_TRY(do_update_iteration(c));
@@ -270,12 +270,13 @@ int do_step(Ctx *c) {
       // the rest of the step up to the dt minimum as one graph replay
       FSPH_TRY(graph_step_tail(c));
       c->batch.dt_ready = c->p.adaptive_dt != 0;
-      if (c->checks) FSPH_TRY(stage_check_state(c));
+      if (c->checks) FSPH_TRY(stage_check_state(c, false));
       {
         PhaseTimer t(c, FSPH_T_DT);
         FSPH_TRY(do_timestep(c));
       }
-      return do_advance(c);
+      FSPH_TRY(do_advance(c));
+      return stage_step_mail(c);
     }
     FSPH_TRY(stage_density_only(c));
     // main_driver.cc:189-192
@@ -291,19 +292,35 @@ int do_step(Ctx *c) {
     }
     if (c->p.evolve_internal_energy) {
       FSPH_TRY(c->p.thermokinetic ? stage_dedt(c) : stage_dudt(c));
-      PhaseTimer t(c, FSPH_T_INTEGRATE);
-      FSPH_TRY(stage_integrate(c, kick_energy));
+      if (fused && closed) {
+        tail_kick = kick_energy;
+      } else {
+        PhaseTimer t(c, FSPH_T_INTEGRATE);
+        FSPH_TRY(stage_integrate(c, kick_energy));
+      }
     }
+  }
+  if (fused) {
+    // the calls below, each particle's in the same order, in one launch
+    // (a Newton or learned h, which works on tiles, first)
+    c->h_gather_words = 0;
+    c->h_kappa = 0;
+    if (!closed) FSPH_TRY(do_update_h(c));
+    PhaseTimer t(c, FSPH_T_DT);
+    FSPH_TRY(stage_step_tail(c, tail_kick));
+    c->iteration++;
+    return 0;
   }
   FSPH_TRY(do_update_h(c));  // hydro/main_driver.cc:247-256
   // check_nans, check_negativity (hydro/main_driver.cc:263-265); the result
   // is read once the step's work has completed
-  if (c->checks) FSPH_TRY(stage_check_state(c));
+  if (c->checks) FSPH_TRY(stage_check_state(c, false));
   {
     PhaseTimer t(c, FSPH_T_DT);
     FSPH_TRY(do_timestep(c));  // hydro/main_driver.cc:267-273
   }
-  return do_advance(c);
+  FSPH_TRY(do_advance(c));
+  return stage_step_mail(c);
 }
 
 int do_gravity(Ctx *c) { return stage_gravity(c); }
@@ -387,15 +404,22 @@ int fsph_create(const fsph_params *p, int device, fsph_ctx **out) {
     return FSPH_E_HIP;
   }
   if (fsph::ensure(c, c->flags, 64) ||
-      fsph::ensure(c, c->mail, fsph::kMail * sizeof(int64_t)) ||
       hipHostMalloc(reinterpret_cast<void **>(&c->mail_h),
-                    fsph::kMail * sizeof(int64_t), hipHostMallocDefault) !=
-          hipSuccess) {
+                    fsph::kMail * sizeof(int64_t),
+                    hipHostMallocMapped | hipHostMallocCoherent) !=
+          hipSuccess ||
+      hipHostGetDevicePointer(reinterpret_cast<void **>(&c->mail_d),
+                              c->mail_h, 0) != hipSuccess) {
     if (c->flags.p) hipFree(c->flags.p);
-    if (c->mail.p) hipFree(c->mail.p);
+    if (c->mail_h) hipHostFree(c->mail_h);
     hipStreamDestroy(c->stream);
     delete c;
     return FSPH_E_OOM;
+  }
+  std::memset(c->mail_h, 0, fsph::kMail * sizeof(int64_t));
+  if (fsph::stage_begin(c) != FSPH_OK) {
+    fsph_destroy(reinterpret_cast<fsph_ctx *>(c));
+    return FSPH_E_HIP;
   }
   for (int i = 0; i < 2 * Ctx::kEvPool; ++i) hipEventCreate(&c->ev[i]);
   hipEventCreateWithFlags(&c->ev_groups, hipEventDisableTiming);
@@ -410,7 +434,7 @@ void fsph_destroy(fsph_ctx *ctx) {
   hipStreamSynchronize(c->stream);
   fsph::DBuf *all[] = {&c->key, &c->key2, &c->val, &c->val2, &c->perm,
                        &c->hist, &c->scan_tmp, &c->scan_state, &c->red_tmp, &c->flags,
-                       &c->mail, &c->range_d,
+                       &c->lvl, &c->range_d,
                        &c->L, &c->pair_cnt, &c->pair_off, &c->nkey,
                        &c->ndepth, &c->nstart, &c->ncount, &c->nparent,
                        &c->nchild, &c->nbox, &c->ncom, &c->nmass, &c->nrad,
@@ -808,10 +832,6 @@ int fsph_step(fsph_ctx *ctx) {
   CTX_OR_FAIL;
   if (c->n < 2) return fsph::fail(c, FSPH_E_ARG, "no particles uploaded");
   FSPH_TRY(fsph::do_step(c));
-  c->mail_h[fsph::kMailScan] = 0;
-  FSPH_HIP(c, hipMemcpyAsync(c->mail_h + fsph::kMailScan,
-                             c->flags.as<int>() + fsph::kScanWord, 4,
-                             hipMemcpyDeviceToHost, c->stream));
   FSPH_HIP(c, hipStreamSynchronize(c->stream));
   if (c->mail_h[fsph::kMailScan] & fsph::kFlagScanStall)
     return fsph::fail(c, FSPH_E_HIP,
@@ -830,7 +850,8 @@ int fsph_step(fsph_ctx *ctx) {
 int fsph_check_state(fsph_ctx *ctx) {
   CTX_OR_FAIL;
   if (c->n < 2) return fsph::fail(c, FSPH_E_ARG, "no particles uploaded");
-  FSPH_TRY(fsph::stage_check_state(c));
+  FSPH_TRY(fsph::stage_check_state(c, true));
+  FSPH_TRY(fsph::stage_step_mail(c));
   FSPH_HIP(c, hipStreamSynchronize(c->stream));
   return fsph::check_result(c);
 }

@@ -17,7 +17,7 @@
 namespace fsph {
 
 constexpr int kMaxDepth = 21;     // filling_curve.h:44-47 (64-bit keys, 3D)
-constexpr int kMail = 64;         // words of the device/host mailbox
+constexpr int kMail = 64;         // words of the mailbox
 constexpr int32_t kChildEmpty = -1;
 // child codes: >= 0 node index; <= -2 leaf particle p stored as -(p+2)
 __host__ __device__ inline int32_t leaf_code(int64_t p) {
@@ -39,6 +39,21 @@ __host__ __device__ inline int64_t xcd_item(int64_t b, int64_t G) {
   const int64_t x = b % kX, j = b / kX;
   return ((j / kXcdRun) * kX + x) * kXcdRun + j % kXcdRun;
 }
+
+#ifdef __HIPCC__
+// Loads and stores that other workgroups of the same kernel see or wrote
+// (device scope, whichever XCD's L2 they run on).
+__device__ inline double ld_agent(const double *p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline void st_agent(double *p, double v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// A word of the mailbox (host memory).
+__device__ inline void mail_put(int64_t *p, int64_t v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+#endif
 
 // Growable device buffer.
 struct DBuf {
@@ -62,9 +77,13 @@ enum : int {
 // [kScanWord]: kFlagScanStall of any scan since the last update_iteration
 // (sticky: every read-back that depends on a scan checks it).
 constexpr int kCheckWord = 4;
+constexpr int kCheckNone = 0x7f7f7f7f;  // above every index
 constexpr int kScanWord = 6;
 // [kWalkWord]: overflow bits of the FMM sink-major walk
 constexpr int kWalkWord = 8;
+// [kRangeCtr], [kDtCtr], [kMaxCtr]: workgroups done in a reduction whose
+// last one finishes it (each is back at 0 when the kernel ends)
+constexpr int kRangeCtr = 10, kDtCtr = 11, kMaxCtr = 12;
 // mail_h slot that receives the state check's two words, and the one that
 // receives the scan word at the end of a step / with the group count
 constexpr int kMailCheck = kMail - 3;
@@ -124,8 +143,11 @@ struct Ctx {
   int scan_parity = 0;   // half used by the next scan
   DBuf red_tmp;        // reduction partials
   DBuf flags;          // int error flags
-  DBuf mail;           // device mailbox: scalars read back in one copy
-  int64_t *mail_h = nullptr;  // its pinned host copy (kMail words)
+  // mailbox of kMail words in pinned host memory, which kernels write
+  // directly (mail_d is its device address): read after the stream or an
+  // event has been waited for, without a copy
+  int64_t *mail_h = nullptr, *mail_d = nullptr;
+  DBuf lvl;            // tree: nodes per depth, then the level cursors
   // pinned halves that gather the small sets of an upload (on first use)
   char *stage_h = nullptr;
   int stage_half = 0;
@@ -384,9 +406,18 @@ int stage_update_h(Ctx *c);            // k_step.hip
 // poly_K where rho and P were not uploaded (k_step.hip)
 int stage_eos_init(Ctx *c);
 // check_nans + check_negativity (default_physics.h:918-979): enqueues the
-// check and the copy of its result to mail_h[kMailCheck]; check_result
-// (fsph_api.hip) reads it after the stream has been synchronised
-int stage_check_state(Ctx *c);
+// check (reset: its two words still hold an earlier check's result);
+// check_result (fsph_api.hip) reads the result from mail_h[kMailCheck] after
+// stage_step_mail and a synchronisation
+int stage_check_state(Ctx *c, bool reset);
+// the check's words and the scan word into the mailbox
+int stage_step_mail(Ctx *c);
+// clears the flags and the tree's level counts (update_iteration's start)
+int stage_begin(Ctx *c);
+// End of a step of a single simulation with an adaptive time step: energy
+// kick (what), closed-form h update (with h_mode FSPH_H_CLOSED), state
+// check, time-step rule, clock and mailbox in one launch (k_step.hip)
+int stage_step_tail(Ctx *c, uint32_t what);
 int check_result(Ctx *c);
 int stage_reductions(Ctx *c, double out[10]);  // k_step.hip
 // set_total_energy of the thermokinetic formulation (k_step.hip)
@@ -398,7 +429,7 @@ int scratch_setup(int device);
 int stage_reductions_noalloc(Ctx *c, double out[10]);
 // device pointer to 2.5 max h (the periodic halo), no host wait
 int stage_halo(Ctx *c, const double **halo);  // k_step.hip
-int read_mail(Ctx *c, int words);             // fsph_api.hip
+int read_mail(Ctx *c);                        // waits for the stream
 // Reads the int64 *dev_total (a scan's total) to *out, failing with
 // FSPH_E_HIP if a scan has stalled (fsph_api.hip).
 int read_scan_total(Ctx *c, const int64_t *dev_total, int64_t *out);

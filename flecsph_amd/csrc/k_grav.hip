@@ -157,14 +157,9 @@ __global__ __launch_bounds__(kT) void k_p2m(Cells c, int64_t nc,
 
 // M2M for the internal cells among the nodes of one level
 template <class T>
-__global__ __launch_bounds__(kT) void k_m2m(Cells c,
-                                            const int32_t *__restrict__ nodes,
-                                            int64_t cnt,
-                                            const int32_t *__restrict__ nodecell,
-                                            T *__restrict__ Q) {
-  const int64_t t = (int64_t)blockIdx.x * kT + threadIdx.x;
-  if (t >= cnt) return;
-  const int32_t cell = nodecell[nodes[t]];
+__device__ inline void m2m_node(const Cells &c, int32_t node,
+                                const int32_t *__restrict__ nodecell, T *Q) {
+  const int32_t cell = nodecell[node];
   if (cell < 0 || c.bucket[cell]) return;
   double q[6] = {0, 0, 0, 0, 0, 0};
   const double cx = c.com[3 * cell], cy = c.com[3 * cell + 1],
@@ -177,6 +172,35 @@ __global__ __launch_bounds__(kT) void k_m2m(Cells c,
              c.com[3 * ch + 2] - cz);
   }
   for (int k = 0; k < 6; ++k) Q[6 * (int64_t)cell + k] = (T)q[k];
+}
+
+template <class T>
+__global__ __launch_bounds__(kT) void k_m2m(Cells c,
+                                            const int32_t *__restrict__ nodes,
+                                            int64_t cnt,
+                                            const int32_t *__restrict__ nodecell,
+                                            T *Q) {
+  const int64_t t = (int64_t)blockIdx.x * kT + threadIdx.x;
+  if (t < cnt) m2m_node(c, nodes[t], nodecell, Q);
+}
+
+// Levels lo .. hi, deepest first, of at most kChainCells nodes each, in one
+// workgroup: such a level is a launch's latency (7 us) otherwise.  (The
+// stores of a level are seen by the next through the barrier: one CU.)
+constexpr int kChainThreads = 1024;
+constexpr int64_t kChainCells = 1024;
+struct LevelOff {
+  int32_t off[kMaxDepth + 2];
+};
+template <class T>
+__global__ __launch_bounds__(kChainThreads) void k_m2m_chain(
+    Cells c, const int32_t *__restrict__ level, LevelOff L, int lo, int hi,
+    const int32_t *__restrict__ nodecell, T *Q) {
+  for (int d = hi; d >= lo; --d) {
+    const int t = L.off[d] + (int)threadIdx.x;
+    if (t < L.off[d + 1]) m2m_node(c, level[t], nodecell, Q);
+    __syncthreads();
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -353,11 +377,12 @@ __global__ void k_pair_mail(const unsigned long long *__restrict__ ctr,
                             int levels, const int *__restrict__ flags,
                             int64_t *__restrict__ mail) {
   if (threadIdx.x != 0) return;
-  mail[0] = (int64_t)ctr[2 + levels];
-  mail[1] = (int64_t)ctr[0];
-  mail[2] = (int64_t)ctr[1];
-  mail[3] = *flags;
-  for (int k = 0; k < 56; ++k) mail[4 + k] = k <= levels ? (int64_t)ctr[2 + k] : 0;
+  mail_put(mail + 0, (int64_t)ctr[2 + levels]);
+  mail_put(mail + 1, (int64_t)ctr[0]);
+  mail_put(mail + 2, (int64_t)ctr[1]);
+  mail_put(mail + 3, *flags);
+  for (int k = 0; k < 56; ++k)
+    mail_put(mail + 4 + k, k <= levels ? (int64_t)ctr[2 + k] : 0);
 }
 
 __global__ void k_pair_init(int2 *q, unsigned long long *ctr) {
@@ -928,11 +953,11 @@ __global__ void k_walk_mail(const int *__restrict__ flags,
     sum += __shfl_xor(sum, o, 64);
   }
   if (lane == 0) {
-    mail[0] = *flags;
-    mail[1] = mx;
-    mail[2] = *p2p_total;
-    mail[3] = *scan_word;
-    mail[4] = sum;
+    mail_put(mail + 0, *flags);
+    mail_put(mail + 1, mx);
+    mail_put(mail + 2, *p2p_total);
+    mail_put(mail + 3, *scan_word);
+    mail_put(mail + 4, sum);
   }
 }
 
@@ -1311,8 +1336,8 @@ int pairs_path(Ctx *c, const Cells &cells, const T *Q, T *Lc) {
       FSPH_HIP(c, hipGetLastError());
       done += batch;
       k_pair_mail<<<1, 64, 0, c->stream>>>(ctr, done, c->flags.as<int>(),
-                                           c->mail.as<int64_t>());
-      FSPH_TRY(read_mail(c, 4 + 56));
+                                           c->mail_d);
+      FSPH_TRY(read_mail(c));
       pending = c->mail_h[0];
       h1 = c->mail_h[1];
       h2 = c->mail_h[2];
@@ -1450,9 +1475,9 @@ int walk_path(Ctx *c, const Cells &cells, const T *Q, T *Lc, int *fallback) {
     k_walk_mail<<<1, 64, 0, c->stream>>>(wflag, used, scap,
                                          G.p2p_off.as<int64_t>() + nc,
                                          c->flags.as<int>() + kScanWord,
-                                         c->mail.as<int64_t>());
+                                         c->mail_d);
     FSPH_HIP(c, hipGetLastError());
-    FSPH_TRY(read_mail(c, 5));
+    FSPH_TRY(read_mail(c));
     if (c->mail_h[3] & kFlagScanStall)
       return fail(c, FSPH_E_HIP, "scan: a tile's look-back did not complete");
     const int fl = (int)c->mail_h[0];
@@ -1547,9 +1572,23 @@ template <class T> int gravity_impl(Ctx *c) {
   k_p2m<T><<<blocks_for(nc), kT, 0, c->stream>>>(
       cells, nc, c->f[PF_X].as<double>(), c->f[PF_Y].as<double>(),
       c->f[PF_Z].as<double>(), c->f[PF_M].as<double>(), Q, (T)c->p.G, prel);
+  LevelOff lo{};
+  for (int d = 0; d <= c->max_depth + 1; ++d)
+    lo.off[d] = (int32_t)c->level_off[d];
   for (int d = c->max_depth; d >= 0; --d) {
     const int64_t cnt = c->level_off[d + 1] - c->level_off[d];
     if (!cnt) continue;
+    int e = d;  // levels e .. d make a chain
+    while (e > 0 && cnt <= kChainCells &&
+           c->level_off[e] - c->level_off[e - 1] <= kChainCells)
+      --e;
+    if (e < d) {
+      k_m2m_chain<T><<<1, kChainThreads, 0, c->stream>>>(
+          cells, c->nlevel.as<int32_t>(), lo, e, d, G.nodecell.as<int32_t>(),
+          Q);
+      d = e;
+      continue;
+    }
     k_m2m<T><<<blocks_for(cnt), kT, 0, c->stream>>>(
         cells, c->nlevel.as<int32_t>() + c->level_off[d], cnt,
         G.nodecell.as<int32_t>(), Q);

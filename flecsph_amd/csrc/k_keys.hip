@@ -229,66 +229,58 @@ __global__ __launch_bounds__(kT) void k_copy_fill(
 // ---------------------------------------------------------------------------
 // Range (bodies_system.h:231-268) and keys (filling_curve.h:503-525)
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kT) void k_range_partial(
+// Every workgroup reduces its particles to one row of `part`; the last one
+// to finish (ctr counts them) reduces the rows into range and clears ctr.
+__global__ __launch_bounds__(kT) void k_range(
     const double *__restrict__ x, const double *__restrict__ y,
     const double *__restrict__ z, const double *__restrict__ h, int64_t n,
-    double *__restrict__ part) {
+    double *part, int *ctr, double *__restrict__ range) {
 #pragma clang fp contract(off)
   __shared__ double s[6][kT];
-  double lo[3] = {INFINITY, INFINITY, INFINITY};
-  double hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+  __shared__ int last_s;
+  const int t = threadIdx.x;
+  auto reduce = [&]() {
+    __syncthreads();
+    for (int st = kT / 2; st > 0; st >>= 1) {
+      if (t < st)
+        for (int d = 0; d < 3; ++d) {
+          s[d][t] = fmin(s[d][t], s[d][t + st]);
+          s[3 + d][t] = fmax(s[3 + d][t], s[3 + d][t + st]);
+        }
+      __syncthreads();
+    }
+  };
+  double v[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
   const double *X[3] = {x, y, z};
-  for (int64_t i = (int64_t)blockIdx.x * kT + threadIdx.x; i < n;
+  for (int64_t i = (int64_t)blockIdx.x * kT + t; i < n;
        i += (int64_t)gridDim.x * kT) {
     const double hh = h[i];
     for (int d = 0; d < 3; ++d) {
-      const double v = X[d][i];
-      lo[d] = fmin(lo[d], v - hh);
-      hi[d] = fmax(hi[d], v + hh);
+      const double c = X[d][i];
+      v[d] = fmin(v[d], c - hh);
+      v[3 + d] = fmax(v[3 + d], c + hh);
     }
   }
-  for (int d = 0; d < 3; ++d) {
-    s[d][threadIdx.x] = lo[d];
-    s[3 + d][threadIdx.x] = hi[d];
-  }
+  for (int d = 0; d < 6; ++d) s[d][t] = v[d];
+  reduce();
+  if (t < 6) st_agent(part + blockIdx.x * 6 + t, s[t][0]);
+  __threadfence();
   __syncthreads();
-  for (int st = kT / 2; st > 0; st >>= 1) {
-    if (threadIdx.x < st)
-      for (int d = 0; d < 3; ++d) {
-        s[d][threadIdx.x] = fmin(s[d][threadIdx.x], s[d][threadIdx.x + st]);
-        s[3 + d][threadIdx.x] =
-            fmax(s[3 + d][threadIdx.x], s[3 + d][threadIdx.x + st]);
-      }
-    __syncthreads();
-  }
-  if (threadIdx.x < 6) part[blockIdx.x * 6 + threadIdx.x] = s[threadIdx.x][0];
-}
-
-__global__ __launch_bounds__(kT) void k_range_final(double *__restrict__ part,
-                                                    int nb,
-                                                    double *__restrict__ keep) {
-  __shared__ double s[6][kT];
+  if (t == 0) last_s = atomicAdd(ctr, 1) == (int)gridDim.x - 1;
+  __syncthreads();
+  if (!last_s) return;
+  __threadfence();
   for (int d = 0; d < 6; ++d) {
-    double v = d < 3 ? INFINITY : -INFINITY;
-    for (int b = threadIdx.x; b < nb; b += kT) {
-      const double q = part[b * 6 + d];
-      v = d < 3 ? fmin(v, q) : fmax(v, q);
+    double w = d < 3 ? INFINITY : -INFINITY;
+    for (int b = t; b < (int)gridDim.x; b += kT) {
+      const double q = ld_agent(part + b * 6 + d);
+      w = d < 3 ? fmin(w, q) : fmax(w, q);
     }
-    s[d][threadIdx.x] = v;
+    s[d][t] = w;
   }
-  __syncthreads();
-  for (int st = kT / 2; st > 0; st >>= 1) {
-    if (threadIdx.x < st)
-      for (int d = 0; d < 6; ++d)
-        s[d][threadIdx.x] = d < 3 ? fmin(s[d][threadIdx.x], s[d][threadIdx.x + st])
-                                  : fmax(s[d][threadIdx.x], s[d][threadIdx.x + st]);
-    __syncthreads();
-  }
-  // result at the end of the partial array: lo[3], hi[3]
-  if (threadIdx.x < 6) {
-    part[nb * 6 + threadIdx.x] = s[threadIdx.x][0];
-    keep[threadIdx.x] = s[threadIdx.x][0];
-  }
+  reduce();
+  if (t < 6) range[t] = s[t][0];
+  if (t == 0) *ctr = 0;
 }
 
 // range: lo[3], hi[3] (one simulation) or 8 doubles per instance
@@ -622,15 +614,6 @@ __global__ __launch_bounds__(1024) void k_sort_one(
     }
 }
 
-__global__ __launch_bounds__(kT) void k_check_dup(
-    const uint64_t *__restrict__ key, const uint32_t *__restrict__ val,
-    const int32_t *__restrict__ inst, int64_t n, int *flags) {
-  const int64_t i = (int64_t)blockIdx.x * kT + threadIdx.x + 1;
-  if (i < n && key[i] == key[i - 1] &&
-      (!inst || inst[val[i]] == inst[val[i - 1]]))
-    atomicOr(flags, kFlagDupKey);
-}
-
 }  // namespace
 
 int persistent_fields(const Ctx *c, int *out) {
@@ -771,18 +754,18 @@ int stage_range_keys(Ctx *c) {
     return hip_check(c, hipGetLastError(), "k_keys");
   }
   const int nb = (int)std::min<int64_t>(1024, (n + kT - 1) / kT);
-  FSPH_TRY(ensure(c, c->red_tmp, (size_t)(nb + 1) * 6 * sizeof(double)));
-  double *part = c->red_tmp.as<double>();
-  k_range_partial<<<nb, kT, 0, c->stream>>>(
-      c->f[PF_X].as<double>(), c->f[PF_Y].as<double>(),
-      c->f[PF_Z].as<double>(), c->f[PF_H].as<double>(), n, part);
+  FSPH_TRY(ensure(c, c->red_tmp, (size_t)nb * 6 * sizeof(double)));
   FSPH_TRY(ensure(c, c->range_d, 6 * sizeof(double)));
-  k_range_final<<<1, kT, 0, c->stream>>>(part, nb, c->range_d.as<double>());
+  k_range<<<nb, kT, 0, c->stream>>>(
+      c->f[PF_X].as<double>(), c->f[PF_Y].as<double>(),
+      c->f[PF_Z].as<double>(), c->f[PF_H].as<double>(), n,
+      c->red_tmp.as<double>(), c->flags.as<int>() + kRangeCtr,
+      c->range_d.as<double>());
   FSPH_TRY(ensure(c, c->key, (size_t)c->pcap * 8));
   FSPH_TRY(ensure(c, c->val, (size_t)c->pcap * 4));
   k_keys<<<blocks_for(n), kT, 0, c->stream>>>(
       c->f[PF_X].as<double>(), c->f[PF_Y].as<double>(),
-      c->f[PF_Z].as<double>(), n, part + nb * 6, nullptr,
+      c->f[PF_Z].as<double>(), n, c->range_d.as<double>(), nullptr,
       c->key.as<uint64_t>(), c->val.as<uint32_t>());
   c->range_pending = true;  // read back on request (fsph_get_range)
   return hip_check(c, hipGetLastError(), "k_keys");
@@ -840,9 +823,6 @@ int stage_sort(Ctx *c) {
     std::swap(c->key, c->key2);
     std::swap(c->val, c->val2);
   }
-  k_check_dup<<<blocks_for(n), kT, 0, c->stream>>>(k0, v0, inst, n,
-                                                   c->flags.as<int>());
-  FSPH_HIP(c, hipGetLastError());
   FSPH_TRY(permute_particles(c, v0, n));
   return c->batch.n_inst ? batch_segments(c) : 0;
 }

@@ -97,6 +97,7 @@ struct TravArgs {
   // out, per row: position relative to the unit's first particle and
   // squared radius in FP32, what the masks screen with
   float4 *rowrel;
+  int64_t *words;  // out: the unit's mask words (rows x 32-candidate words)
 };
 
 // MAXG: the largest group (64 when group_max <= 64, else kMaxGroup), which
@@ -287,17 +288,10 @@ __global__ __launch_bounds__(kW) void k_traverse(TravArgs a) {
     ncand += tl;
     __syncthreads();
   }
-  if (lane == 0) a.ccount[gi] = overflow ? 0 : (int32_t)ncand;
-}
-
-__global__ __launch_bounds__(256) void k_mask_words(
-    const int32_t *__restrict__ ccount, const int32_t *__restrict__ gcount,
-    const int32_t *__restrict__ glist, int64_t ng,
-    int64_t *__restrict__ words) {
-  const int64_t gi = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (gi < ng) {
-    const int64_t g = glist ? glist[gi] : gi;
-    words[gi] = (int64_t)gcount[g] * ((ccount[gi] + 31) / 32);
+  if (lane == 0) {  // (an overflowed walk leaves zero candidates)
+    const int32_t cc = overflow ? 0 : (int32_t)ncand;
+    a.ccount[gi] = cc;
+    a.words[gi] = (int64_t)gc * ((cc + 31) / 32);
   }
 }
 
@@ -306,8 +300,8 @@ __global__ void k_tile_mail(const int *__restrict__ flags,
                             const int64_t *__restrict__ words,
                             int64_t *__restrict__ mail) {
   if (threadIdx.x == 0) {
-    mail[0] = flags[0] | flags[kScanWord];
-    mail[1] = *words;
+    mail_put(mail + 0, flags[0] | flags[kScanWord]);
+    mail_put(mail + 1, *words);
   }
 }
 
@@ -665,7 +659,9 @@ int build_tiles(Ctx *c, TileBufs tb, bool gather, double scale,
   FSPH_TRY(ensure(c, c->rowrel, (size_t)(c->pcap + kW) * sizeof(float4)));
   for (int attempt = 0;; ++attempt) {
     FSPH_TRY(ensure(c, tb.cand, (size_t)nslots * tb.ccap * 4));
-    FSPH_HIP(c, hipMemsetAsync(c->flags.p, 0, sizeof(int), c->stream));
+    // (update_iteration has cleared the flags for the SPH tiles' first try)
+    if (gather || attempt)
+      FSPH_HIP(c, hipMemsetAsync(c->flags.p, 0, sizeof(int), c->stream));
     TravArgs t{c->f[PF_X].as<double>(), c->f[PF_Y].as<double>(),
                c->f[PF_Z].as<double>(), c->f[PF_H].as<double>(),
                c->nbox.as<double>(),    c->nchild.as<int32_t>(),
@@ -678,7 +674,7 @@ int build_tiles(Ctx *c, TileBufs tb, bool gather, double scale,
                glist,
                c->batch.n_inst ? c->f[PF_INST].as<int32_t>() : nullptr,
                c->batch.n_inst ? c->batch.root.as<int32_t>() : nullptr,
-               c->rowrel.as<float4>()};
+               c->rowrel.as<float4>(),  tb.moff.as<int64_t>()};
     {
       PhaseTimer tm(c, gather ? FSPH_T_H : FSPH_T_TRAVERSE);
       const int tier = c->stack_tier[gather ? 1 : 0];
@@ -705,16 +701,12 @@ int build_tiles(Ctx *c, TileBufs tb, bool gather, double scale,
         go(std::false_type{});
     }
     FSPH_HIP(c, hipGetLastError());
-    // mask offsets (an overflowed traversal leaves zero candidates), then
-    // the flags and the word count in one read-back
-    k_mask_words<<<(unsigned)((nu + 255) / 256), 256, 0, c->stream>>>(
-        tb.ccount.as<int32_t>(), ucount, glist, nu, tb.moff.as<int64_t>());
-    FSPH_HIP(c, hipGetLastError());
+    // mask offsets, then the flags and the word count in one read-back
     FSPH_TRY(scan_i64(c, tb.moff.as<int64_t>(), tb.moff.as<int64_t>(), nu));
     k_tile_mail<<<1, 64, 0, c->stream>>>(c->flags.as<int>(),
                                          tb.moff.as<int64_t>() + nu,
-                                         c->mail.as<int64_t>());
-    FSPH_TRY(read_mail(c, 2));
+                                         c->mail_d);
+    FSPH_TRY(read_mail(c));
     const int fl = (int)c->mail_h[0];
     if (fl & kFlagScanStall)
       return fail(c, FSPH_E_HIP, "scan: a tile's look-back did not complete");

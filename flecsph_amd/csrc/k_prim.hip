@@ -10,33 +10,66 @@ namespace {
 
 constexpr int kScanThreads = 256;
 
+// Inclusive scan over the wavefront with DPP moves (both halves of the word;
+// the sum carries between them).
+template <int CTRL, int ROWS>
+__device__ inline int64_t dpp_add(int64_t v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, CTRL, ROWS,
+                                             0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(
+      0, (int)(uint32_t)((uint64_t)v >> 32), CTRL, ROWS, 0xf, false);
+  return v + (int64_t)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
+}
 __device__ inline int64_t wave_inclusive_scan(int64_t v) {
-  const int lane = threadIdx.x & 63;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    int64_t t = __shfl_up(v, off, 64);
-    if (lane >= off) v += t;
-  }
-  return v;
+  v = dpp_add<0x111, 0xf>(v);  // row_shr 1, 2, 4, 8
+  v = dpp_add<0x112, 0xf>(v);
+  v = dpp_add<0x114, 0xf>(v);
+  v = dpp_add<0x118, 0xf>(v);
+  v = dpp_add<0x142, 0xa>(v);  // lane 15 of rows 0, 2 to rows 1, 3
+  return dpp_add<0x143, 0xc>(v);  // lane 31 to rows 2, 3
+}
+__device__ inline int64_t last_lane(int64_t v) {
+  const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)v, 63);
+  const uint32_t hi =
+      __builtin_amdgcn_readlane((int)(uint32_t)((uint64_t)v >> 32), 63);
+  return (int64_t)(((uint64_t)hi << 32) | lo);
 }
 
-// Exclusive scan of one value per thread over a block of kScanThreads;
-// returns the exclusive prefix and writes the block total to *total.
-__device__ inline int64_t block_exclusive_scan(int64_t v, int64_t *total) {
-  __shared__ int64_t wsum[kScanThreads / 64];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  int64_t inc = wave_inclusive_scan(v);
-  if (lane == 63) wsum[w] = inc;
-  __syncthreads();
-  int64_t base = 0, tot = 0;
+// Exclusive scan of the ROWS x 64 consecutive items from `base` that a
+// wavefront owns, lane l holding item 64 r + l of row r (so that loads and
+// stores are coalesced; with each thread holding consecutive items, 128
+// bytes apart from its neighbour's, the one-workgroup scan took 17 us for
+// 10,000 items, half of it waiting for the strided loads).  v: the items,
+// then their prefixes.  Returns the sum.
+template <int ROWS, class In>
+__device__ inline int64_t scan_rows(const In *in, int64_t base, int rows,
+                                    int64_t n, int64_t (&v)[ROWS]) {
+  const int lane = threadIdx.x & 63;
 #pragma unroll
-  for (int i = 0; i < kScanThreads / 64; ++i) {
-    if (i < w) base += wsum[i];
-    tot += wsum[i];
+  for (int r = 0; r < ROWS; ++r) {
+    const int64_t i = base + r * 64 + lane;
+    v[r] = r < rows && i < n ? (int64_t)in[i] : 0;
   }
-  __syncthreads();
-  *total = tot;
-  return base + inc - v;
+  int64_t run = 0;
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r)
+    if (r < rows) {
+      const int64_t inc = wave_inclusive_scan(v[r]);
+      v[r] = run + inc - v[r];
+      run += last_lane(inc);
+    }
+  return run;
+}
+template <int ROWS>
+__device__ inline void put_rows(int64_t *out, int64_t base, int rows,
+                                int64_t n, int64_t ex,
+                                const int64_t (&v)[ROWS]) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r) {
+    const int64_t i = base + r * 64 + lane;
+    if (r < rows && i < n) out[i] = ex + v[r];
+  }
 }
 
 // Single-pass scan.  Each workgroup draws its tile from a counter (so every
@@ -92,17 +125,19 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_one(
        j += (int64_t)nt * kScanThreads)
     S.clear[j] = 0;
   if (tile == 0 && threadIdx.x == 0) *S.ctr_clear = 0;
-  const int64_t base =
-      (int64_t)tile * kOneTile + (int64_t)threadIdx.x * kOneItems;
+  __shared__ int64_t wsum[kScanThreads / 64];
+  const int w = threadIdx.x >> 6;
+  const int64_t base = (int64_t)tile * kOneTile + w * (kOneItems * 64);
   int64_t v[kOneItems];
-  int64_t s = 0;
+  const int64_t s = scan_rows<kOneItems>(in, base, kOneItems, n, v);
+  if (lane == 0) wsum[w] = s;
+  __syncthreads();
+  int64_t ex = 0, tot = 0;
 #pragma unroll
-  for (int i = 0; i < kOneItems; ++i) {
-    v[i] = (base + i < n) ? (int64_t)in[base + i] : 0;
-    s += v[i];
+  for (int i = 0; i < kScanThreads / 64; ++i) {
+    if (i < w) ex += wsum[i];
+    tot += wsum[i];
   }
-  int64_t tot;
-  const int64_t ex = block_exclusive_scan(s, &tot);
   if (threadIdx.x < 64) {
     int64_t excl = 0;
     if (tile == 0) {
@@ -140,19 +175,13 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_one(
     if (lane == 0) prefix_s = excl;
   }
   __syncthreads();
-  int64_t e = prefix_s + ex;
-#pragma unroll
-  for (int i = 0; i < kOneItems; ++i) {
-    if (base + i < n) out[base + i] = e;
-    e += v[i];
-  }
+  put_rows(out, base, kOneItems, n, prefix_s + ex, v);
   if (tile == nt - 1 && threadIdx.x == 0) out[n] = prefix_s + tot;
 }
 
 
-// One-workgroup scan: thread t sums its kSmallItems consecutive items, the
-// workgroup scans the sums, and thread t writes its items' prefixes (each
-// item is read before its prefix is written, so in may equal out).
+// One-workgroup scan: wavefront w takes the w-th run of `rows` x 64 items
+// (every item is read before a prefix is written, so in may equal out).
 constexpr int kSmallThreads = 1024;
 constexpr int kSmallItems = 16;
 constexpr int64_t kSmallMax = (int64_t)kSmallThreads * kSmallItems;
@@ -161,29 +190,21 @@ template <class In>
 __global__ __launch_bounds__(kSmallThreads) void k_scan_small(
     const In *in, int64_t n, int64_t *out) {
   __shared__ int64_t wsum[kSmallThreads / 64];
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-  const int64_t base = (int64_t)t * kSmallItems;
-  int64_t s = 0;
-#pragma unroll 16
-  for (int i = 0; i < kSmallItems; ++i)
-    if (base + i < n) s += (int64_t)in[base + i];
-  const int64_t inc = wave_inclusive_scan(s);
-  if (lane == 63) wsum[w] = inc;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int rows = (int)((n + kSmallThreads - 1) / kSmallThreads);
+  const int64_t base = (int64_t)w * rows * 64;
+  int64_t v[kSmallItems];
+  const int64_t s = scan_rows<kSmallItems>(in, base, rows, n, v);
+  if (lane == 0) wsum[w] = s;
   __syncthreads();
-  int64_t ex = inc - s, tot = 0;
+  int64_t ex = 0, tot = 0;
 #pragma unroll
   for (int i = 0; i < kSmallThreads / 64; ++i) {
     if (i < w) ex += wsum[i];
     tot += wsum[i];
   }
-#pragma unroll 16
-  for (int i = 0; i < kSmallItems; ++i)
-    if (base + i < n) {
-      const int64_t x = (int64_t)in[base + i];
-      out[base + i] = ex;
-      ex += x;
-    }
-  if (t == 0) out[n] = tot;
+  put_rows(out, base, rows, n, ex, v);
+  if (threadIdx.x == 0) out[n] = tot;
 }
 
 template <class In>

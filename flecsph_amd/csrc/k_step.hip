@@ -62,16 +62,35 @@ __global__ __launch_bounds__(kT) void k_integrate(IntArgs<T> a, int64_t n,
 // The clock of a single simulation: ts = {dt, totaltime, totaltime_next}.
 // set_adaptive_timestep (default_physics.h:762-823, no output matching) on
 // the reduced minimum, in the host code's operation order.
-__global__ void k_dt_rule(const double *__restrict__ dtmin, double *ts) {
+__device__ inline void dt_rule_device(double m, double *ts) {
 #pragma clang fp contract(off)
-  if (threadIdx.x != 0) return;
-  const double m = *dtmin, t = ts[1];
+  const double t = ts[1];
   double dt = ts[0];
   if (m < dt) dt = (dt / 2.0 < m) ? dt / 2.0 : m;
   if (m > 2.0 * dt) dt = dt * 2.0;
   const double tn = t + dt;
   ts[0] = tn - t;
   ts[2] = tn;
+}
+
+// The state check's words and the scan word into the mailbox.
+__device__ inline void step_mail(int *flags, int64_t *mail) {
+  const uint32_t w0 = (uint32_t)__hip_atomic_load(
+      flags + kCheckWord, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const uint32_t w1 = (uint32_t)__hip_atomic_load(
+      flags + kCheckWord + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  mail_put(mail + kMailCheck, (int64_t)(((uint64_t)w1 << 32) | w0));
+  mail_put(mail + kMailScan, flags[kScanWord]);
+}
+__global__ void k_step_mail(int *flags, int64_t *mail) {
+  if (threadIdx.x == 0) step_mail(flags, mail);
+}
+
+__global__ __launch_bounds__(64) void k_begin(int *flags,
+                                              unsigned long long *lvl) {
+  const int t = threadIdx.x;
+  if (t < 16) flags[t] = t == kCheckWord + 1 ? kCheckNone : 0;
+  if (t < kMaxDepth + 2) lvl[t] = 0;
 }
 
 __global__ void k_advance(double *ts, int adaptive) {
@@ -87,15 +106,21 @@ __global__ void k_set_time(double *ts, double dt, double t, double tn) {
   }
 }
 
+template <class T> struct HArgs {
+  double *h;
+  const double *m;
+  const T *rho;
+  double eta, kw;
+};
 template <class T>
-__global__ __launch_bounds__(kT) void k_update_h(double *h, const double *m,
-                                                 const T *rho, int64_t n,
-                                                 double eta_kw_eta,
-                                                 double kw) {
+__device__ inline void update_h_one(const HArgs<T> &a, int64_t i) {
 #pragma clang fp contract(off)
+  a.h[i] = cbrt(a.m[i] / (double)a.rho[i]) * a.eta * a.kw;
+}
+template <class T>
+__global__ __launch_bounds__(kT) void k_update_h(HArgs<T> a, int64_t n) {
   const int64_t i = (int64_t)blockIdx.x * kT + threadIdx.x;
-  if (i >= n) return;
-  h[i] = cbrt(m[i] / (double)rho[i]) * eta_kw_eta * kw;
+  if (i < n) update_h_one(a, i);
 }
 
 template <class T> struct DtArgs {
@@ -131,67 +156,158 @@ __device__ inline double particle_dt(const DtArgs<T> &a, int64_t i) {
   return a.cfl * smin(smin(dt_v, dt_a), dt_c);
 }
 
+// check_nans and check_negativity (default_physics.h:918-979) over every
+// particle: a NaN in any field the reference checks sets kFlagNaN, a
+// negative density, pressure or internal energy kFlagNeg, and the lowest
+// offending index is kept (out[0] flags, out[1] index).
+template <class T> struct CheckArgs {
+  const double *d[12];  // x y z vx vy vz vhx vhy vhz m u, adiabat (or null)
+  const T *r[11];       // ax ay az gx gy gz phi rho P dudt vsig
+  const double *e;      // thermokinetic energy and de/dt (or null)
+  const T *dedt;
+  int evolve_u;         // evolve_internal_energy: u is checked
+  // the energy rate the configuration computes (du/dt, de/dt or neither):
+  // the other is 0 in every body_u of the reference, and here is never
+  // written (WALL copies would read stale memory), so it is not checked
+  int check_dudt, check_dedt;
+  int *out;
+};
+
 template <class T>
-__global__ __launch_bounds__(kT) void k_dt_partial(DtArgs<T> a, int64_t n,
-                                                   double *part) {
+__device__ inline void check_one(const CheckArgs<T> &a, int64_t i) {
+  bool nan = false;
+#pragma unroll
+  for (int q = 0; q < 10; ++q) nan |= a.d[q][i] != a.d[q][i];
+  if (a.evolve_u) nan |= a.d[10][i] != a.d[10][i];
+  if (a.d[11]) nan |= a.d[11][i] != a.d[11][i];
+#pragma unroll
+  for (int q = 0; q < 11; ++q)
+    if (q != 9 || a.check_dudt) nan |= a.r[q][i] != a.r[q][i];
+  bool neg = a.r[7][i] < T(0) || a.r[8][i] < T(0) ||
+             (a.evolve_u && a.d[10][i] < 0.0);
+  if (a.e) {
+    nan |= a.e[i] != a.e[i];
+    if (a.check_dedt) nan |= a.dedt[i] != a.dedt[i];
+    // recover_internal_energy stops at u <= 0 (default_physics.h:134-143)
+    if (a.evolve_u) neg |= !(a.d[10][i] > 0.0);
+  }
+  if (nan || neg) {
+    atomicOr(&a.out[0], (nan ? kFlagNaN : 0) | (neg ? kFlagNeg : 0));
+    atomicMin(&a.out[1], (int)i);
+  }
+}
+
+template <class T>
+__global__ __launch_bounds__(kT) void k_check_state(CheckArgs<T> a,
+                                                    int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * kT + threadIdx.x;
+  if (i < n) check_one(a, i);
+}
+
+// Several per-particle stages and the time-step minimum in one launch, for
+// one simulation: the energy kick `what`, the closed-form h (do_h) and the
+// state check (do_check), each particle's in that order, then its dt.  The
+// last workgroup to finish reduces the rows, applies the time-step rule and,
+// at the end of a step, advances the clock and fills the mailbox.  As eight
+// launches (kick, h, check with two fills, partial and final minimum, rule,
+// clock) and two copies these took 45 us per step at 2,000 particles, where
+// each is a launch's latency; the fields that several of them read are also
+// read once.
+template <class T> struct TailArgs {
+  IntArgs<T> ia;
+  HArgs<T> ha;
+  CheckArgs<T> ca;
+  DtArgs<T> da;
+  uint32_t what;
+  int do_h, do_check, end;
+  double *part, *ts;
+  int *flags;
+  int64_t *mail;
+};
+
+template <class T>
+__global__ __launch_bounds__(kT) void k_tail(TailArgs<T> a, int64_t n) {
   __shared__ double s[kT];
+  __shared__ int last_s;
+  const int t = threadIdx.x;
+  const double dt = a.ts[0];
   double dmin = 1e24;
-  for (int64_t i = (int64_t)blockIdx.x * kT + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * kT)
-    dmin = smin(dmin, particle_dt(a, i));
-  s[threadIdx.x] = dmin;
-  __syncthreads();
-  for (int st = kT / 2; st > 0; st >>= 1) {
-    if (threadIdx.x < st) s[threadIdx.x] = smin(s[threadIdx.x], s[threadIdx.x + st]);
-    __syncthreads();
+  for (int64_t i = (int64_t)blockIdx.x * kT + t; i < n;
+       i += (int64_t)gridDim.x * kT) {
+    if (a.what) integrate_one(a.ia, i, a.what, dt);
+    if (a.do_h) update_h_one(a.ha, i);
+    if (a.do_check) check_one(a.ca, i);
+    dmin = smin(dmin, particle_dt(a.da, i));
   }
-  if (threadIdx.x == 0) part[blockIdx.x] = s[0];
-}
-
-__global__ __launch_bounds__(kT) void k_min_final(double *part, int nb) {
-  __shared__ double s[kT];
+  auto reduce = [&](double v) {
+    s[t] = v;
+    __syncthreads();
+    for (int st = kT / 2; st > 0; st >>= 1) {
+      if (t < st) s[t] = smin(s[t], s[t + st]);
+      __syncthreads();
+    }
+    return s[0];
+  };
+  const double row = reduce(dmin);
+  if (t == 0) {
+    st_agent(a.part + blockIdx.x, row);
+    __threadfence();
+    last_s = atomicAdd(a.flags + kDtCtr, 1) == (int)gridDim.x - 1;
+  }
+  __syncthreads();
+  if (!last_s) return;
+  __threadfence();
   double v = 1e24;
-  for (int b = threadIdx.x; b < nb; b += kT) v = smin(v, part[b]);
-  s[threadIdx.x] = v;
-  __syncthreads();
-  for (int st = kT / 2; st > 0; st >>= 1) {
-    if (threadIdx.x < st) s[threadIdx.x] = smin(s[threadIdx.x], s[threadIdx.x + st]);
-    __syncthreads();
+  for (int b = t; b < (int)gridDim.x; b += kT) v = smin(v, ld_agent(a.part + b));
+  const double m = reduce(v);
+  if (t != 0) return;
+  a.flags[kDtCtr] = 0;
+  dt_rule_device(m, a.ts);
+  if (a.end) {
+    a.ts[1] = a.ts[2];
+    step_mail(a.flags, a.mail);
   }
-  if (threadIdx.x == 0) part[nb] = s[0];
 }
 
-__global__ __launch_bounds__(kT) void k_max_partial(const double *v, int64_t n,
-                                                    double *part) {
+// max of v and 2.5 times it (getSmoothinglength's halo) into out[0], out[1]
+__global__ __launch_bounds__(kT) void k_max(const double *v, int64_t n,
+                                            double *part, int *ctr,
+                                            double *out) {
   __shared__ double s[kT];
+  __shared__ int last_s;
+  const int t = threadIdx.x;
+  auto reduce = [&](double x) {
+    s[t] = x;
+    __syncthreads();
+    for (int st = kT / 2; st > 0; st >>= 1) {
+      if (t < st && s[t] < s[t + st]) s[t] = s[t + st];
+      __syncthreads();
+    }
+    return s[0];
+  };
   double mx = 0;
-  for (int64_t i = (int64_t)blockIdx.x * kT + threadIdx.x; i < n;
+  for (int64_t i = (int64_t)blockIdx.x * kT + t; i < n;
        i += (int64_t)gridDim.x * kT)
     mx = (mx < v[i]) ? v[i] : mx;
-  s[threadIdx.x] = mx;
-  __syncthreads();
-  for (int st = kT / 2; st > 0; st >>= 1) {
-    if (threadIdx.x < st && s[threadIdx.x] < s[threadIdx.x + st])
-      s[threadIdx.x] = s[threadIdx.x + st];
-    __syncthreads();
+  const double row = reduce(mx);
+  if (t == 0) {
+    st_agent(part + blockIdx.x, row);
+    __threadfence();
+    last_s = atomicAdd(ctr, 1) == (int)gridDim.x - 1;
   }
-  if (threadIdx.x == 0) part[blockIdx.x] = s[0];
-}
-
-__global__ __launch_bounds__(kT) void k_max_final(double *part, int nb) {
-  __shared__ double s[kT];
-  double mx = 0;
-  for (int b = threadIdx.x; b < nb; b += kT) mx = (mx < part[b]) ? part[b] : mx;
-  s[threadIdx.x] = mx;
   __syncthreads();
-  for (int st = kT / 2; st > 0; st >>= 1) {
-    if (threadIdx.x < st && s[threadIdx.x] < s[threadIdx.x + st])
-      s[threadIdx.x] = s[threadIdx.x + st];
-    __syncthreads();
+  if (!last_s) return;
+  __threadfence();
+  mx = 0;
+  for (int b = t; b < (int)gridDim.x; b += kT) {
+    const double q = ld_agent(part + b);
+    mx = (mx < q) ? q : mx;
   }
-  if (threadIdx.x == 0) {
-    part[nb] = s[0];
-    part[nb + 1] = 2.5 * s[0];  // getSmoothinglength's halo
+  const double m = reduce(mx);
+  if (t == 0) {
+    *ctr = 0;
+    out[0] = m;
+    out[1] = 2.5 * m;
   }
 }
 
@@ -420,10 +536,7 @@ __global__ __launch_bounds__(kT) void k_seg_roots(
 template <class T> struct StepSlot {
   IntArgs<T> ia;
   DtArgs<T> da;
-  double *h;
-  const double *m;
-  const T *rho;
-  double eta, kw;
+  HArgs<T> ha;
   const int32_t *inst;
   const double *dtv;
   double *bounds;
@@ -438,10 +551,9 @@ __global__ __launch_bounds__(kT) void k_integrate_p(StepSlot<T> s, int64_t n) {
 
 template <class T>
 __global__ __launch_bounds__(kT) void k_update_h_p(StepSlot<T> s, int64_t n) {
-#pragma clang fp contract(off)
   for (int64_t i = (int64_t)blockIdx.x * kT + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * kT)
-    s.h[i] = cbrt(s.m[i] / (double)s.rho[i]) * s.eta * s.kw;
+    update_h_one(s.ha, i);
 }
 
 template <class T>
@@ -464,17 +576,28 @@ template <class T> DtArgs<T> dt_args(Ctx *c) {
                    c->p.visc_alpha};
 }
 
+template <class T> IntArgs<T> int_args(Ctx *c) {
+  return IntArgs<T>{c->f[PF_X].as<double>(),   c->f[PF_Y].as<double>(),
+                    c->f[PF_Z].as<double>(),   c->f[PF_VX].as<double>(),
+                    c->f[PF_VY].as<double>(),  c->f[PF_VZ].as<double>(),
+                    c->f[PF_VHX].as<double>(), c->f[PF_VHY].as<double>(),
+                    c->f[PF_VHZ].as<double>(), c->f[PF_U].as<double>(),
+                    c->f[PF_AX].as<T>(),       c->f[PF_AY].as<T>(),
+                    c->f[PF_AZ].as<T>(),       c->f[PF_GX].as<T>(),
+                    c->f[PF_GY].as<T>(),       c->f[PF_GZ].as<T>(),
+                    c->f[PF_DUDT].as<T>(),     c->f[PF_E].as<double>(),
+                    c->f[PF_DEDT].as<T>()};
+}
+
+template <class T> HArgs<T> h_args(Ctx *c) {
+  return HArgs<T>{c->f[PF_H].as<double>(), c->f[PF_M].as<double>(),
+                  c->f[PF_RHO].as<T>(), c->p.eta, 2.0};  // kernels.h:753-756
+}
+
+template <class T> CheckArgs<T> check_args(Ctx *c);  // below
+
 template <class T> int integrate_impl(Ctx *c, uint32_t what) {
-  IntArgs<T> a{c->f[PF_X].as<double>(),   c->f[PF_Y].as<double>(),
-               c->f[PF_Z].as<double>(),   c->f[PF_VX].as<double>(),
-               c->f[PF_VY].as<double>(),  c->f[PF_VZ].as<double>(),
-               c->f[PF_VHX].as<double>(), c->f[PF_VHY].as<double>(),
-               c->f[PF_VHZ].as<double>(), c->f[PF_U].as<double>(),
-               c->f[PF_AX].as<T>(),       c->f[PF_AY].as<T>(),
-               c->f[PF_AZ].as<T>(),       c->f[PF_GX].as<T>(),
-               c->f[PF_GY].as<T>(),       c->f[PF_GZ].as<T>(),
-               c->f[PF_DUDT].as<T>(),     c->f[PF_E].as<double>(),
-               c->f[PF_DEDT].as<T>()};
+  const IntArgs<T> a = int_args<T>(c);
   const bool b = c->batch.n_inst > 0;
   k_integrate<T><<<blocks_for(c->n), kT, 0, c->stream>>>(
       a, c->n, what, 0.0,
@@ -483,21 +606,27 @@ template <class T> int integrate_impl(Ctx *c, uint32_t what) {
   return hip_check(c, hipGetLastError(), "k_integrate");
 }
 
-template <class T> int dt_impl(Ctx *c) {
+// The time-step rule; `end`: as the end of a step, after the kick `what`,
+// the closed-form h and the state check.
+template <class T> int tail_impl(Ctx *c, bool end, uint32_t what) {
   const int nb = (int)std::min<int64_t>(1024, (c->n + kT - 1) / kT);
-  FSPH_TRY(ensure(c, c->red_tmp, (size_t)(nb + 1) * 8));
-  double *part = c->red_tmp.as<double>();
-  DtArgs<T> a{c->f[PF_H].as<double>(), c->f[PF_VX].as<double>(),
-              c->f[PF_VY].as<double>(), c->f[PF_VZ].as<double>(),
-              c->f[PF_AX].as<T>(), c->f[PF_AY].as<T>(), c->f[PF_AZ].as<T>(),
-              c->f[PF_GX].as<T>(), c->f[PF_GY].as<T>(), c->f[PF_GZ].as<T>(),
-              c->f[PF_VSIG].as<T>(), c->p.eta * 2.0, c->p.cfl,
-              c->p.visc_alpha};
-  k_dt_partial<T><<<nb, kT, 0, c->stream>>>(a, c->n, part);
-  k_min_final<<<1, kT, 0, c->stream>>>(part, nb);
-  k_dt_rule<<<1, 64, 0, c->stream>>>(part + nb, c->tstate.as<double>());
+  FSPH_TRY(ensure(c, c->red_tmp, (size_t)nb * 8));
+  TailArgs<T> a{};
+  a.ia = int_args<T>(c);
+  a.ha = h_args<T>(c);
+  a.ca = check_args<T>(c);
+  a.da = dt_args<T>(c);
+  a.what = what;
+  a.do_h = end && c->p.h_mode == FSPH_H_CLOSED;
+  a.do_check = end && c->checks;
+  a.end = end;
+  a.part = c->red_tmp.as<double>();
+  a.ts = c->tstate.as<double>();
+  a.flags = c->flags.as<int>();
+  a.mail = c->mail_d;
+  k_tail<T><<<nb, kT, 0, c->stream>>>(a, c->n);
   c->time_dirty = true;
-  return hip_check(c, hipGetLastError(), "k_dt_rule");
+  return hip_check(c, hipGetLastError(), "k_tail");
 }
 
 // Workgroups of the reduction: at most kRedRows, each writes one row of 10
@@ -586,63 +715,17 @@ int stage_integrate(Ctx *c, uint32_t what) {
 }
 
 int stage_update_h(Ctx *c) {
-  const double kw = 2.0;  // kernels.h:753-756
   if (c->rsize == 4)
     k_update_h<float><<<blocks_for(c->n), kT, 0, c->stream>>>(
-        c->f[PF_H].as<double>(), c->f[PF_M].as<double>(),
-        c->f[PF_RHO].as<float>(), c->n, c->p.eta, kw);
+        h_args<float>(c), c->n);
   else
     k_update_h<double><<<blocks_for(c->n), kT, 0, c->stream>>>(
-        c->f[PF_H].as<double>(), c->f[PF_M].as<double>(),
-        c->f[PF_RHO].as<double>(), c->n, c->p.eta, kw);
+        h_args<double>(c), c->n);
   return hip_check(c, hipGetLastError(), "k_update_h");
 }
 
-// check_nans and check_negativity (default_physics.h:918-979) over every
-// particle: a NaN in any field the reference checks sets kFlagNaN, a
-// negative density, pressure or internal energy kFlagNeg, and the lowest
-// offending index is kept (out[0] flags, out[1] index).
-template <class T> struct CheckArgs {
-  const double *d[12];  // x y z vx vy vz vhx vhy vhz m u, adiabat (or null)
-  const T *r[11];       // ax ay az gx gy gz phi rho P dudt vsig
-  const double *e;      // thermokinetic energy and de/dt (or null)
-  const T *dedt;
-  int evolve_u;         // evolve_internal_energy: u is checked
-  // the energy rate the configuration computes (du/dt, de/dt or neither):
-  // the other is 0 in every body_u of the reference, and here is never
-  // written (WALL copies would read stale memory), so it is not checked
-  int check_dudt, check_dedt;
-  int *out;
-};
-
-template <class T>
-__global__ __launch_bounds__(kT) void k_check_state(CheckArgs<T> a,
-                                                    int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * kT + threadIdx.x;
-  if (i >= n) return;
-  bool nan = false;
-#pragma unroll
-  for (int q = 0; q < 10; ++q) nan |= a.d[q][i] != a.d[q][i];
-  if (a.evolve_u) nan |= a.d[10][i] != a.d[10][i];
-  if (a.d[11]) nan |= a.d[11][i] != a.d[11][i];
-#pragma unroll
-  for (int q = 0; q < 11; ++q)
-    if (q != 9 || a.check_dudt) nan |= a.r[q][i] != a.r[q][i];
-  bool neg = a.r[7][i] < T(0) || a.r[8][i] < T(0) ||
-             (a.evolve_u && a.d[10][i] < 0.0);
-  if (a.e) {
-    nan |= a.e[i] != a.e[i];
-    if (a.check_dedt) nan |= a.dedt[i] != a.dedt[i];
-    // recover_internal_energy stops at u <= 0 (default_physics.h:134-143)
-    if (a.evolve_u) neg |= !(a.d[10][i] > 0.0);
-  }
-  if (nan || neg) {
-    atomicOr(&a.out[0], (nan ? kFlagNaN : 0) | (neg ? kFlagNeg : 0));
-    atomicMin(&a.out[1], (int)i);
-  }
-}
-
-template <class T> int check_impl(Ctx *c, int *out) {
+namespace {
+template <class T> CheckArgs<T> check_args(Ctx *c) {
   CheckArgs<T> a{};
   const int df[11] = {PF_X,   PF_Y,   PF_Z,   PF_VX, PF_VY, PF_VZ,
                       PF_VHX, PF_VHY, PF_VHZ, PF_M,  PF_U};
@@ -659,22 +742,38 @@ template <class T> int check_impl(Ctx *c, int *out) {
   a.evolve_u = c->p.evolve_internal_energy;
   a.check_dudt = c->p.evolve_internal_energy && !c->p.thermokinetic;
   a.check_dedt = c->p.evolve_internal_energy && c->p.thermokinetic;
-  a.out = out;
-  k_check_state<T><<<blocks_for(c->n), kT, 0, c->stream>>>(a, c->n);
+  a.out = c->flags.as<int>() + kCheckWord;
+  return a;
+}
+}  // namespace
+
+int stage_check_state(Ctx *c, bool reset) {
+  if (c->n <= 0) return 0;
+  if (reset) FSPH_TRY(stage_begin(c));
+  if (c->rsize == 4)
+    k_check_state<float><<<blocks_for(c->n), kT, 0, c->stream>>>(
+        check_args<float>(c), c->n);
+  else
+    k_check_state<double><<<blocks_for(c->n), kT, 0, c->stream>>>(
+        check_args<double>(c), c->n);
   return hip_check(c, hipGetLastError(), "k_check_state");
 }
 
-int stage_check_state(Ctx *c) {
-  if (c->n <= 0) return 0;
-  int *out = c->flags.as<int>() + kCheckWord;
-  FSPH_HIP(c, hipMemsetAsync(out, 0, 4, c->stream));
-  FSPH_HIP(c, hipMemsetAsync(out + 1, 0x7f, 4, c->stream));
-  FSPH_TRY(c->rsize == 4 ? check_impl<float>(c, out)
-                         : check_impl<double>(c, out));
-  // into the mailbox's host copy; read after the caller's synchronisation
-  FSPH_HIP(c, hipMemcpyAsync(c->mail_h + kMailCheck, out, 8,
-                             hipMemcpyDeviceToHost, c->stream));
-  return 0;
+int stage_step_mail(Ctx *c) {
+  k_step_mail<<<1, 64, 0, c->stream>>>(c->flags.as<int>(), c->mail_d);
+  return hip_check(c, hipGetLastError(), "k_step_mail");
+}
+
+int stage_begin(Ctx *c) {
+  FSPH_TRY(ensure(c, c->lvl, 2 * (kMaxDepth + 2) * 8));
+  k_begin<<<1, 64, 0, c->stream>>>(c->flags.as<int>(),
+                                   c->lvl.as<unsigned long long>());
+  return hip_check(c, hipGetLastError(), "k_begin");
+}
+
+int stage_step_tail(Ctx *c, uint32_t what) {
+  return c->rsize == 4 ? tail_impl<float>(c, true, what)
+                       : tail_impl<double>(c, true, what);
 }
 
 // initialize_alpha (viscosity.h:164-171): 0 for the Cullen-Dehnen switch,
@@ -755,22 +854,9 @@ int stage_eos_init(Ctx *c) {
 template <class T> void step_graph_args_t(Ctx *c, char *slot) {
   static_assert(sizeof(StepSlot<T>) <= kGraphSlot, "slot");
   StepSlot<T> s{};
-  s.ia = IntArgs<T>{c->f[PF_X].as<double>(),   c->f[PF_Y].as<double>(),
-                    c->f[PF_Z].as<double>(),   c->f[PF_VX].as<double>(),
-                    c->f[PF_VY].as<double>(),  c->f[PF_VZ].as<double>(),
-                    c->f[PF_VHX].as<double>(), c->f[PF_VHY].as<double>(),
-                    c->f[PF_VHZ].as<double>(), c->f[PF_U].as<double>(),
-                    c->f[PF_AX].as<T>(),       c->f[PF_AY].as<T>(),
-                    c->f[PF_AZ].as<T>(),       c->f[PF_GX].as<T>(),
-                    c->f[PF_GY].as<T>(),       c->f[PF_GZ].as<T>(),
-                    c->f[PF_DUDT].as<T>(),     c->f[PF_E].as<double>(),
-                    c->f[PF_DEDT].as<T>()};
+  s.ia = int_args<T>(c);
   s.da = dt_args<T>(c);
-  s.h = c->f[PF_H].as<double>();
-  s.m = c->f[PF_M].as<double>();
-  s.rho = c->f[PF_RHO].as<T>();
-  s.eta = c->p.eta;
-  s.kw = 2.0;  // kernels.h:753-756
+  s.ha = h_args<T>(c);
   s.inst = c->f[PF_INST].as<int32_t>();
   s.dtv = c->batch.dt.as<double>();
   s.bounds = c->batch.bounds.as<double>();
@@ -860,7 +946,8 @@ int batch_roots(Ctx *c) {
 }
 
 int stage_dt_rule(Ctx *c) {
-  return c->rsize == 4 ? dt_impl<float>(c) : dt_impl<double>(c);
+  return c->rsize == 4 ? tail_impl<float>(c, false, 0)
+                       : tail_impl<double>(c, false, 0);
 }
 
 int stage_advance(Ctx *c) {
@@ -899,10 +986,10 @@ int stage_halo(Ctx *c, const double **halo) {
   const int nb = (int)std::min<int64_t>(1024, (c->n + kT - 1) / kT);
   FSPH_TRY(ensure(c, c->red_tmp, (size_t)(nb + 2) * 8));
   double *part = c->red_tmp.as<double>();
-  k_max_partial<<<nb, kT, 0, c->stream>>>(c->f[PF_H].as<double>(), c->n, part);
-  k_max_final<<<1, kT, 0, c->stream>>>(part, nb);
+  k_max<<<nb, kT, 0, c->stream>>>(c->f[PF_H].as<double>(), c->n, part,
+                                  c->flags.as<int>() + kMaxCtr, part + nb);
   *halo = part + nb + 1;
-  return hip_check(c, hipGetLastError(), "k_max_final");
+  return hip_check(c, hipGetLastError(), "k_max");
 }
 
 int convert_to_double(Ctx *c, const void *src, size_t esize, double *dst,

@@ -103,17 +103,25 @@ __device__ inline int64_t containing_node(const uint64_t *__restrict__ k,
 
 // Common-prefix depth of sorted keys i and i+1; -1 at the end of the array
 // (or of an instance, which makes every instance a tree of its own).
+// Equal keys raise kFlagDupKey; the child table's first `rows` rows (the
+// nodes are not counted yet) are set to empty on the way.
 __global__ __launch_bounds__(kT) void k_prefix(const uint64_t *__restrict__ k,
                                                int64_t n,
                                                const int32_t *__restrict__ inst,
-                                               int32_t *__restrict__ L) {
+                                               int32_t *__restrict__ L,
+                                               int4 *__restrict__ child,
+                                               int64_t rows, int *flags) {
   const int64_t i = (int64_t)blockIdx.x * kT + threadIdx.x;
   if (i >= n) return;
+  if (i < rows)
+    child[2 * i] = child[2 * i + 1] =
+        make_int4(kChildEmpty, kChildEmpty, kChildEmpty, kChildEmpty);
   if (i == n - 1 || (inst && inst[i] != inst[i + 1])) {
     L[i] = -1;
     return;
   }
   const uint64_t x = k[i] ^ k[i + 1];
+  if (x == 0) atomicOr(flags, kFlagDupKey);
   const int lz = x ? __clzll(x) : 64;
   int d = (lz - 1) / 3;  // common digits below the leading 1
   L[i] = d > kMaxDepth - 1 ? kMaxDepth - 1 : d;
@@ -164,11 +172,11 @@ __global__ void k_tree_mail(const int64_t *__restrict__ nn,
                             unsigned long long *__restrict__ cursor,
                             int64_t *__restrict__ mail) {
   if (threadIdx.x != 0) return;
-  mail[0] = *nn;
-  mail[1] = flags[0] | flags[kScanWord];
+  mail_put(mail + 0, *nn);
+  mail_put(mail + 1, flags[0] | flags[kScanWord]);
   unsigned long long acc = 0;
   for (int d = 0; d <= kMaxDepth; ++d) {
-    mail[2 + d] = (int64_t)lvl[d];
+    mail_put(mail + 2 + d, (int64_t)lvl[d]);
     cursor[d] = acc;
     acc += lvl[d];
   }
@@ -260,18 +268,26 @@ struct CofmArgs {
 // reductions (mass-weighted sums, box bounds, radius and lap maxima) are then
 // taken serially in the reference's order from LDS, one lane per component,
 // so the results are those of a serial walk over the children.
-constexpr int kCofmNodes = kT / 8;  // nodes per workgroup
-
-__global__ __launch_bounds__(kT) void k_cofm(CofmArgs a,
-                                             const int32_t *__restrict__ ids,
-                                             int64_t cnt) {
-#pragma clang fp contract(off)
+template <int THREADS> struct CofmLds {
   // per child: m*x, m*y, m*z, m, box lo xyz, box hi xyz, radius, lap terms
-  __shared__ double v[kCofmNodes][12][8];
-  __shared__ double sums[kCofmNodes][4];
-  __shared__ int kind[kCofmNodes][8];  // 0 none, 1 particle, 2 node
+  double v[THREADS / 8][12][8];
+  double sums[THREADS / 8][4];
+  int kind[THREADS / 8][8];  // 0 none, 1 particle, 2 node
+};
+
+// The nodes ids[t0 .. min(t0 + THREADS / 8, cnt)) of one level; the
+// aggregates are plainly stored and loaded: no __restrict__ on them, the
+// chained form reads what its own workgroup has written.
+template <int THREADS>
+__device__ inline void cofm_nodes(const CofmArgs &a,
+                                  const int32_t *__restrict__ ids, int64_t t0,
+                                  int64_t cnt, CofmLds<THREADS> &lds) {
+#pragma clang fp contract(off)
+  auto &v = lds.v;
+  auto &sums = lds.sums;
+  auto &kind = lds.kind;
   const int ln = threadIdx.x >> 3, j = threadIdx.x & 7;
-  const int64_t t = (int64_t)blockIdx.x * kCofmNodes + ln;
+  const int64_t t = t0 + ln;
   const bool valid = t < cnt;
   const int64_t nd = valid ? ids[t] : 0;
   const int32_t ch = valid ? a.child[nd * 8 + j] : -1;
@@ -369,6 +385,37 @@ __global__ __launch_bounds__(kT) void k_cofm(CofmArgs a,
   if (j < 2) a.box[6 * nd + 4 + j] = out[1];
 }
 
+constexpr int kCofmNodes = kT / 8;  // nodes per workgroup
+
+__global__ __launch_bounds__(kT) void k_cofm(CofmArgs a,
+                                             const int32_t *__restrict__ ids,
+                                             int64_t cnt) {
+  __shared__ CofmLds<kT> lds;
+  cofm_nodes<kT>(a, ids, (int64_t)blockIdx.x * kCofmNodes, cnt, lds);
+}
+
+// Levels lo .. hi, deepest first, of at most kChainNodes nodes each, in one
+// workgroup: a level of a few nodes is a launch's latency (6 us) for three
+// dependent loads and a division (about 2.5 us a pass of 128 nodes), so up to
+// two passes cost less here.
+constexpr int kChainThreads = 1024;
+constexpr int64_t kChainNodes = 2 * kChainThreads / 8;
+struct LevelOff {
+  int32_t off[kMaxDepth + 2];
+};
+__global__ __launch_bounds__(kChainThreads) void k_cofm_chain(
+    CofmArgs a, const int32_t *__restrict__ level, LevelOff L, int lo,
+    int hi) {
+  __shared__ CofmLds<kChainThreads> lds;
+  for (int d = hi; d >= lo; --d) {
+    const int64_t cnt = L.off[d + 1] - L.off[d];
+    for (int64_t t = 0; t < cnt; t += kChainThreads / 8) {
+      cofm_nodes<kChainThreads>(a, level + L.off[d], t, cnt, lds);
+      __syncthreads();  // (the level's aggregates, and the LDS, are reused)
+    }
+  }
+}
+
 // Groups (tree_topology.h:222-235): nodes with at most gmax particles whose
 // parent has more (or the root), and single leaves whose parent has more.
 // The flag of a group also says how many pair-kernel tiles it makes: a
@@ -437,6 +484,16 @@ __global__ __launch_bounds__(kT) void k_group_write(
   }
 }
 
+// Mailbox of the groups: their packed count and the scan word.
+__global__ void k_group_mail(const int64_t *__restrict__ packed,
+                             const int *__restrict__ scan_word,
+                             int64_t *__restrict__ mail) {
+  if (threadIdx.x == 0) {
+    mail_put(mail + kMail - 1, *packed);
+    mail_put(mail + kMailScan, *scan_word);
+  }
+}
+
 }  // namespace
 
 int group_flags(Ctx *c);  // below
@@ -451,20 +508,21 @@ int stage_tree(Ctx *c) {
   int32_t *L = c->L.as<int32_t>();
   const Seg sg{c->batch.n_inst ? c->f[PF_INST].as<int32_t>() : nullptr,
                c->batch.seg.as<int64_t>(), n};
-  // level histogram and the level order's cursors
-  FSPH_TRY(ensure(c, c->red_tmp, 2 * (kMaxDepth + 2) * 8));
-  unsigned long long *lvl = c->red_tmp.as<unsigned long long>();
+  // level histogram (cleared by stage_begin) and the level order's cursors
+  unsigned long long *lvl = c->lvl.as<unsigned long long>();
   unsigned long long *cursor = lvl + (kMaxDepth + 2);
-  FSPH_HIP(c, hipMemsetAsync(lvl, 0, (kMaxDepth + 2) * 8, c->stream));
-  k_prefix<<<blocks_for(n), kT, 0, c->stream>>>(k, n, sg.inst, L);
+  const int64_t rows = std::min(c->ncap, n);
+  k_prefix<<<blocks_for(n), kT, 0, c->stream>>>(k, n, sg.inst, L,
+                                                c->nchild.as<int4>(), rows,
+                                                c->flags.as<int>());
   k_pair_count<<<std::min<unsigned>(blocks_for(n), kPairCountBlocks), kT, 0,
                  c->stream>>>(L, n, c->pair_cnt.as<int32_t>(), lvl);
   FSPH_HIP(c, hipGetLastError());
   int64_t *off = c->pair_off.as<int64_t>();
   FSPH_TRY(scan_i32_to_i64(c, c->pair_cnt.as<int32_t>(), off, n));
   k_tree_mail<<<1, 64, 0, c->stream>>>(off + n, c->flags.as<int>(), lvl,
-                                       cursor, c->mail.as<int64_t>());
-  FSPH_TRY(read_mail(c, 2 + kMaxDepth + 1));
+                                       cursor, c->mail_d);
+  FSPH_TRY(read_mail(c));
   if (c->mail_h[1] & kFlagScanStall)
     return fail(c, FSPH_E_HIP, "scan: a tile's look-back did not complete");
   if (c->mail_h[1] & kFlagDupKey)
@@ -484,6 +542,7 @@ int stage_tree(Ctx *c) {
     }
     c->level_off[kMaxDepth + 1] = acc;
   }
+  const int64_t filled = nn > c->ncap ? 0 : rows;  // rows k_prefix has set
   if (nn > c->ncap) {
     const int64_t cap = (int64_t)(nn * 1.25) + 1024;
     FSPH_TRY(ensure(c, c->nkey, cap * 8));
@@ -500,7 +559,9 @@ int stage_tree(Ctx *c) {
     FSPH_TRY(ensure(c, c->nlevel, cap * 4));
     c->ncap = cap;
   }
-  FSPH_HIP(c, hipMemsetAsync(c->nchild.p, 0xff, (size_t)nn * 32, c->stream));
+  if (nn > filled)
+    FSPH_HIP(c, hipMemsetAsync(c->nchild.as<char>() + filled * 32, 0xff,
+                               (size_t)(nn - filled) * 32, c->stream));
   NodeOut o{c->nkey.as<uint64_t>(), c->ndepth.as<int32_t>(),
             c->nstart.as<int32_t>(), c->ncount.as<int32_t>(),
             c->nparent.as<int32_t>(), c->nchild.as<int32_t>()};
@@ -523,9 +584,22 @@ int stage_tree(Ctx *c) {
              c->nbox.as<double>(),    c->ncom.as<double>(),
              c->nmass.as<double>(),   c->nrad.as<double>(),
              c->nlap.as<double>()};
+  LevelOff lo{};
+  for (int d = 0; d <= c->max_depth + 1; ++d)
+    lo.off[d] = (int32_t)c->level_off[d];
   for (int d = c->max_depth; d >= 0; --d) {
     const int64_t cntd = c->level_off[d + 1] - c->level_off[d];
     if (!cntd) continue;
+    int e = d;  // levels e .. d make a chain
+    while (e > 0 && cntd <= kChainNodes &&
+           c->level_off[e] - c->level_off[e - 1] <= kChainNodes)
+      --e;
+    if (e < d) {
+      k_cofm_chain<<<1, kChainThreads, 0, c->stream>>>(
+          a, c->nlevel.as<int32_t>(), lo, e, d);
+      d = e;
+      continue;
+    }
     k_cofm<<<(unsigned)((cntd + kCofmNodes - 1) / kCofmNodes), kT, 0,
              c->stream>>>(
         a, c->nlevel.as<int32_t>() + c->level_off[d], cntd);
@@ -548,13 +622,10 @@ int group_flags(Ctx *c) {
       c->gflag.as<int64_t>());
   FSPH_HIP(c, hipGetLastError());
   FSPH_TRY(scan_i64(c, c->gflag.as<int64_t>(), c->gscan.as<int64_t>(), tot));
-  FSPH_HIP(c, hipMemcpyAsync(c->mail_h + (kMail - 1),
-                             c->gscan.as<int64_t>() + tot, 8,
-                             hipMemcpyDeviceToHost, c->stream));
-  c->mail_h[kMailScan] = 0;
-  FSPH_HIP(c, hipMemcpyAsync(c->mail_h + kMailScan,
-                             c->flags.as<int>() + kScanWord, 4,
-                             hipMemcpyDeviceToHost, c->stream));
+  k_group_mail<<<1, 64, 0, c->stream>>>(c->gscan.as<int64_t>() + tot,
+                                        c->flags.as<int>() + kScanWord,
+                                        c->mail_d);
+  FSPH_HIP(c, hipGetLastError());
   FSPH_HIP(c, hipEventRecord(c->ev_groups, c->stream));
   return 0;
 }
