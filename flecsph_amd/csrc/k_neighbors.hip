@@ -18,6 +18,7 @@
 #include <type_traits>
 
 #include "fsph_internal.h"
+#include "pair_sched.h"
 
 namespace fsph {
 
@@ -65,31 +66,23 @@ __device__ inline bool within_distance2(double a0, double a1, double a2,
   return d <= r * r;
 }
 
-__device__ inline int wave_excl_scan(int v, int *total) {
-  const int lane = threadIdx.x & 63;
-  int inc = v;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const int t = __shfl_up(inc, off, 64);
-    if (lane >= off) inc += t;
-  }
-  *total = __shfl(inc, 63, 64);
-  return inc - v;
+__device__ inline float lane_f(float v, int lane) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
 
 struct TravArgs {
   const double *x, *y, *z, *h;
   const double *box;     // 6 per node
+  const double *com, *nrad;  // 3 and 1 per node (gather form)
   const int32_t *child;  // 8 per node
   const int32_t *gstart, *gcount, *gnode;
   int32_t *cand;
   int32_t *ccount;
   int64_t ccap;
   int *flags;
-  // gather mode (smoothing-length solver): sphere radius rscale * h_k and
-  // no group-box test; the SPH mode uses rscale = 1 with the box test.
+  // gather form (smoothing-length solver): sphere radius rscale * h_k and
+  // no group-box test; the SPH form takes h_k and the box test.
   double rscale;
-  int gather;
   const float *hprop;    // gather radius base instead of h (or null)
   const int32_t *glist;  // tile slot -> group (or null: slot = group)
   // batched mode: the walk starts at the root of the group's instance
@@ -104,57 +97,115 @@ struct TravArgs {
 // sizes the group's LDS arrays.
 //
 // A node passes the sphere test if some particle's sphere meets its box.
-// The particles are taken eight at a time: a node box that misses the
-// hull box of a chunk's spheres (each sphere's bounding cube, widened by
-// 1e-9 of |centre| + radius, well beyond the rounding of the sphere test)
-// fails the sphere test of every particle of the chunk, so only chunks
-// whose hull it meets are tested particle by particle.  The accepted nodes
-// are the same.  All hull tests of a node run first, as one unrolled pass
-// (independent instructions; a chunk-by-chunk loop waited on each test),
-// then the spheres of the chunks that passed, in order, until one meets the
-// node (1M polytrope: 0.85 -> 0.63 ms per traversal; chunks of 4 or 16
-// were slower, and so was testing a chunk's eight spheres together).
-constexpr int kHullChunk = 8;
+// The test is FP64 in the reference's operation order; nearly every node is
+// decided by FP32 forms of it, in coordinates relative to the group's first
+// particle and in units of R, the largest coordinate or sphere bound of the
+// group there: every value that can decide a test is at most 2, its rounding
+// at most 2^-23, and the rounding of d^2 - r^2 below 18 * 2^-24, so a
+// difference beyond kScreen = 2^-19 has the exact test's sign.
+//   1. lanes = nodes: for every eight particles, the sphere about all their
+//      spheres (a node that meets none of these is rejected) and the sphere
+//      of the particle nearest its centre (a node that meets one of these is
+//      accepted).
+//   2. lanes = particles: the nodes still open, one after the other (the
+//      node's box from its lane, the spheres in registers).
+//   3. where no sphere accepts a node and one is too close to tell, the exact
+//      test, lanes = particles, from memory.
+// The gather form, whose masks decide, needs a superset of the leaves within
+// the particles' own radii: there a node is kept if the ball about its centre
+// of mass that holds its particles meets the sphere about some eight (the
+// ball has no margin of h / 2 around the particles, as the box has, and costs
+// fewer operations), and the leaves under kept nodes, 64 at a time in the
+// order they were reached, stay candidates if they lie in such a sphere.
+//
+// Measured: SPH form 551 -> 290 us for 1.5M particles of a collapse, 505 ->
+// 286 for a 1M polytrope, 200 -> 99 for 64^3 (testing each node's own
+// particles in FP64, one after the other, waited for the slowest lane: the
+// one node of 64 that meets many groups of eight and no sphere); gather form
+// 2,560 -> 800 us (1,260 with three scattered coordinate loads per leaf child
+// in place of the queue).  Filtering the SPH form's leaves the same way takes
+// 40% of the masks' work off and costs as much here: 64^3 was slower.
+constexpr int kEight = 8;
+constexpr float kScreen = 1.0f / (1 << 19);
+
+// d^2 - r^2 of the box l .. h and the sphere p (r^2 in p.w)
+__device__ inline float sphere_gap(const float (&l)[3], const float (&h)[3],
+                                   const float4 &p) {
+  const float dx = fmaxf(fmaxf(l[0] - p.x, p.x - h[0]), 0.f),
+              dy = fmaxf(fmaxf(l[1] - p.y, p.y - h[1]), 0.f),
+              dz = fmaxf(fmaxf(l[2] - p.z, p.z - h[2]), 0.f);
+  return __builtin_fmaf(
+      dx, dx, __builtin_fmaf(dy, dy, __builtin_fmaf(dz, dz, -p.w)));
+}
 template <int kStack, int MAXG, bool GF>
 __global__ __launch_bounds__(kW) void k_traverse(TravArgs a) {
 #pragma clang fp contract(off)
-  __shared__ double sx[MAXG], sy[MAXG], sz[MAXG], sh[MAXG];
-  __shared__ double hull[MAXG / kHullChunk][6];
+  __shared__ float4 sph[MAXG];  // x, y, z, r^2 of the screen
+  // of each eight: the sphere about them, the sphere of the one inside
+  __shared__ float4 outer[MAXG / kEight], inner[MAXG / kEight];
+  __shared__ int32_t leaves[GF ? 9 * kW : 1];  // reached, not yet filtered
   __shared__ int32_t stk[kStack];
+  constexpr int NK = MAXG / kW;
   const int lane = threadIdx.x;
   const int64_t gi = xcd_item(blockIdx.x, gridDim.x);
   const int64_t g = a.glist ? a.glist[gi] : gi;
   const int64_t gs = a.gstart[g];
   const int gc = a.gcount[g];
-  const int gn = a.gather ? -1 : a.gnode[g];
-  for (int k = lane; k < gc; k += kW) {
-    sx[k] = a.x[gs + k];
-    sy[k] = a.y[gs + k];
-    sz[k] = a.z[gs + k];
-    sh[k] = !a.gather ? a.h[gs + k]
-            : a.rscale * (a.hprop ? (double)a.hprop[gs + k] : a.h[gs + k]);
-    a.rowrel[gs + k] = make_float4(
-        (float)(sx[k] - a.x[gs]), (float)(sy[k] - a.y[gs]),
-        (float)(sz[k] - a.z[gs]), (float)(sh[k] * sh[k]));
+  const int gn = GF ? -1 : a.gnode[g];
+  auto radius = [&](int64_t p) {
+    return !GF ? a.h[p] : a.rscale * (a.hprop ? (double)a.hprop[p] : a.h[p]);
+  };
+  const double c0 = a.x[gs], c1 = a.y[gs], c2 = a.z[gs];
+  double X[NK][3], rad[NK], R = 0;
+  float4 own[NK];  // this lane's spheres
+#pragma unroll
+  for (int q = 0; q < NK; ++q) {
+    const int k = lane + q * kW;
+    if (k >= gc) continue;
+    X[q][0] = a.x[gs + k];
+    X[q][1] = a.y[gs + k];
+    X[q][2] = a.z[gs + k];
+    rad[q] = radius(gs + k);
+    const double e0 = X[q][0] - c0, e1 = X[q][1] - c1, e2 = X[q][2] - c2;
+    a.rowrel[gs + k] = make_float4((float)e0, (float)e1, (float)e2,
+                                   (float)(rad[q] * rad[q]));
+    R = fmax(R, fmax(fmax(fabs(e0), fabs(e1)), fabs(e2)) + fabs(rad[q]));
+  }
+  for (int o = 32; o > 0; o >>= 1) R = fmax(R, __shfl_xor(R, o, 64));
+  // (outside this range, infinities included, every test is the exact one)
+  const bool scr = R > 1e-150 && R < 1e150 && c0 - c0 + c1 - c1 + c2 - c2 == 0;
+  const double inv = scr ? 1.0 / R : 0.0;
+#pragma unroll
+  for (int q = 0; q < NK; ++q) {
+    const int k = lane + q * kW;
+    // past the group, or with a NaN: a sphere that nothing meets
+    const double nan = k < gc ? X[q][0] + X[q][1] + X[q][2] + rad[q] : NAN;
+    own[q] = nan == nan ? make_float4((float)((X[q][0] - c0) * inv),
+                                      (float)((X[q][1] - c1) * inv),
+                                      (float)((X[q][2] - c2) * inv),
+                                      (float)((rad[q] * inv) * (rad[q] * inv)))
+                        : make_float4(0.f, 0.f, 0.f, -4.f);
+    sph[k] = own[q];
   }
   double gb[6];
   if (gn >= 0) {
     for (int d = 0; d < 6; ++d) gb[d] = a.box[6 * (int64_t)gn + d];
   } else {
     // Without a group node (gather mode, single-particle groups): the box
-    // hull of the group's spheres, widened as the chunk hulls below.  A
-    // node that meets a sphere meets the hull, so testing it first only
-    // saves sphere tests.
+    // hull of the group's spheres, widened by 1e-9 of |centre| + radius,
+    // well beyond the rounding of the sphere test.  A node that meets a
+    // sphere meets the hull, so testing it first only saves sphere tests.
     for (int d = 0; d < 3; ++d) {
       gb[d] = DBL_MAX;
       gb[d + 3] = -DBL_MAX;
     }
-    for (int k = lane; k < gc; k += kW) {
-      const double c[3] = {sx[k], sy[k], sz[k]};
+#pragma unroll
+    for (int q = 0; q < NK; ++q) {
+      if (lane + q * kW >= gc) continue;
       for (int d = 0; d < 3; ++d) {
-        const double r = sh[k] + 1e-9 * (fabs(c[d]) + sh[k]);
-        gb[d] = fmin(gb[d], c[d] - r);
-        gb[d + 3] = fmax(gb[d + 3], c[d] + r);
+        const double r = rad[q] + 1e-9 * (fabs(X[q][d]) + rad[q]);
+        gb[d] = fmin(gb[d], X[q][d] - r);
+        gb[d + 3] = fmax(gb[d + 3], X[q][d] + r);
       }
     }
     for (int o = 32; o > 0; o >>= 1)
@@ -163,46 +214,67 @@ __global__ __launch_bounds__(kW) void k_traverse(TravArgs a) {
         gb[d + 3] = fmax(gb[d + 3], __shfl_xor(gb[d + 3], o, 64));
       }
   }
-  // Leaf filter (gather form): a leaf child of an accepted node becomes a
-  // candidate only if it lies within the hull box of the particles' gather
-  // spheres and within the sphere about the box's centre that holds them
-  // all (both slightly widened), outside of which it fails every particle's
-  // gather predicate (4M collapse: Newton-h phase 20.2 -> 18.0 ms).  The SPH form keeps every leaf: the
-  // same test with the centre-of-mass filter of tree_topology.h:365-371
-  // (which the masks apply) cost the traversal more than it saved.
-  constexpr bool filt = GF;  // (GF: gather form, a.gather set)
-  double fc[3] = {0, 0, 0}, frad = 0;
-  if (filt) {
-    for (int d = 0; d < 3; ++d) fc[d] = 0.5 * (gb[d] + gb[d + 3]);
-    for (int k = lane; k < gc; k += kW) {
-      const double e0 = sx[k] - fc[0], e1 = sy[k] - fc[1], e2 = sz[k] - fc[2];
-      frad = fmax(frad, sqrt(e0 * e0 + e1 * e1 + e2 * e2) + sh[k]);
-    }
-    for (int o = 32; o > 0; o >>= 1) frad = fmax(frad, __shfl_xor(frad, o, 64));
-    frad *= 1.0 + 1e-9;
-  }
   __syncthreads();
-  const int nhull = (gc + kHullChunk - 1) / kHullChunk;
-  if (lane < nhull) {
-    double lo[3] = {DBL_MAX, DBL_MAX, DBL_MAX},
-           hi[3] = {-DBL_MAX, -DBL_MAX, -DBL_MAX};
-    const int k1 = min(gc, (lane + 1) * kHullChunk);
-    for (int k = lane * kHullChunk; k < k1; ++k) {
-      const double c[3] = {sx[k], sy[k], sz[k]};
+  const int n8 = (gc + kEight - 1) / kEight;
+  if (lane >= n8 && lane < MAXG / kEight) {  // (the loops below go in pairs)
+    outer[lane] = make_float4(INFINITY, 0.f, 0.f, 0.f);
+    inner[lane] = make_float4(0.f, 0.f, 0.f, -4.f);
+  }
+  if (lane < n8) {
+    float lo[3] = {INFINITY, INFINITY, INFINITY},
+          hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+    float4 p[kEight];
+#pragma unroll
+    for (int u = 0; u < kEight; ++u) {
+      p[u] = sph[lane * kEight + u];
+      if (p[u].w < 0.f) continue;
+      const float c[3] = {p[u].x, p[u].y, p[u].z};
       for (int d = 0; d < 3; ++d) {
-        const double pad = 1e-9 * (fabs(c[d]) + sh[k]);
-        lo[d] = fmin(lo[d], c[d] - sh[k] - pad);
-        hi[d] = fmax(hi[d], c[d] + sh[k] + pad);
+        lo[d] = fminf(lo[d], c[d]);
+        hi[d] = fmaxf(hi[d], c[d]);
       }
     }
-    for (int d = 0; d < 3; ++d) {
-      hull[lane][d] = lo[d];
-      hull[lane][d + 3] = hi[d];
+    const float m[3] = {0.5f * (lo[0] + hi[0]), 0.5f * (lo[1] + hi[1]),
+                        0.5f * (lo[2] + hi[2])};
+    float far = -1.f, best = INFINITY;
+    float4 in = make_float4(0.f, 0.f, 0.f, -4.f);
+#pragma unroll
+    for (int u = 0; u < kEight; ++u) {
+      if (p[u].w < 0.f) continue;
+      const float e0 = p[u].x - m[0], e1 = p[u].y - m[1], e2 = p[u].z - m[2];
+      const float dd = sqrtf(e0 * e0 + e1 * e1 + e2 * e2);
+      far = fmaxf(far, dd + sqrtf(p[u].w));
+      if (dd < best) {
+        best = dd;
+        in = p[u];
+      }
     }
+    // (|centre| <= 1 and far <= 5: 4 kScreen is many of their roundings, and
+    // of those of the tests below; eight NaNs meet nothing)
+    outer[lane] = far < 0.f ? make_float4(INFINITY, 0.f, 0.f, 0.f)
+                            : make_float4(m[0], m[1], m[2],
+                                          far + 4.f * kScreen);
+    inner[lane] = in;
   }
   if (lane == 0) stk[0] = a.root ? a.root[a.inst[gs]] : 0;  // root
   __syncthreads();
-  int sp = 1;
+  // Whether the ball of radius r about e (normalised) meets the sphere about
+  // some eight.  The margins of the spheres' radii are many roundings of
+  // coordinates and radii up to 5, the factor many of larger ones; a NaN
+  // meets every sphere.
+  auto meets = [&](float e0, float e1, float e2, float r) {
+    bool miss = true;
+    for (int q0 = 0; q0 < n8; q0 += 2)
+#pragma unroll
+      for (int q = q0; q < q0 + 2; ++q) {
+        const float4 o = outer[q];
+        const float f0 = e0 - o.x, f1 = e1 - o.y, f2 = e2 - o.z, s = r + o.w;
+        miss &= __builtin_fmaf(f0, f0, __builtin_fmaf(f1, f1, f2 * f2)) >
+                s * s * (1.f + 4.f * kScreen);
+      }
+    return !miss;
+  };
+  int sp = 1, nl = 0;
   int64_t ncand = 0;
   const int64_t cbase = gi * a.ccap;
   bool overflow = false;
@@ -212,80 +284,155 @@ __global__ __launch_bounds__(kW) void k_traverse(TravArgs a) {
     const int node = lane < nb ? stk[sp + lane] : -1;
     __syncthreads();
     bool acc = false;
+    // the children are loaded with the box or ball (one memory latency per
+    // step; a rejected node's are not used)
     int32_t ch[8];
-    if (node >= 0) {
-      // the children are loaded with the box (one memory latency per step;
-      // a rejected node's are not used)
-      double bx[6];
-      for (int d = 0; d < 6; ++d) bx[d] = a.box[6 * (int64_t)node + d];
-      for (int j = 0; j < 8; ++j) ch[j] = a.child[8 * (int64_t)node + j];
-      if (box_box(bx, gb)) {
-        // the chunks whose hull the node meets, all tested at once (for
-        // independent instructions); then their spheres in order until one
-        // meets the node
-        uint32_t hm = 0;
+    if (GF) {
+      if (node >= 0) {
+        const double *nc = a.com + 3 * (int64_t)node;
+        const int32_t *nch = a.child + 8 * (int64_t)node;
+        const float e0 = (float)((nc[0] - c0) * inv),
+                    e1 = (float)((nc[1] - c1) * inv),
+                    e2 = (float)((nc[2] - c2) * inv);
+        const float r = (float)(a.nrad[node] * inv);
+        for (int j = 0; j < 8; ++j) ch[j] = nch[j];
+        acc = !scr || meets(e0, e1, e2, r);
+      }
+    } else {
+      double bx[6] = {0, 0, 0, 0, 0, 0};
+      bool open = false;
+      if (node >= 0) {
+        const double *nbx = a.box + 6 * (int64_t)node;
+        const int32_t *nch = a.child + 8 * (int64_t)node;
+        for (int d = 0; d < 6; ++d) bx[d] = nbx[d];
+        for (int j = 0; j < 8; ++j) ch[j] = nch[j];
+        open = box_box(bx, gb);
+      }
+      const float l[3] = {(float)((bx[0] - c0) * inv),
+                          (float)((bx[1] - c1) * inv),
+                          (float)((bx[2] - c2) * inv)},
+                  h[3] = {(float)((bx[3] - c0) * inv),
+                          (float)((bx[4] - c1) * inv),
+                          (float)((bx[5] - c2) * inv)};
+      if (scr) {
+        float to = INFINITY, ti = INFINITY;
+        for (int q0 = 0; q0 < n8; q0 += 2)
 #pragma unroll
-        for (int q = 0; q < MAXG / kHullChunk; ++q)
-          if (q < nhull && box_box(bx, hull[q])) hm |= 1u << q;
-        while (hm && !acc) {
-          const int q = __builtin_ctz(hm);
-          hm &= hm - 1;
-          const int k1 = min(gc, (q + 1) * kHullChunk);
-          for (int k = q * kHullChunk; k < k1; ++k)
-            if (sphere_box(bx, sx[k], sy[k], sz[k], sh[k])) {
-              acc = true;
-              break;
-            }
+          for (int q = q0; q < q0 + 2; ++q) {
+            float4 o = outer[q];
+            o.w *= o.w;
+            to = fminf(to, sphere_gap(l, h, o));
+            ti = fminf(ti, sphere_gap(l, h, inner[q]));
+          }
+        acc = open && ti < -kScreen;
+        open = open && !acc && to <= 0.f;
+      }
+      uint64_t todo = __ballot(open);
+      while (todo) {
+        const int u = __builtin_ctzll(todo);
+        todo &= todo - 1;
+        bool in = false, unsure = !scr;
+        if (scr) {
+          float lu[3], hu[3], t = INFINITY;
+#pragma unroll
+          for (int d = 0; d < 3; ++d) {
+            lu[d] = lane_f(l[d], u);
+            hu[d] = lane_f(h[d], u);
+          }
+#pragma unroll
+          for (int q = 0; q < NK; ++q)
+            t = fminf(t, sphere_gap(lu, hu, own[q]));
+          in = t < -kScreen;
+          unsure = t <= kScreen;
         }
+        uint64_t hit = __ballot(in);
+        if (!hit && __ballot(unsure)) {
+          const double *nbx =
+              a.box + 6 * (int64_t)__builtin_amdgcn_readlane(node, u);
+          bool ex = false;
+#pragma unroll
+          for (int q = 0; q < NK; ++q) {
+            const int64_t p = gs + lane + q * kW;
+            if (unsure && lane + q * kW < gc)
+              ex |= sphere_box(nbx, a.x[p], a.y[p], a.z[p], radius(p));
+          }
+          hit = __ballot(ex);
+        }
+        if (lane == u) acc = hit != 0;
       }
     }
     int nnode = 0, nleaf = 0;
-    uint32_t keep = 0;  // leaf children that pass the leaf filter
     if (acc) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         nnode += ch[j] >= 0;
-        if (ch[j] <= -2) {
-          if (!filt) {
-            keep |= 1u << j;
-            continue;
-          }
-          const int64_t p = leaf_of(ch[j]);
-          const double bx = a.x[p], by = a.y[p], bz = a.z[p];
-          // inside the hull box of the gather spheres and the sphere
-          if (bx >= gb[0] && bx <= gb[3] && by >= gb[1] && by <= gb[4] &&
-              bz >= gb[2] && bz <= gb[5] &&
-              within_distance2(bx, by, bz, fc[0], fc[1], fc[2], frad))
-            keep |= 1u << j;
-        }
+        nleaf += ch[j] <= -2;
       }
-      nleaf = __popc(keep);
     }
-    int tn, tl;
-    const int pn = wave_excl_scan(nnode, &tn);
-    const int pl = wave_excl_scan(nleaf, &tl);
+    // both counts are at most 512 over the wavefront: one packed scan
+    const int cnt = nnode | nleaf << 16;
+    const int inc = sched::wave_scan_incl(cnt);
+    const int all = __builtin_amdgcn_readlane(inc, 63);
+    const int tn = all & 0xffff, tl = all >> 16;
     if (sp + tn > kStack) {
       overflow = true;
       if (lane == 0) atomicOr(a.flags, kFlagStack);
       break;
     }
-    if (ncand + tl > a.ccap) {
+    if (!GF && ncand + tl > a.ccap) {
       overflow = true;
       if (lane == 0) atomicOr(a.flags, kFlagCand);
       break;
     }
     if (acc) {
-      int qn = sp + pn;
-      int64_t ql = cbase + ncand + pl;
+      int qn = sp + ((inc - cnt) & 0xffff);
+      int ql = nl + ((inc - cnt) >> 16);
+      int32_t *lp = GF ? leaves : a.cand + cbase + ncand;
+#pragma unroll
       for (int j = 0; j < 8; ++j) {
         if (ch[j] >= 0)
           stk[qn++] = ch[j];
-        else if (keep >> j & 1u)
-          a.cand[ql++] = (int32_t)leaf_of(ch[j]);
+        else if (ch[j] <= -2)
+          lp[ql++] = (int32_t)leaf_of(ch[j]);
       }
     }
     sp += tn;
-    ncand += tl;
+    if (GF)
+      nl += tl;
+    else
+      ncand += tl;
+    __syncthreads();
+    if (!GF) continue;
+    int done = 0;
+    while (nl - done >= kW || (sp == 0 && nl > done)) {
+      const bool on = lane < nl - done;
+      const int64_t p = on ? leaves[done + lane] : gs;
+      const float e0 = (float)((a.x[p] - c0) * inv),
+                  e1 = (float)((a.y[p] - c1) * inv),
+                  e2 = (float)((a.z[p] - c2) * inv);
+      const bool keep = on && (!scr || meets(e0, e1, e2, 0.f));
+      const uint64_t km = __ballot(keep);
+      const int nk = __popcll(km);
+      if (ncand + nk > a.ccap) {
+        overflow = true;
+        break;
+      }
+      if (keep)
+        a.cand[cbase + ncand + __popcll(km & ((1ull << lane) - 1))] =
+            (int32_t)p;
+      ncand += nk;
+      done += kW;
+    }
+    if (overflow) {
+      if (lane == 0) atomicOr(a.flags, kFlagCand);
+      break;
+    }
+    if (done && nl > done) {  // fewer than kW are left: to the front
+      const int32_t v = leaves[min(done + lane, 9 * kW - 1)];
+      __syncthreads();
+      leaves[lane] = v;
+    }
+    nl = max(nl - done, 0);
     __syncthreads();
   }
   if (lane == 0) {  // (an overflowed walk leaves zero candidates)
@@ -664,14 +811,14 @@ int build_tiles(Ctx *c, TileBufs tb, bool gather, double scale,
       FSPH_HIP(c, hipMemsetAsync(c->flags.p, 0, sizeof(int), c->stream));
     TravArgs t{c->f[PF_X].as<double>(), c->f[PF_Y].as<double>(),
                c->f[PF_Z].as<double>(), c->f[PF_H].as<double>(),
-               c->nbox.as<double>(),    c->nchild.as<int32_t>(),
+               c->nbox.as<double>(),    c->ncom.as<double>(),
+               c->nrad.as<double>(),    c->nchild.as<int32_t>(),
                ustart,                  ucount,
                gather ? nullptr : c->gnode.as<int32_t>(),
                tb.cand.as<int32_t>(),
                tb.ccount.as<int32_t>(), tb.ccap,
                c->flags.as<int>(),      scale,
-               gather ? 1 : 0,          hprop,
-               glist,
+               hprop,                   glist,
                c->batch.n_inst ? c->f[PF_INST].as<int32_t>() : nullptr,
                c->batch.n_inst ? c->batch.root.as<int32_t>() : nullptr,
                c->rowrel.as<float4>(),  tb.moff.as<int64_t>()};

@@ -1,0 +1,58 @@
+"""The traversals' FP32 screen: outside its range every node takes the exact
+test, so neighbour lists equal the oracle's at extreme scales; groups of a
+few particles and gather tiles (Newton-h) at several sizes, scales and a
+common offset."""
+import numpy as np
+import pytest
+
+from flecsph_amd import BodySystem, _abi, generators
+
+pytestmark = pytest.mark.gpu
+
+
+def scaled(n, scale, offset, n_ngb):
+    parts, prm = generators.random_box(n, seed=n, h_spread=0.6, n_ngb=n_ngb)
+    for k in ("x", "y", "z"):
+        parts[k] = parts[k] * scale + offset
+    parts["h"] = parts["h"] * scale
+    return parts, prm
+
+
+@pytest.mark.parametrize("scale", [1e-151, 1e-149, 1e149, 1e152])
+@pytest.mark.parametrize("n", [9, 700, 5000])
+def test_lists_at_extreme_scales(oracle_mod, n, scale):
+    parts, prm = scaled(n, scale, 0.0, 20)
+    p = _abi.default_params(**prm)
+    g, o = BodySystem(p), oracle_mod.OracleSystem(p, threads=8)
+    for s in (g, o):
+        s.upload(parts)
+        s.update_iteration()
+    og, ig = g.neighbor_lists()
+    oo, io = o.neighbor_lists()
+    assert np.array_equal(og, oo)
+    io = np.concatenate([np.sort(io[oo[i]:oo[i + 1]]) for i in range(n)])
+    assert np.array_equal(ig, io)
+    o.close()
+    g.close()
+
+
+@pytest.mark.parametrize("n,n_target,scale,offset", [
+    (65, 10, 1.0, 0.0), (1000, 40, 1.0, 0.0), (3000, 40, 1e9, 0.0),
+    (3000, 40, 1.0, 1e4)])
+@pytest.mark.parametrize("tile_rows", [64, 128])
+def test_newton_h_over_gather_tiles(oracle_mod, n, n_target, scale, offset,
+                                    tile_rows):
+    """Both solvers stop within newton_tol * h of the same root."""
+    parts, prm = scaled(n, scale, offset, n_target)
+    prm.update(h_mode=_abi.H_NEWTON, n_target=n_target,
+               precision=_abi.PREC_FP64)
+    p = _abi.default_params(**prm)
+    g, o = BodySystem(p), oracle_mod.OracleSystem(p, threads=8)
+    g._call("set_tuning", tile_rows, 128)
+    for s in (g, o):
+        s.upload(parts)
+        s.update_iteration()
+        s.update_h()
+    assert np.allclose(g.get("h"), o.get("h"), rtol=2e-4, atol=0)
+    o.close()
+    g.close()
