@@ -133,18 +133,22 @@ int do_update_iteration(Ctx *c) {
     PhaseTimer t(c, FSPH_T_BOUNDARY);
     FSPH_TRY(stage_boundary(c));
   }
-  {
-    PhaseTimer t(c, FSPH_T_RANGE_KEYS);
-    FSPH_TRY(stage_range_keys(c));
-  }
-  {
-    PhaseTimer t(c, FSPH_T_SORT);
-    FSPH_TRY(stage_sort(c));
-  }
-  {  // (stage_tree fails on the sort's duplicate-key flag)
+  for (bool again = true; again;) {
+    {
+      PhaseTimer t(c, FSPH_T_RANGE_KEYS);
+      FSPH_TRY(stage_range_keys(c));
+    }
+    {
+      PhaseTimer t(c, FSPH_T_SORT);
+      FSPH_TRY(stage_sort(c));
+    }
+    // (stage_tree reads the flags of duplicate keys and unsorted runs)
     PhaseTimer t(c, FSPH_T_TREE);
-    FSPH_TRY(stage_tree(c));
-    FSPH_TRY(stage_groups(c));
+    FSPH_TRY(stage_tree(c, &again));
+    if (again)
+      FSPH_TRY(stage_begin(c));
+    else
+      FSPH_TRY(stage_groups(c));
   }
   FSPH_TRY(stage_neighbors(c));
   c->have_tree = true;
@@ -558,6 +562,7 @@ struct SetCopy {
 // start at zero are one kernel (1M particles: 3.5 -> 2.4 ms; 32 instances of
 // 1.2M particles, concatenated on the host before: 24 -> 8.2 ms).
 int fsph::upload_sets(Ctx *c, const fsph_particles *sets, int ns) {
+  c->sort_full = false;
   if (!sets) return fsph::fail(c, FSPH_E_ARG, "no particles");
   int64_t n = 0;
   const bool opt[3] = {sets[0].rho != nullptr, sets[0].P != nullptr,

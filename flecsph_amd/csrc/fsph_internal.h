@@ -70,6 +70,7 @@ enum : int {
   kFlagNaN = 8,
   kFlagNeg = 16,
   kFlagScanStall = 32,
+  kFlagLongRun = 64,  // the sort left a long run of equal prefixes unsorted
 };
 
 // Words of ctx->flags (an int array of 16): [0] the error bits above;
@@ -147,6 +148,7 @@ struct Ctx {
   // directly (mail_d is its device address): read after the stream or an
   // event has been waited for, without a copy
   int64_t *mail_h = nullptr, *mail_d = nullptr;
+  bool sort_full = false;  // sort by all key bytes (a long run turned up)
   DBuf lvl;            // tree: nodes per depth, then the level cursors
   // pinned halves that gather the small sets of an upload (on first use)
   char *stage_h = nullptr;
@@ -364,7 +366,8 @@ int stage_boundary(Ctx *c);            // k_keys.hip
 int stage_range_keys(Ctx *c);          // k_keys.hip
 int stage_sort(Ctx *c);                // k_keys.hip
 int permute_particles(Ctx *c, const uint32_t *perm, int64_t n_out);
-int stage_tree(Ctx *c);                // k_tree.hip
+// *again: the keys are not sorted, sort once more (sort_full is set)
+int stage_tree(Ctx *c, bool *again);   // k_tree.hip
 int stage_groups(Ctx *c);              // k_tree.hip
 int stage_neighbors(Ctx *c);           // k_neighbors.hip
 // gather tiles: all b with r_ab < scale * h_a per group particle a, with

@@ -498,7 +498,7 @@ __global__ void k_group_mail(const int64_t *__restrict__ packed,
 
 int group_flags(Ctx *c);  // below
 
-int stage_tree(Ctx *c) {
+int stage_tree(Ctx *c, bool *again) {
   const int64_t n = c->n;
   const uint64_t *k = c->key.as<uint64_t>();
   FSPH_TRY(ensure(c, c->L, (size_t)c->pcap * 4));
@@ -525,6 +525,11 @@ int stage_tree(Ctx *c) {
   FSPH_TRY(read_mail(c));
   if (c->mail_h[1] & kFlagScanStall)
     return fail(c, FSPH_E_HIP, "scan: a tile's look-back did not complete");
+  *again = c->mail_h[1] & kFlagLongRun;
+  if (*again) {
+    c->sort_full = true;
+    return 0;
+  }
   if (c->mail_h[1] & kFlagDupKey)
     return fail(c, FSPH_E_DUPKEY,
                 "two particles share a Morton key (positions closer than "

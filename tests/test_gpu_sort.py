@@ -49,3 +49,54 @@ def test_sorted_keys_of_a_batch(sizes):
         s.close()
         o += n
     b.close()
+
+
+def with_cluster(n, m):
+    """n random particles, m of them on a lattice of neighbouring keys that
+    share the 32 bits by which the sort's passes order them, in random
+    order (at 40,000 and 200 some lie in the next such cell)."""
+    parts, prm = generators.random_box(n, seed=n + m)
+    side = int(np.ceil(m ** (1.0 / 3.0)))
+    q = np.random.default_rng(m).permutation(side ** 3)[:m]
+    for d, k in enumerate(("x", "y", "z")):
+        parts[k][1:2 * m:2] = 0.4 + 2e-6 * (q // side ** d % side)
+    return parts, prm
+
+
+@pytest.mark.parametrize("m", [2, 27, 32, 33, 34, 600])
+@pytest.mark.parametrize("n", [1500, 12288, 12289, 40000])
+def test_runs_of_equal_prefixes(oracle_mod, n, m):
+    parts, prm = with_cluster(n, m)
+    p = _abi.default_params(**prm)
+    g, o = BodySystem(p), oracle_mod.OracleSystem(p, threads=8)
+    for s in (g, o):
+        s.upload(parts)
+        s.update_iteration()
+        s.update_iteration()  # (of sorted particles)
+    for f in ("key", "id", "x", "h"):
+        assert np.array_equal(g.get(f), o.get(f)), f
+    o.close()
+    g.close()
+
+
+@pytest.mark.parametrize("sizes,m", [((1300, 700, 900), 25),
+                                     ((1300, 700, 900), 200),
+                                     ((9000, 7000), 25), ((9000, 7000), 200)])
+def test_runs_of_equal_prefixes_in_a_batch(sizes, m):
+    sets = [with_cluster(n, m) for n in sizes]
+    prm = sets[0][1]
+    b = BatchSystem(_abi.default_params(**prm), len(sizes))
+    b.upload([parts for parts, _ in sets])
+    b.update_iteration()
+    key, ids = b.get("key"), b.get("id")
+    o = 0
+    for parts, _ in sets:
+        n = len(parts["x"])
+        s = BodySystem(_abi.default_params(**prm))
+        s.upload(parts)
+        s.update_iteration()
+        assert np.array_equal(key[o:o + n], s.get("key"))
+        assert np.array_equal(ids[o:o + n], s.get("id"))
+        s.close()
+        o += n
+    b.close()
