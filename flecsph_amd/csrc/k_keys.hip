@@ -229,58 +229,36 @@ __global__ __launch_bounds__(kT) void k_copy_fill(
 // ---------------------------------------------------------------------------
 // Range (bodies_system.h:231-268) and keys (filling_curve.h:503-525)
 // ---------------------------------------------------------------------------
-// Every workgroup reduces its particles to one row of `part`; the last one
-// to finish (ctr counts them) reduces the rows into range and clears ctr.
-__global__ __launch_bounds__(kT) void k_range(
+__global__ __launch_bounds__(kRedThreads) void k_range(
     const double *__restrict__ x, const double *__restrict__ y,
     const double *__restrict__ z, const double *__restrict__ h, int64_t n,
     double *part, int *ctr, double *__restrict__ range) {
 #pragma clang fp contract(off)
-  __shared__ double s[6][kT];
-  __shared__ int last_s;
-  const int t = threadIdx.x;
-  auto reduce = [&]() {
-    __syncthreads();
-    for (int st = kT / 2; st > 0; st >>= 1) {
-      if (t < st)
-        for (int d = 0; d < 3; ++d) {
-          s[d][t] = fmin(s[d][t], s[d][t + st]);
-          s[3 + d][t] = fmax(s[3 + d][t], s[3 + d][t + st]);
-        }
-      __syncthreads();
-    }
+  __shared__ double s[6][kRedThreads / 64];
+  __shared__ int sh;
+  auto op = [](int q, double a, double b) {
+    return q < 3 ? fmin(a, b) : fmax(a, b);
   };
   double v[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
-  const double *X[3] = {x, y, z};
-  for (int64_t i = (int64_t)blockIdx.x * kT + t; i < n;
-       i += (int64_t)gridDim.x * kT) {
-    const double hh = h[i];
+  const int64_t step = (int64_t)gridDim.x * kRedThreads;
+#pragma unroll 4
+  for (int64_t i = (int64_t)blockIdx.x * kRedThreads + threadIdx.x; i < n;
+       i += step) {
+    const double hh = h[i], c[3] = {x[i], y[i], z[i]};
     for (int d = 0; d < 3; ++d) {
-      const double c = X[d][i];
-      v[d] = fmin(v[d], c - hh);
-      v[3 + d] = fmax(v[3 + d], c + hh);
+      v[d] = fmin(v[d], c[d] - hh);
+      v[3 + d] = fmax(v[3 + d], c[d] + hh);
     }
   }
-  for (int d = 0; d < 6; ++d) s[d][t] = v[d];
-  reduce();
-  if (t < 6) st_agent(part + blockIdx.x * 6 + t, s[t][0]);
-  __threadfence();
-  __syncthreads();
-  if (t == 0) last_s = atomicAdd(ctr, 1) == (int)gridDim.x - 1;
-  __syncthreads();
-  if (!last_s) return;
-  __threadfence();
-  for (int d = 0; d < 6; ++d) {
-    double w = d < 3 ? INFINITY : -INFINITY;
-    for (int b = t; b < (int)gridDim.x; b += kT) {
-      const double q = ld_agent(part + b * 6 + d);
-      w = d < 3 ? fmin(w, q) : fmax(w, q);
-    }
-    s[d][t] = w;
-  }
-  reduce();
-  if (t < 6) range[t] = s[t][0];
-  if (t == 0) *ctr = 0;
+  block_reduce(v, s, op);
+  if (!last_block(v, part, ctr, &sh)) return;
+#pragma unroll
+  for (int q = 0; q < 6; ++q)
+    v[q] = threadIdx.x < gridDim.x ? ld_agent(part + threadIdx.x * 6 + q)
+                                   : (q < 3 ? INFINITY : -INFINITY);
+  block_reduce(v, s, op);
+  if (threadIdx.x == 0)
+    for (int q = 0; q < 6; ++q) range[q] = v[q];
 }
 
 // range: lo[3], hi[3] (one simulation) or 8 doubles per instance
@@ -864,10 +842,10 @@ int stage_range_keys(Ctx *c) {
         c->val.as<uint32_t>());
     return hip_check(c, hipGetLastError(), "k_keys");
   }
-  const int nb = (int)std::min<int64_t>(1024, (n + kT - 1) / kT);
+  const int nb = red_grid(n);
   FSPH_TRY(ensure(c, c->red_tmp, (size_t)nb * 6 * sizeof(double)));
   FSPH_TRY(ensure(c, c->range_d, 6 * sizeof(double)));
-  k_range<<<nb, kT, 0, c->stream>>>(
+  k_range<<<nb, kRedThreads, 0, c->stream>>>(
       c->f[PF_X].as<double>(), c->f[PF_Y].as<double>(),
       c->f[PF_Z].as<double>(), c->f[PF_H].as<double>(), n,
       c->red_tmp.as<double>(), c->flags.as<int>() + kRangeCtr,

@@ -226,43 +226,26 @@ template <class T> struct TailArgs {
 };
 
 template <class T>
-__global__ __launch_bounds__(kT) void k_tail(TailArgs<T> a, int64_t n) {
-  __shared__ double s[kT];
-  __shared__ int last_s;
-  const int t = threadIdx.x;
+__global__ __launch_bounds__(kRedThreads) void k_tail(TailArgs<T> a,
+                                                      int64_t n) {
+  __shared__ double s[1][kRedThreads / 64];
+  __shared__ int sh;
+  auto op = [](int, double p, double q) { return smin(p, q); };
   const double dt = a.ts[0];
-  double dmin = 1e24;
-  for (int64_t i = (int64_t)blockIdx.x * kT + t; i < n;
-       i += (int64_t)gridDim.x * kT) {
+  double v[1] = {1e24};
+  for (int64_t i = (int64_t)blockIdx.x * kRedThreads + threadIdx.x; i < n;
+       i += (int64_t)gridDim.x * kRedThreads) {
     if (a.what) integrate_one(a.ia, i, a.what, dt);
     if (a.do_h) update_h_one(a.ha, i);
     if (a.do_check) check_one(a.ca, i);
-    dmin = smin(dmin, particle_dt(a.da, i));
+    v[0] = smin(v[0], particle_dt(a.da, i));
   }
-  auto reduce = [&](double v) {
-    s[t] = v;
-    __syncthreads();
-    for (int st = kT / 2; st > 0; st >>= 1) {
-      if (t < st) s[t] = smin(s[t], s[t + st]);
-      __syncthreads();
-    }
-    return s[0];
-  };
-  const double row = reduce(dmin);
-  if (t == 0) {
-    st_agent(a.part + blockIdx.x, row);
-    __threadfence();
-    last_s = atomicAdd(a.flags + kDtCtr, 1) == (int)gridDim.x - 1;
-  }
-  __syncthreads();
-  if (!last_s) return;
-  __threadfence();
-  double v = 1e24;
-  for (int b = t; b < (int)gridDim.x; b += kT) v = smin(v, ld_agent(a.part + b));
-  const double m = reduce(v);
-  if (t != 0) return;
-  a.flags[kDtCtr] = 0;
-  dt_rule_device(m, a.ts);
+  block_reduce(v, s, op);
+  if (!last_block(v, a.part, a.flags + kDtCtr, &sh)) return;
+  v[0] = threadIdx.x < gridDim.x ? ld_agent(a.part + threadIdx.x) : 1e24;
+  block_reduce(v, s, op);
+  if (threadIdx.x != 0) return;
+  dt_rule_device(v[0], a.ts);
   if (a.end) {
     a.ts[1] = a.ts[2];
     step_mail(a.flags, a.mail);
@@ -270,44 +253,23 @@ __global__ __launch_bounds__(kT) void k_tail(TailArgs<T> a, int64_t n) {
 }
 
 // max of v and 2.5 times it (getSmoothinglength's halo) into out[0], out[1]
-__global__ __launch_bounds__(kT) void k_max(const double *v, int64_t n,
-                                            double *part, int *ctr,
-                                            double *out) {
-  __shared__ double s[kT];
-  __shared__ int last_s;
-  const int t = threadIdx.x;
-  auto reduce = [&](double x) {
-    s[t] = x;
-    __syncthreads();
-    for (int st = kT / 2; st > 0; st >>= 1) {
-      if (t < st && s[t] < s[t + st]) s[t] = s[t + st];
-      __syncthreads();
-    }
-    return s[0];
-  };
-  double mx = 0;
-  for (int64_t i = (int64_t)blockIdx.x * kT + t; i < n;
-       i += (int64_t)gridDim.x * kT)
-    mx = (mx < v[i]) ? v[i] : mx;
-  const double row = reduce(mx);
-  if (t == 0) {
-    st_agent(part + blockIdx.x, row);
-    __threadfence();
-    last_s = atomicAdd(ctr, 1) == (int)gridDim.x - 1;
-  }
-  __syncthreads();
-  if (!last_s) return;
-  __threadfence();
-  mx = 0;
-  for (int b = t; b < (int)gridDim.x; b += kT) {
-    const double q = ld_agent(part + b);
-    mx = (mx < q) ? q : mx;
-  }
-  const double m = reduce(mx);
-  if (t == 0) {
-    *ctr = 0;
-    out[0] = m;
-    out[1] = 2.5 * m;
+__global__ __launch_bounds__(kRedThreads) void k_max(const double *v,
+                                                     int64_t n, double *part,
+                                                     int *ctr, double *out) {
+  __shared__ double s[1][kRedThreads / 64];
+  __shared__ int sh;
+  auto op = [](int, double a, double b) { return (a < b) ? b : a; };
+  double m[1] = {0};
+  for (int64_t i = (int64_t)blockIdx.x * kRedThreads + threadIdx.x; i < n;
+       i += (int64_t)gridDim.x * kRedThreads)
+    m[0] = op(0, m[0], v[i]);
+  block_reduce(m, s, op);
+  if (!last_block(m, part, ctr, &sh)) return;
+  m[0] = threadIdx.x < gridDim.x ? ld_agent(part + threadIdx.x) : 0.0;
+  block_reduce(m, s, op);
+  if (threadIdx.x == 0) {
+    out[0] = m[0];
+    out[1] = 2.5 * m[0];
   }
 }
 
@@ -609,7 +571,7 @@ template <class T> int integrate_impl(Ctx *c, uint32_t what) {
 // The time-step rule; `end`: as the end of a step, after the kick `what`,
 // the closed-form h and the state check.
 template <class T> int tail_impl(Ctx *c, bool end, uint32_t what) {
-  const int nb = (int)std::min<int64_t>(1024, (c->n + kT - 1) / kT);
+  const int nb = red_grid(c->n);
   FSPH_TRY(ensure(c, c->red_tmp, (size_t)nb * 8));
   TailArgs<T> a{};
   a.ia = int_args<T>(c);
@@ -624,7 +586,7 @@ template <class T> int tail_impl(Ctx *c, bool end, uint32_t what) {
   a.ts = c->tstate.as<double>();
   a.flags = c->flags.as<int>();
   a.mail = c->mail_d;
-  k_tail<T><<<nb, kT, 0, c->stream>>>(a, c->n);
+  k_tail<T><<<nb, kRedThreads, 0, c->stream>>>(a, c->n);
   c->time_dirty = true;
   return hip_check(c, hipGetLastError(), "k_tail");
 }
@@ -983,10 +945,10 @@ int stage_reductions(Ctx *c, double out[10]) {
 }
 
 int stage_halo(Ctx *c, const double **halo) {
-  const int nb = (int)std::min<int64_t>(1024, (c->n + kT - 1) / kT);
+  const int nb = red_grid(c->n);
   FSPH_TRY(ensure(c, c->red_tmp, (size_t)(nb + 2) * 8));
   double *part = c->red_tmp.as<double>();
-  k_max<<<nb, kT, 0, c->stream>>>(c->f[PF_H].as<double>(), c->n, part,
+  k_max<<<nb, kRedThreads, 0, c->stream>>>(c->f[PF_H].as<double>(), c->n, part,
                                   c->flags.as<int>() + kMaxCtr, part + nb);
   *halo = part + nb + 1;
   return hip_check(c, hipGetLastError(), "k_max");
