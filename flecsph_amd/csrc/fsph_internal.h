@@ -301,8 +301,8 @@ struct Ctx {
 
   // Graph mode (batched contexts, closed-form h, no gravity): the sync-free
   // tail of a step (pair passes, kicks, h, per-instance dt minimum) is
-  // captured once as a hipGraph of persistent kernels that read their
-  // arguments and sizes from device memory, and replayed every step.
+  // captured once as a hipGraph, and replayed every step with the kernels'
+  // arguments and grids set to the step's.
   struct Graph {
     bool on = false;
     hipGraph_t graph = nullptr;
