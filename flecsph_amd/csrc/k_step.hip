@@ -494,7 +494,7 @@ __global__ __launch_bounds__(kT) void k_seg_roots(
   if (i < ni) root[i] = (int32_t)off[seg[i]];  // the depth-0 node of pair seg[i]
 }
 
-// ---- graph mode: persistent (grid-stride) forms reading device arguments --
+// ---- graph mode: grid-stride forms, arguments set per replay --
 template <class T> struct StepSlot {
   IntArgs<T> ia;
   DtArgs<T> da;

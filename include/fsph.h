@@ -524,7 +524,7 @@ int fsph_instance_time(const fsph_ctx *ctx, int inst, int64_t *iteration,
 /* Graph mode of a batched context (new): the sync-free tail of every step
    after the neighbour tiles (density, signal speed, acceleration, kick v,
    du/dt, kick u, closed-form h, per-instance dt minimum) runs as one
-   replayed hipGraph of persistent kernels.  Needs h_mode FSPH_H_CLOSED,
+   replayed hipGraph.  Needs h_mode FSPH_H_CLOSED,
    no gravity and the constant viscosity; results are those of the eager
    path. */
 int fsph_enable_graph(fsph_ctx *ctx, int on);
