@@ -540,7 +540,9 @@ __device__ int write_lane(int v, int lane, int old)
 // tau = 2^-17 max(R^2, h^2) the sign of u decides, and a round of rows with
 // a u inside it (or not a number; about one in a hundred rounds) is tested
 // over in FP64 with the reference's operations.  A tau too small to be
-// normal counts as infinite: everything is then tested in FP64.
+// normal counts as infinite: everything is then tested in FP64.  So it is
+// from 2^107 on, where tau becomes not a number: d^2 (at most 12 R^2) or h^2
+// may overflow there, and an infinite u says nothing of the exact one's sign.
 // d <= max(h_k, h_b)^2 is tested there as d <= h_k^2 or d <= h_b^2: squaring
 // and rounding are monotone, so the outcome is the same.
 //
@@ -654,7 +656,8 @@ __global__ __launch_bounds__(kW) void k_masks(MaskArgs a) {
       const float m = fmaxf(fmaxf(fabsf((float)(cx - ox)), fabsf(fy)),
                             fabsf(fz));
       const float t2 = 0x1p-17f * fmaxf(scale2, fmaxf(m * m, fh2));
-      if (t2 > 0x1p-100f) tau = t2;
+      // (0 for a finite product, else not a number)
+      if (t2 > 0x1p-100f) tau = __builtin_fmaf(t2 * 0x1p21f, 0.f, t2);
     }
     const uint64_t far = __ballot(!on);
     fetch(cnext);

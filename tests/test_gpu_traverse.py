@@ -36,6 +36,45 @@ def test_lists_at_extreme_scales(oracle_mod, n, scale):
     g.close()
 
 
+def test_lists_where_fp32_squares_overflow(oracle_mod):
+    """h^2 just below the largest FP32 number; two rows of particles far
+    from the tile's first one, each a little closer than h to its partner in
+    the other row, where rounding to FP32 takes every such pair beyond h: the
+    squared distance is infinite there, h^2 is not."""
+    rng = np.random.default_rng(3)
+    f32 = np.float32
+    far, h = 1e23, float(np.sqrt(np.finfo(f32).max)) * (1 - 1e-6)
+    m = 60
+    rows = []
+    while len(rows) < m:
+        y0 = 0.5 * far - h * rng.uniform(0.1, 0.9)
+        y1 = y0 + h * (1 - 1e-5)
+        with np.errstate(over="ignore"):
+            if np.isinf((f32(y1) - f32(y0)) * (f32(y1) - f32(y0))):
+                rows.append((y0, y1))
+    rows = np.array(rows)
+    x = np.linspace(0.0, far, m)
+    x = np.concatenate([[0.0, far], x, x])
+    y = np.concatenate([[0.0, far], rows[:, 0], rows[:, 1]])
+    n = x.size
+    z = np.zeros(n)
+    parts = dict(x=x, y=y, z=z, vx=z, vy=z, vz=z, u=z + 1, m=z + 1,
+                 h=z + h, id=np.arange(n))
+    p = _abi.default_params()
+    g, o = BodySystem(p), oracle_mod.OracleSystem(p, threads=8)
+    for s in (g, o):
+        s.upload(parts)
+        s.update_iteration()
+    og, ig = g.neighbor_lists()
+    oo, io = o.neighbor_lists()
+    assert oo[n] == n + 2 * m
+    assert np.array_equal(og, oo)
+    io = np.concatenate([np.sort(io[oo[i]:oo[i + 1]]) for i in range(n)])
+    assert np.array_equal(ig, io)
+    o.close()
+    g.close()
+
+
 @pytest.mark.parametrize("n,n_target,scale,offset", [
     (65, 10, 1.0, 0.0), (1000, 40, 1.0, 0.0), (3000, 40, 1e9, 0.0),
     (3000, 40, 1.0, 1e4)])
