@@ -45,6 +45,7 @@ def build(verbose=False):
         raise RuntimeError(f"link failed:\n{r.stderr[-6000:]}")
     os.replace(tmp, OUT)
     build_driver()
+    build_probe()
     if verbose:
         print(f"built {OUT} and {DRIVER}")
     return OUT
@@ -52,6 +53,7 @@ def build(verbose=False):
 
 DRIVER = os.path.join(HERE, "fsph_hydro_driver")
 FUNCTOR_CHECK = os.path.join(HERE, "fsph_functor_check")
+PROBE = os.path.join(HERE, "libfsph_probe.so")
 
 
 def build_driver():
@@ -68,6 +70,17 @@ def build_driver():
         if r.returncode != 0:
             raise RuntimeError(f"{src} build failed:\n{r.stderr[-4000:]}")
     return DRIVER
+
+
+def build_probe():
+    """The tests' view into a context (host code over the internal header)."""
+    cmd = [HIPCC, *FLAGS, "-shared", os.path.join(HERE, "host",
+                                                  "ctx_probe.cpp"),
+           "-o", PROBE]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"ctx_probe.cpp build failed:\n{r.stderr[-4000:]}")
+    return PROBE
 
 
 if __name__ == "__main__":

@@ -117,6 +117,10 @@ struct TravArgs {
 // ball has no margin of h / 2 around the particles, as the box has, and costs
 // fewer operations), and the leaves under kept nodes, 64 at a time in the
 // order they were reached, stay candidates if they lie in such a sphere.
+// Where the screen is off (a position that is not a number or infinite in the
+// unit's first particle, or a scale beyond FP32's reach), its nodes take the
+// exact box test and the leaves under them all stay, so that a particle whose
+// position is not a number still meets nothing.
 //
 // Measured: SPH form 551 -> 290 us for 1.5M particles of a collapse, 505 ->
 // 286 for a 1M polytrope, 200 -> 99 for 64^3 (testing each node's own
@@ -296,7 +300,13 @@ __global__ __launch_bounds__(kW) void k_traverse(TravArgs a) {
                     e2 = (float)((nc[2] - c2) * inv);
         const float r = (float)(a.nrad[node] * inv);
         for (int j = 0; j < 8; ++j) ch[j] = nch[j];
-        acc = !scr || meets(e0, e1, e2, r);
+        if (scr) {
+          acc = meets(e0, e1, e2, r);
+        } else {
+          for (int64_t p = gs; p < gs + gc && !acc; ++p)
+            acc = sphere_box(a.box + 6 * (int64_t)node, a.x[p], a.y[p],
+                             a.z[p], radius(p));
+        }
       }
     } else {
       double bx[6] = {0, 0, 0, 0, 0, 0};

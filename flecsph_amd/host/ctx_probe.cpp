@@ -1,0 +1,17 @@
+// ctx_probe.cpp -- state of a context that the C ABI does not show, for the
+// tests (libfsph_probe.so, built beside libfsph.so from the same header).
+#include "fsph_internal.h"
+
+using fsph::Ctx;
+
+extern "C" {
+
+// Candidate capacity and stack tier of the gather tiles.
+int64_t fsph_probe_gather(const fsph_ctx *ctx, int64_t out[2]) {
+  const Ctx *c = reinterpret_cast<const Ctx *>(ctx);
+  out[0] = c->gccap;
+  out[1] = c->stack_tier[1];
+  return 0;
+}
+
+}  // extern "C"

@@ -1,6 +1,9 @@
 """State checks (check_nans, check_negativity, default_physics.h:918-979):
 the driver's step returns FSPH_E_NAN / FSPH_E_NEG as the reference's
 asserts would stop the run, and the oracle agrees on the same input."""
+import ctypes as C
+import os
+
 import numpy as np
 import pytest
 
@@ -86,4 +89,47 @@ def test_a_drift_needs_a_new_tree_before_the_neighbour_passes():
     g.update_iteration()
     g.density_eos()
     g.update_h()
+    g.close()
+
+
+def _probe(name, g, *args):
+    """A function of libfsph_probe.so (flecsph_amd/host/ctx_probe.cpp) on
+    g's context."""
+    lib = C.CDLL(os.path.join(os.path.dirname(_abi.__file__),
+                              "libfsph_probe.so"))
+    fn = getattr(lib, "fsph_probe_" + name)
+    fn.restype = C.c_int64
+    return fn(g._h, *args)
+
+
+@pytest.mark.parametrize("n", [5000, 280_001])
+def test_nan_position_under_newton_h_is_reported(n):
+    """A particle whose position is not a number (its key is the lowest, so
+    it is the first of a tile) meets nothing: the solver's gather tiles stay
+    as small as without it, the step reports the NaN, and the context works
+    after an upload of sound data."""
+    parts, prm = generators.random_box(n, seed=5, h_spread=0.3)
+    prm.update(h_mode=_abi.H_NEWTON, n_target=40)
+    bad = dict(parts)
+    for k in ("x", "y", "z"):
+        bad[k] = parts[k].copy()
+        bad[k][n // 2] = np.nan
+    sizes = []
+    for p in (parts, bad):
+        g = BodySystem(_abi.default_params(**prm))
+        g.upload(p)
+        if p is bad:
+            print("one particle of", n, "without a position", flush=True)
+            with pytest.raises(FsphError) as e:
+                g.step()
+            assert e.value.code == _abi.FSPH_E_NAN
+        else:
+            g.step()
+        sizes.append((C.c_int64 * 2)())
+        _probe("gather", g, sizes[-1])
+    assert list(sizes[1]) == list(sizes[0])
+    g.upload(parts)
+    g.step()
+    h = g.get("h")
+    assert np.all(np.isfinite(h)) and np.all(h > 0)
     g.close()

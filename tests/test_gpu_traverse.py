@@ -1,7 +1,7 @@
 """The traversals' FP32 screen: outside its range every node takes the exact
 test, so neighbour lists equal the oracle's at extreme scales; groups of a
-few particles and gather tiles (Newton-h) at several sizes, scales and a
-common offset."""
+few particles and gather tiles (Newton-h) at several sizes, scales, a common
+offset and with a position that is not a number."""
 import numpy as np
 import pytest
 
@@ -75,6 +75,13 @@ def test_lists_where_fp32_squares_overflow(oracle_mod):
     g.close()
 
 
+def within_h(g):
+    """#{b : r < h} of every particle at the context's own h, by all pairs."""
+    x, y, z, h = (g.get(f) for f in ("x", "y", "z", "h"))
+    d2 = (x[:, None] - x) ** 2 + (y[:, None] - y) ** 2 + (z[:, None] - z) ** 2
+    return (d2 < (h * h)[:, None]).sum(axis=1)
+
+
 @pytest.mark.parametrize("n,n_target,scale,offset", [
     (65, 10, 1.0, 0.0), (1000, 40, 1.0, 0.0), (3000, 40, 1e9, 0.0),
     (3000, 40, 1.0, 1e4)])
@@ -94,4 +101,25 @@ def test_newton_h_over_gather_tiles(oracle_mod, n, n_target, scale, offset,
         s.update_h()
     assert np.allclose(g.get("h"), o.get("h"), rtol=2e-4, atol=0)
     o.close()
+    g.close()
+
+
+@pytest.mark.parametrize("tile_rows", [64, 128])
+def test_gather_tile_of_a_nan_position(tile_rows):
+    """A tile whose first particle has no position takes the exact test: its
+    other particles find their neighbours, that one finds none."""
+    n = 3000
+    parts, prm = scaled(n, 1.0, 0.0, 40)
+    prm.update(h_mode=_abi.H_NEWTON, n_target=40)
+    for k in ("x", "y", "z"):
+        parts[k][7] = np.nan
+    g = BodySystem(_abi.default_params(**prm))
+    g._call("set_tuning", tile_rows, 128)
+    g.upload(parts)
+    g.update_iteration()
+    assert g.get("id")[0] == 7  # (the lowest key)
+    g.update_h()
+    ok = np.arange(n) != 0
+    assert np.array_equal(g.get("hngb")[ok], within_h(g)[ok])
+    assert g.get("hngb")[0] == 0
     g.close()
