@@ -93,6 +93,14 @@ __global__ __launch_bounds__(64) void k_begin(int *flags,
   if (t < kMaxDepth + 2) lvl[t] = 0;
 }
 
+// The state check's two words only: a stalled scan stays on record.
+__global__ void k_check_begin(int *flags) {
+  if (threadIdx.x == 0) {
+    flags[kCheckWord] = 0;
+    flags[kCheckWord + 1] = kCheckNone;
+  }
+}
+
 __global__ void k_advance(double *ts, int adaptive) {
 #pragma clang fp contract(off)
   if (threadIdx.x == 0) ts[1] = adaptive ? ts[2] : ts[1] + ts[0];
@@ -711,7 +719,7 @@ template <class T> CheckArgs<T> check_args(Ctx *c) {
 
 int stage_check_state(Ctx *c, bool reset) {
   if (c->n <= 0) return 0;
-  if (reset) FSPH_TRY(stage_begin(c));
+  if (reset) k_check_begin<<<1, 64, 0, c->stream>>>(c->flags.as<int>());
   if (c->rsize == 4)
     k_check_state<float><<<blocks_for(c->n), kT, 0, c->stream>>>(
         check_args<float>(c), c->n);

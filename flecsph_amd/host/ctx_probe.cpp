@@ -14,4 +14,13 @@ int64_t fsph_probe_gather(const fsph_ctx *ctx, int64_t out[2]) {
   return 0;
 }
 
+// Whether a scan's stall is on record; set: records one first.
+int64_t fsph_probe_scan_stall(const fsph_ctx *ctx, int set) {
+  const Ctx *c = reinterpret_cast<const Ctx *>(ctx);
+  int *word = c->flags.as<int>() + fsph::kScanWord, v = fsph::kFlagScanStall;
+  if (set && hipMemcpy(word, &v, sizeof(v), hipMemcpyHostToDevice)) return -1;
+  if (hipMemcpy(&v, word, sizeof(v), hipMemcpyDeviceToHost)) return -1;
+  return v == fsph::kFlagScanStall;
+}
+
 }  // extern "C"

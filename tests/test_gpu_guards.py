@@ -133,3 +133,24 @@ def test_nan_position_under_newton_h_is_reported(n):
     h = g.get("h")
     assert np.all(np.isfinite(h)) and np.all(h > 0)
     g.close()
+
+
+def test_check_state_keeps_an_unread_scan_stall():
+    """A stalled scan whose result nothing has read yet stays on record
+    through a state check, until the next update_iteration: the next call
+    that needs a scan fails."""
+    parts, prm = _case()
+    g = BodySystem(_abi.default_params(**prm))
+    g.upload(parts)
+    g.step()
+    assert _probe("scan_stall", g, 1) == 1
+    g.check_state()
+    assert _probe("scan_stall", g, 0) == 1
+    with pytest.raises(FsphError) as e:
+        g.neighbor_lists()
+    assert e.value.code == _abi.FSPH_E_HIP
+    g.update_iteration()
+    assert _probe("scan_stall", g, 0) == 0
+    g.neighbor_lists()
+    g.check_state()
+    g.close()
