@@ -579,9 +579,10 @@ int fsph::upload_sets(Ctx *c, const fsph_particles *sets, int ns) {
   const bool per = c->p.periodic[0] || c->p.periodic[1] || c->p.periodic[2];
   FSPH_TRY(fsph::ensure_particles(c, per ? (int64_t)(n * 2.2) + 4096 : n,
                                   false));
-  // rho, P, c as given (double), converted on the device
-  FSPH_TRY(fsph::ensure(c, c->red_tmp, (size_t)n * 3 * 8));
-  double *tmp = c->red_tmp.as<double>();
+  // rho, P, c as given (double), converted on the device; they wait in the
+  // permutation's targets
+  double *given[3] = {c->g[PF_X].as<double>(), c->g[PF_Y].as<double>(),
+                      c->g[PF_Z].as<double>()};
   auto field = [&](void *dst, auto get) {
     SetCopy sc(c, dst, ns > 1);
     for (int i = 0; i < ns; ++i)
@@ -599,12 +600,12 @@ int fsph::upload_sets(Ctx *c, const fsph_particles *sets, int ns) {
   FSPH_TRY(field(c->f[PF_H].p, [](Q q) { return q.h; }));
   FSPH_TRY(field(c->f[PF_M].p, [](Q q) { return q.m; }));
   FSPH_TRY(field(c->f[PF_ID].p, [](Q q) { return q.id; }));
-  if (opt[0]) FSPH_TRY(field(tmp, [](Q q) { return q.rho; }));
-  if (opt[1]) FSPH_TRY(field(tmp + n, [](Q q) { return q.P; }));
-  if (opt[2]) FSPH_TRY(field(tmp + 2 * n, [](Q q) { return q.c; }));
-  FSPH_TRY(stage_upload_init(c, n, opt[0] ? tmp : nullptr,
-                             opt[1] ? tmp + n : nullptr,
-                             opt[2] ? tmp + 2 * n : nullptr));
+  if (opt[0]) FSPH_TRY(field(given[0], [](Q q) { return q.rho; }));
+  if (opt[1]) FSPH_TRY(field(given[1], [](Q q) { return q.P; }));
+  if (opt[2]) FSPH_TRY(field(given[2], [](Q q) { return q.c; }));
+  FSPH_TRY(stage_upload_init(c, n, opt[0] ? given[0] : nullptr,
+                             opt[1] ? given[1] : nullptr,
+                             opt[2] ? given[2] : nullptr));
   c->have_rhoP = opt[0] && opt[1];
   c->n = c->n_real = n;
   c->have_tree = false;

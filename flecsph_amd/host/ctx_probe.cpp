@@ -23,4 +23,9 @@ int64_t fsph_probe_scan_stall(const fsph_ctx *ctx, int set) {
   return v == fsph::kFlagScanStall;
 }
 
+// Bytes of the scratch buffer that the reductions share.
+int64_t fsph_probe_scratch_bytes(const fsph_ctx *ctx) {
+  return (int64_t) reinterpret_cast<const Ctx *>(ctx)->red_tmp.bytes;
+}
+
 }  // extern "C"

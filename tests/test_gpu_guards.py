@@ -154,3 +154,19 @@ def test_check_state_keeps_an_unread_scan_stall():
     g.neighbor_lists()
     g.check_state()
     g.close()
+
+
+def test_upload_needs_no_memory_beyond_the_fields():
+    """rho, P and c are converted through the fields' own scratch."""
+    parts, prm = _case()
+    for given in ((), ("rho", "P", "c")):
+        q = dict(parts)
+        for k in ("rho", "P", "c"):
+            q[k] = np.linspace(1.0, 2.0, len(q["x"])) if k in given else None
+        g = BodySystem(_abi.default_params(**prm))
+        g.upload(q)
+        assert _probe("scratch_bytes", g) == 0
+        for k in ("rho", "P", "c"):
+            want = q[k] if k in given else np.zeros(len(q["x"]))
+            assert np.array_equal(g.get(k), want.astype(np.float32))
+        g.close()
