@@ -227,7 +227,8 @@ int do_update_h(Ctx *c) {
 int do_step(Ctx *c) {
   c->ev_used = 0;
   uint32_t tail_kick = 0;  // energy kick left to the fused end of the step
-  const bool fused = !c->batch.n_inst && c->p.adaptive_dt;
+  // (with the phase timers on, every phase is launched and timed by itself)
+  const bool fused = !c->batch.n_inst && c->p.adaptive_dt && !c->timing;
   const bool closed = c->p.h_mode == FSPH_H_CLOSED;
   if (!c->initial_done) {
     // hydro/main_driver.cc:102-173 (iteration 0: no integration)

@@ -468,9 +468,7 @@ enum fsph_timer {
   FSPH_T_GRAVITY,       /* self-gravity                                  */
   FSPH_T_DUDT,          /* du/dt + P, c at the half step (1 kernel)      */
   FSPH_T_H,             /* smoothing-length update                       */
-  FSPH_T_DT,            /* time-step reduction; in a single simulation's
-                           step with an adaptive time step also its
-                           last energy kick, closed-form h and check     */
+  FSPH_T_DT,            /* time-step reduction                           */
   FSPH_T_GRAPH,         /* graph replay of a batched step's tail (pair
                            passes, kicks, h, dt minimum)                 */
   FSPH_T_GRAV_PAIRS,    /* FMM interaction lists: dual-tree pair levels

@@ -170,3 +170,27 @@ def test_upload_needs_no_memory_beyond_the_fields():
             want = q[k] if k in given else np.zeros(len(q["x"]))
             assert np.array_equal(g.get(k), want.astype(np.float32))
         g.close()
+
+
+@pytest.mark.parametrize("thermokinetic", [0, 1])
+def test_phase_times_are_the_phases_own(thermokinetic):
+    """With the timers on, each phase of a single simulation's step is timed
+    by itself (the smoothing-length update is no part of the time step's),
+    and the state is that of a step without timers."""
+    parts, prm = _case()
+    prm.update(thermokinetic=thermokinetic)
+    runs = []
+    for timed in (False, True):
+        g = BodySystem(_abi.default_params(**prm))
+        g.upload(parts)
+        g.enable_timing(timed)
+        for _ in range(3):
+            g.step()
+            if timed:
+                t = g.phase_times()
+                assert t["h"] > 0 and t["dt"] > 0 and t["integrate"] > 0
+        runs.append([g.get(f) for f in ("x", "vx", "u", "e", "h", "rho")] +
+                    [np.array(g.time())])
+        g.close()
+    for a, b in zip(*runs):
+        assert np.array_equal(a, b)
