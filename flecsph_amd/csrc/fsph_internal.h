@@ -123,6 +123,7 @@ enum : int {
   kFlagNeg = 16,
   kFlagScanStall = 32,
   kFlagLongRun = 64,  // the sort left a long run of equal prefixes unsorted
+  kFlagFullSort = 128,  // the sort met a long run and took all key bits
 };
 
 // Words of ctx->flags (an int array of 16): [0] the error bits above;

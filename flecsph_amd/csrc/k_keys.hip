@@ -299,8 +299,9 @@ __global__ __launch_bounds__(kT) void k_keys(
 // the tree and two thirds of the next, by which nearly all keys differ; runs
 // of equal prefixes of up to kRunMax keys are then sorted in place by one
 // thread each.  Where a longer run turns up, all 64 bits are sorted instead
-// (in the same launch or, in the second form, by sorting again, which the
-// context keeps doing until the next upload).  With all eight passes 2,000
+// (in the same launch or, in the second form, by sorting again), and the
+// context does so at once from then on until the next upload.  With all
+// eight passes 2,000
 // keys took 33 us, 10,007 91, 38,880 141 and 474,552 181; now 23, 55, 78 and
 // 111 (with the permutation).
 // One of two forms by the number of keys:
@@ -589,10 +590,11 @@ __global__ __launch_bounds__(kT) void k_radix_scatter(
 
 // All passes for up to 1024 ITEMS keys in one workgroup: the ranking of
 // k_radix_scatter over 16 wavefronts, the entries reordered in LDS.
+// all: by all the key's bytes from the start.
 template <int ITEMS>
 __global__ __launch_bounds__(1024) void k_sort_one(
     const uint64_t *kin, uint64_t *kout, uint32_t *vout, int n,
-    const int32_t *__restrict__ inst) {
+    const int32_t *__restrict__ inst, bool all, int *flags) {
   constexpr int kWv = 16;
   __shared__ uint64_t sk[1024 * ITEMS];
   __shared__ uint16_t sv[1024 * ITEMS];
@@ -611,8 +613,7 @@ __global__ __launch_bounds__(1024) void k_sort_one(
   }
   // the prefix passes (and the instance's), then the runs; again with all
   // the key's bytes if a run is too long
-  int shift = kPrefixShift;
-  for (bool all = false;;) {
+  for (int shift = all ? 0 : kPrefixShift;;) {
     const int32_t *pi = shift > 56 ? inst : nullptr;
 #pragma unroll
     for (int j = 0; j < 4; ++j) wcnt[w][lane * 4 + j] = 0;
@@ -684,7 +685,10 @@ __global__ __launch_bounds__(1024) void k_sort_one(
         fits &= sort_run(sk, sv, i, n, same) != 0;
       }
       all = __syncthreads_or(!fits);
-      if (all) shift = 0;
+      if (all) {
+        shift = 0;
+        if (t == 0) atomicOr(flags, kFlagFullSort);
+      }
     }
 #pragma unroll
     for (int r = 0; r < ITEMS; ++r)
@@ -873,7 +877,7 @@ int stage_sort(Ctx *c) {
   if (n <= kSortOne) {
     auto go = [&](auto items) {
       k_sort_one<decltype(items)::value><<<1, 1024, 0, c->stream>>>(
-          k0, k0, v0, (int)n, inst);
+          k0, k0, v0, (int)n, inst, c->sort_full, c->flags.as<int>());
     };
     if (n <= 2048)
       go(std::integral_constant<int, 2>{});

@@ -532,11 +532,9 @@ int stage_tree(Ctx *c, bool *again) {
   FSPH_TRY(read_mail(c));
   if (c->mail_h[1] & kFlagScanStall)
     return fail(c, FSPH_E_HIP, "scan: a tile's look-back did not complete");
+  if (c->mail_h[1] & (kFlagLongRun | kFlagFullSort)) c->sort_full = true;
   *again = c->mail_h[1] & kFlagLongRun;
-  if (*again) {
-    c->sort_full = true;
-    return 0;
-  }
+  if (*again) return 0;
   if (c->mail_h[1] & kFlagDupKey)
     return fail(c, FSPH_E_DUPKEY,
                 "two particles share a Morton key (positions closer than "

@@ -28,4 +28,9 @@ int64_t fsph_probe_scratch_bytes(const fsph_ctx *ctx) {
   return (int64_t) reinterpret_cast<const Ctx *>(ctx)->red_tmp.bytes;
 }
 
+// Whether the sort takes all key bits.
+int64_t fsph_probe_sort_full(const fsph_ctx *ctx) {
+  return reinterpret_cast<const Ctx *>(ctx)->sort_full;
+}
+
 }  // extern "C"

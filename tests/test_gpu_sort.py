@@ -1,6 +1,9 @@
 """The two forms of the radix sort (one workgroup, three launches per pass)
 at the edges of their ranges and of their tiles:
 keys and ids in the oracle's order, and a batch in its instances' own."""
+import ctypes as C
+import os
+
 import numpy as np
 import pytest
 
@@ -100,3 +103,23 @@ def test_runs_of_equal_prefixes_in_a_batch(sizes, m):
         s.close()
         o += n
     b.close()
+
+
+@pytest.mark.parametrize("n", [1500, 12288, 12289])
+def test_a_full_sort_is_remembered_until_the_next_upload(n):
+    """Both forms: once a run of equal prefixes was too long, the following
+    sorts take all key bits at once."""
+    full = C.CDLL(os.path.join(os.path.dirname(_abi.__file__),
+                               "libfsph_probe.so")).fsph_probe_sort_full
+    full.restype = C.c_int64
+    long_run, prm = with_cluster(n, 600)
+    short_run, _ = with_cluster(n, 27)
+    g = BodySystem(_abi.default_params(**prm))
+    for parts, want in ((long_run, 1), (short_run, 0), (long_run, 1)):
+        g.upload(parts)
+        assert full(g._h) == 0
+        for _ in range(3):
+            g.update_iteration()
+            assert full(g._h) == want
+            assert np.all(np.diff(g.get("key").astype(np.int64)) > 0)
+    g.close()
