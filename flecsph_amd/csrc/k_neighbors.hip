@@ -117,6 +117,14 @@ struct TravArgs {
 // ball has no margin of h / 2 around the particles, as the box has, and costs
 // fewer operations), and the leaves under kept nodes, 64 at a time in the
 // order they were reached, stay candidates if they lie in such a sphere.
+// Particles far apart for their radii (a diffuse tile beside a dense clump,
+// which the sphere about eight of them may hold although no own sphere comes
+// near it) are tested by their own spheres instead: where such an eight's
+// sphere has more than kSparse times the largest own radius (1.5 to 2.5 times
+// for particles with 40 to 100 neighbours each), and where a walk by eights
+// overflows the largest stack or kFineCap candidates or more, which starts it
+// over (below that the capacity grows: 300 neighbours each need 8,192, and
+// starting over on every call took 10% longer).
 // Where the screen is off (a position that is not a number or infinite in the
 // unit's first particle, or a scale beyond FP32's reach), its nodes take the
 // exact box test and the leaves under them all stay, so that a particle whose
@@ -130,6 +138,8 @@ struct TravArgs {
 // in place of the queue).  Filtering the SPH form's leaves the same way takes
 // 40% of the masks' work off and costs as much here: 64^3 was slower.
 constexpr int kEight = 8;
+constexpr float kSparse = 8.f;
+constexpr int64_t kFineCap = 16384;
 constexpr float kScreen = 1.0f / (1 << 19);
 
 // d^2 - r^2 of the box l .. h and the sphere p (r^2 in p.w)
@@ -144,9 +154,11 @@ __device__ inline float sphere_gap(const float (&l)[3], const float (&h)[3],
 template <int kStack, int MAXG, bool GF>
 __global__ __launch_bounds__(kW) void k_traverse(TravArgs a) {
 #pragma clang fp contract(off)
-  __shared__ float4 sph[MAXG];  // x, y, z, r^2 of the screen
-  // of each eight: the sphere about them, the sphere of the one inside
-  __shared__ float4 outer[MAXG / kEight], inner[MAXG / kEight];
+  // x, y, z, r^2 of the screen (gather form, after the eights are made: r),
+  // then of each eight the sphere about them (r); the sphere of the one inside
+  constexpr int kOuter = MAXG, kSph = MAXG + MAXG / kEight;
+  __shared__ float4 sph[kSph], inner[MAXG / kEight];
+  float4 *const outer = sph + kOuter;
   __shared__ int32_t leaves[GF ? 9 * kW : 1];  // reached, not yet filtered
   __shared__ int32_t stk[kStack];
   constexpr int NK = MAXG / kW;
@@ -224,6 +236,7 @@ __global__ __launch_bounds__(kW) void k_traverse(TravArgs a) {
     outer[lane] = make_float4(INFINITY, 0.f, 0.f, 0.f);
     inner[lane] = make_float4(0.f, 0.f, 0.f, -4.f);
   }
+  bool sparse = false;
   if (lane < n8) {
     float lo[3] = {INFINITY, INFINITY, INFINITY},
           hi[3] = {-INFINITY, -INFINITY, -INFINITY};
@@ -240,7 +253,7 @@ __global__ __launch_bounds__(kW) void k_traverse(TravArgs a) {
     }
     const float m[3] = {0.5f * (lo[0] + hi[0]), 0.5f * (lo[1] + hi[1]),
                         0.5f * (lo[2] + hi[2])};
-    float far = -1.f, best = INFINITY;
+    float far = -1.f, best = INFINITY, rmax = 0.f;
     float4 in = make_float4(0.f, 0.f, 0.f, -4.f);
 #pragma unroll
     for (int u = 0; u < kEight; ++u) {
@@ -248,6 +261,7 @@ __global__ __launch_bounds__(kW) void k_traverse(TravArgs a) {
       const float e0 = p[u].x - m[0], e1 = p[u].y - m[1], e2 = p[u].z - m[2];
       const float dd = sqrtf(e0 * e0 + e1 * e1 + e2 * e2);
       far = fmaxf(far, dd + sqrtf(p[u].w));
+      rmax = fmaxf(rmax, p[u].w);
       if (dd < best) {
         best = dd;
         in = p[u];
@@ -259,19 +273,35 @@ __global__ __launch_bounds__(kW) void k_traverse(TravArgs a) {
                             : make_float4(m[0], m[1], m[2],
                                           far + 4.f * kScreen);
     inner[lane] = in;
+    sparse = far > kSparse * sqrtf(rmax);
+  }
+  // gather form: the spheres tested, the eights' or the particles' own
+  int q_lo = kOuter, q_hi = kOuter + n8;
+  if (GF && __ballot(sparse)) {
+    q_lo = 0;
+    q_hi = gc;
   }
   if (lane == 0) stk[0] = a.root ? a.root[a.inst[gs]] : 0;  // root
   __syncthreads();
-  // Whether the ball of radius r about e (normalised) meets the sphere about
-  // some eight.  The margins of the spheres' radii are many roundings of
+  if (GF) {
+#pragma unroll
+    for (int q = 0; q < NK; ++q)
+      sph[lane + q * kW] =
+          own[q].w < 0.f ? make_float4(INFINITY, 0.f, 0.f, 0.f)
+                         : make_float4(own[q].x, own[q].y, own[q].z,
+                                       sqrtf(own[q].w) + 4.f * kScreen);
+    __syncthreads();
+  }
+  // Whether the ball of radius r about e (normalised) meets some of these
+  // spheres.  The margins of the spheres' radii are many roundings of
   // coordinates and radii up to 5, the factor many of larger ones; a NaN
   // meets every sphere.
   auto meets = [&](float e0, float e1, float e2, float r) {
     bool miss = true;
-    for (int q0 = 0; q0 < n8; q0 += 2)
+    for (int q0 = q_lo; q0 < q_hi; q0 += 2)
 #pragma unroll
       for (int q = q0; q < q0 + 2; ++q) {
-        const float4 o = outer[q];
+        const float4 o = sph[q];
         const float f0 = e0 - o.x, f1 = e1 - o.y, f2 = e2 - o.z, s = r + o.w;
         miss &= __builtin_fmaf(f0, f0, __builtin_fmaf(f1, f1, f2 * f2)) >
                 s * s * (1.f + 4.f * kScreen);
@@ -282,6 +312,18 @@ __global__ __launch_bounds__(kW) void k_traverse(TravArgs a) {
   int64_t ncand = 0;
   const int64_t cbase = gi * a.ccap;
   bool overflow = false;
+  // (gather form) after an overflow of a walk by eights: from the root again
+  auto again = [&] {
+    q_lo = 0;
+    q_hi = gc;
+    overflow = false;
+    sp = 1;
+    nl = 0;
+    ncand = 0;
+    __syncthreads();
+    if (lane == 0) stk[0] = a.root ? a.root[a.inst[gs]] : 0;
+    __syncthreads();
+  };
   while (sp > 0) {
     const int nb = sp < kW ? sp : kW;
     sp -= nb;
@@ -385,6 +427,10 @@ __global__ __launch_bounds__(kW) void k_traverse(TravArgs a) {
     const int all = __builtin_amdgcn_readlane(inc, 63);
     const int tn = all & 0xffff, tl = all >> 16;
     if (sp + tn > kStack) {
+      if (GF && kStack == kStackLarge && scr && q_lo) {
+        again();
+        continue;
+      }
       overflow = true;
       if (lane == 0) atomicOr(a.flags, kFlagStack);
       break;
@@ -434,6 +480,10 @@ __global__ __launch_bounds__(kW) void k_traverse(TravArgs a) {
       done += kW;
     }
     if (overflow) {
+      if (scr && q_lo && a.ccap >= kFineCap) {
+        again();
+        continue;
+      }
       if (lane == 0) atomicOr(a.flags, kFlagCand);
       break;
     }

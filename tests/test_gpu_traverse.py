@@ -1,7 +1,10 @@
 """The traversals' FP32 screen: outside its range every node takes the exact
 test, so neighbour lists equal the oracle's at extreme scales; groups of a
 few particles and gather tiles (Newton-h) at several sizes, scales, a common
-offset and with a position that is not a number."""
+offset, with a position that is not a number and beside a dense clump."""
+import ctypes as C
+import os
+
 import numpy as np
 import pytest
 
@@ -75,11 +78,12 @@ def test_lists_where_fp32_squares_overflow(oracle_mod):
     g.close()
 
 
-def within_h(g):
-    """#{b : r < h} of every particle at the context's own h, by all pairs."""
+def within_h(g, rows=slice(None)):
+    """#{b : r < h} of the particles `rows` at the context's own h, by all
+    pairs."""
     x, y, z, h = (g.get(f) for f in ("x", "y", "z", "h"))
-    d2 = (x[:, None] - x) ** 2 + (y[:, None] - y) ** 2 + (z[:, None] - z) ** 2
-    return (d2 < (h * h)[:, None]).sum(axis=1)
+    d2 = sum((c[rows, None] - c) ** 2 for c in (x, y, z))
+    return (d2 < (h * h)[rows, None]).sum(axis=1)
 
 
 @pytest.mark.parametrize("n,n_target,scale,offset", [
@@ -122,4 +126,48 @@ def test_gather_tile_of_a_nan_position(tile_rows):
     ok = np.arange(n) != 0
     assert np.array_equal(g.get("hngb")[ok], within_h(g)[ok])
     assert g.get("hngb")[0] == 0
+    g.close()
+
+
+@pytest.mark.parametrize("clump", [6000, 280_000])
+@pytest.mark.parametrize("k", [2, 4, 6])
+@pytest.mark.parametrize("wide", [False, True])
+def test_a_clump_beside_a_diffuse_tile(clump, k, wide):
+    """A dense clump among 20,000 particles: its particles lie within the
+    sphere about some eight of a neighbouring tile but near none of the
+    eight, and are no candidates of that tile.  Starting with the clump's h,
+    the particles around it are tested one by one and the capacity stays as
+    it was; with a wider one it may grow to 16,384, not by the clump."""
+    rng = np.random.default_rng(k)
+    v = rng.standard_normal((clump, 3))
+    v *= (rng.random(clump) ** (1 / 3) / np.linalg.norm(v, axis=1))[:, None]
+    mid, rad = 0.15 + 0.06 * k, 0.004
+    h0, gap = rad * (40 / clump) ** (1 / 3), 0.03 if wide else 1.5 * rad
+    a = rng.random((20_000, 3))
+    a = a[np.linalg.norm(a - mid, axis=1) > gap]
+    X = np.concatenate([mid + rad * v, a])
+    n = len(X)
+    z = np.zeros(n)
+    h = z + h0
+    if wide:
+        h[clump:] = 0.015
+    parts = dict(x=X[:, 0], y=X[:, 1], z=X[:, 2], vx=z, vy=z, vz=z, u=z + 1,
+                 m=z + 1 / n, h=h, id=np.arange(n))
+    _, prm = generators.random_box(100)
+    prm.update(h_mode=_abi.H_NEWTON, n_target=40)
+    g = BodySystem(_abi.default_params(**prm))
+    g.upload(parts)
+    g.update_iteration()
+    print(clump, "particles within", rad, "of", mid, flush=True)
+    g.update_h()
+    sizes = (C.c_int64 * 2)()
+    lib = C.CDLL(os.path.join(os.path.dirname(_abi.__file__),
+                              "libfsph_probe.so"))
+    lib.fsph_probe_gather(g._h, sizes)
+    assert sizes[0] == 4096 or (wide and sizes[0] <= 16384)
+    x, y, zz = (g.get(f) for f in ("x", "y", "z"))
+    d = np.sqrt((x - mid) ** 2 + (y - mid) ** 2 + (zz - mid) ** 2)
+    outside = np.flatnonzero(d > 1.2 * rad)
+    rows = outside[np.argsort(d[outside])[:100]]
+    assert np.array_equal(g.get("hngb")[rows], within_h(g, rows))
     g.close()
