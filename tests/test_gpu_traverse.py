@@ -90,20 +90,32 @@ def within_h(g, rows=slice(None)):
     (65, 10, 1.0, 0.0), (1000, 40, 1.0, 0.0), (3000, 40, 1e9, 0.0),
     (3000, 40, 1.0, 1e4)])
 @pytest.mark.parametrize("tile_rows", [64, 128])
+@pytest.mark.parametrize("edge", [False, True])
 def test_newton_h_over_gather_tiles(oracle_mod, n, n_target, scale, offset,
-                                    tile_rows):
-    """Both solvers stop within newton_tol * h of the same root."""
+                                    tile_rows, edge):
+    """Both solvers stop within newton_tol * h of the same root, and the
+    neighbours within the result are all counted; with `edge` the roots lie
+    just inside the gather radius (h_search times the starting h), so that
+    the candidates at its end count."""
     parts, prm = scaled(n, scale, offset, n_target)
     prm.update(h_mode=_abi.H_NEWTON, n_target=n_target,
                precision=_abi.PREC_FP64)
     p = _abi.default_params(**prm)
     g, o = BodySystem(p), oracle_mod.OracleSystem(p, threads=8)
     g._call("set_tuning", tile_rows, 128)
+    if edge:
+        o.upload(parts)
+        for _ in range(4):
+            o.update_iteration()
+            o.update_h()
+        parts = dict(parts, h=np.empty(n))
+        parts["h"][o.get("id")] = o.get("h") / (p.h_search * 0.998)
     for s in (g, o):
         s.upload(parts)
         s.update_iteration()
         s.update_h()
     assert np.allclose(g.get("h"), o.get("h"), rtol=2e-4, atol=0)
+    assert np.array_equal(g.get("hngb"), within_h(g))
     o.close()
     g.close()
 
