@@ -117,13 +117,6 @@ int read_scan_total(Ctx *c, const int64_t *dev_total, int64_t *out) {
   return 0;
 }
 
-int read_flags(Ctx *c, int *flags) {
-  FSPH_HIP(c, hipMemcpyAsync(flags, c->flags.p, sizeof(int),
-                             hipMemcpyDeviceToHost, c->stream));
-  FSPH_HIP(c, hipStreamSynchronize(c->stream));
-  return 0;
-}
-
 namespace {
 
 int do_update_iteration(Ctx *c) {

@@ -6,7 +6,7 @@
 // stage then runs once for all instances: one launch per kernel per step
 // whatever the number of instances.  Only the steps that are defined per
 // simulation look at the instance table: the range and the keys (per
-// instance), the sort (a ninth, stable radix pass on the instance gives
+// instance), the sort (a last, stable radix pass on the instance gives
 // (instance, key, id) order, so every instance is a contiguous segment),
 // the octree (common prefixes end at instance boundaries, every instance
 // has its own root), the traversal (starts at the root of the group's

@@ -403,7 +403,6 @@ int ensure(Ctx *c, DBuf &b, size_t bytes, bool keep = false);
 int ensure_particles(Ctx *c, int64_t cap, bool keep);
 size_t field_size(const Ctx *c, int f);
 int download_map(int field);
-int read_flags(Ctx *c, int *flags);
 
 // ---- primitives (k_prim.hip) --------------------------------------------
 // exclusive scan of n int64 values; out has n+1 entries (out[n] = total).

@@ -4,8 +4,8 @@
 //
 // Bound by the copy to the host (8 bytes per neighbour).  Expanding on the
 // host instead (one copy per tile, then a sort of every row) took 39 ms for
-// the 38,880-particle Sod tube (60 neighbours); here the kernel takes
-// and the copy 1.7 ms.
+// the 38,880-particle Sod tube (60 neighbours); now the tree, the lists and
+// their copy take 1.6 ms, 0.09 of it this kernel.
 #include "fsph_internal.h"
 
 namespace fsph {

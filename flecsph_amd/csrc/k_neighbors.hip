@@ -6,13 +6,18 @@
 // within h_k of some particle k of G (intersects_sphere_box).  Leaves under
 // accepted nodes are then kept if they pass a centre-of-mass filter and
 // d(k,b) <= max(h_k, h_b).  Here one wavefront per group walks the octree
-// with an LDS stack, 64 nodes per step (lanes over nodes, FP64 predicates
-// in the reference's operation order, no FMA contraction), and appends
-// reached leaves to the group's candidate tile.  A second kernel computes,
-// for every (group particle, candidate) pair, the reference's exact
-// neighbour predicate and stores it as a bitmask row per particle:
-// mask[moff[g] + w*gcount + k] bit j <=> candidate 32w+j neighbours k.
-// The SPH passes stage candidates in LDS and walk these bits.
+// with an LDS stack, 64 nodes per step, and appends reached leaves to the
+// group's candidate tile; a second kernel finds, for every (tile row,
+// candidate) pair, whether the reference's predicate holds and stores it as a
+// bitmask row per particle: mask[moff[t] + w*rows + k] bit j <=> candidate
+// 32w+j neighbours row k.  The SPH passes stage candidates in LDS and walk
+// these bits.
+// Both decide nearly every test in FP32, on coordinates relative to the unit,
+// where the rounding cannot change the outcome, and the others in FP64 in the
+// reference's operation order without FMA contraction, so nodes and bits are
+// the reference's.  The gather form (tiles of the smoothing-length solver)
+// needs only the masks to be exact: its traversal keeps a superset, by balls
+// about the nodes' centres of mass and spheres about eight particles.
 #include <cfloat>
 
 #include <type_traits>
@@ -523,7 +528,6 @@ struct MaskArgs {
   int32_t *nngb;  // may be null
   // gather mode: bit set iff r_kb < rscale * h_k (strict, own radius only)
   double rscale;
-  int gather;
   const float *hprop;    // gather radius base instead of h (or null)
   const int32_t *glist;  // tile slot -> group (or null)
   // SPH tiles: each tile's group, rows and candidate slot, and the outputs
@@ -579,8 +583,12 @@ __device__ inline ConstF const_view(const float4 *p) {
   return (ConstF)(uintptr_t)p;
 }
 
-// v_writelane_b32: `old` with lane `lane` (uniform) replaced by v (uniform);
-// the compiler has no __builtin_ form of it
+// v_writelane_b32: `old` with lane `lane` (uniform) replaced by v (uniform).
+// The compiler has no __builtin_ form of it; the intrinsic is named (a name it
+// does not know fails to link) and not written as inline assembly because an
+// instruction that reads a scalar register needs two wait states after the
+// comparison that writes it, which the compiler keeps for the instructions it
+// knows and not for the text of an assembly block.
 __device__ int write_lane(int v, int lane, int old)
     __asm("llvm.amdgcn.writelane.i32");
 
@@ -952,8 +960,8 @@ int build_tiles(Ctx *c, TileBufs tb, bool gather, double scale,
              tb.cand.as<int32_t>(),   tb.ccount.as<int32_t>(),
              tb.moff.as<int64_t>(),   tb.ccap,
              tb.mask.as<uint32_t>(),  nngb,
-             scale,                   gather ? 1 : 0,
-             hprop,                   glist,
+             scale,                   hprop,
+             glist,
              tiled ? c->tgrp.as<int32_t>() : nullptr,
              c->tstart.as<int32_t>(), c->tcount.as<int32_t>(),
              tiled ? c->tslot.as<int32_t>() : nullptr,

@@ -65,7 +65,6 @@ template <class T> struct alignas(4 * sizeof(T)) V4 { T a, b, c, d; };
 template <class T> struct alignas(2 * sizeof(T)) V2 { T a, b; };
 
 struct Phys {
-  int kernel;
   double gamma, alpha, beta, eps;
   int eos;
   const double *kad;  // per-particle adiabat (polytropic EOS)
@@ -297,7 +296,6 @@ template <class T> struct VsigArgs {
   const T *c, *c_old, *rho;
   T *vsig;
   T *divv;  // with DIV: div v_a = -(1/rho_a) sum_b m_b v_ab . grad_a W_ab
-  int kernel;
 };
 
 // Candidate index relative to the tile's first particle, as a T: it is only
@@ -414,7 +412,6 @@ template <class T> struct AlphaArgs {
   T *alpha;
   const double *dtv;
   const int32_t *inst;
-  int kernel;
   double alpha_max, delta, l;
 };
 
@@ -882,7 +879,6 @@ template <class F> void dispatch(const Ctx *c, F &&f) {
 
 Phys phys_of(const Ctx *c) {
   Phys p;
-  p.kernel = c->p.kernel;
   p.gamma = c->p.gamma;
   p.kad = c->f[PF_KAD].as<double>();
   p.alpha = c->p.visc_alpha;
@@ -955,7 +951,6 @@ template <class T> VsigArgs<T> vsig_args(Ctx *c) {
   v.h = c->f[PF_H].as<double>(); v.m = c->f[PF_M].as<double>();
   v.rho = c->f[PF_RHO].as<T>();
   v.divv = c->f[PF_LDIV].as<T>();
-  v.kernel = c->p.kernel;
   return v;
 }
 
@@ -1162,7 +1157,6 @@ template <class T> int alpha_impl(Ctx *c) {
     a.dtv = c->batch.dt.as<double>();
     a.inst = c->f[PF_INST].as<int32_t>();
   }
-  a.kernel = c->p.kernel;
   a.alpha_max = c->p.visc_alpha_max;
   a.delta = c->p.visc_delta;
   a.l = c->p.visc_l;
