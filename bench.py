@@ -94,9 +94,9 @@ VALU_FP32_PEAK_TFLOPS = 157.3  # MI355X FP32 vector, AMD published
 # commands.  A run with another tuning reports no traffic (None: the kernel
 # does not depend on the tuning).
 TRAFFIC = {
-    ("sedov64", "accel"): ((64, 64), 637_743_869),
-    ("sedov64", "masks"): ((64, 64), 223_822_856),
-    ("polytrope1m", "p2p"): (None, 389_688_786),
+    ("sedov64", "accel"): ((64, 64), 693_429_475),
+    ("sedov64", "masks"): ((64, 64), 261_565_483),
+    ("polytrope1m", "p2p"): (None, 386_897_614),
 }
 
 # Side workloads measured after the headline one.
