@@ -622,7 +622,7 @@ __device__ int write_lane(int v, int lane, int old)
 // Sedov 64^3 (474,552 rows and copies) 418 -> 214 us, 1M star 1,000 -> 512,
 // 1.5M collapse 1,594 -> 987 and 1,036 -> 713 (gather), against lanes that
 // held (row, word) pairs, read the candidates from LDS and put the words
-// together bit by bit in FP64; it issues a VALU instruction per 3.7 cycles
+// together bit by bit in FP64; it issues a VALU instruction per 4.3 cycles
 // and SIMD there, 13 per row and round.  A hull box over every eight rows
 // that skips the rounds which miss it saved nothing: 64 candidates in a row
 // cover about the extent of a tile.
